@@ -913,14 +913,7 @@ int tdyhip_create(const tdyhip_mesh *m, const tdyhip_materials *mat, tdyhip_ctx 
     }
     if (W > kJacSlots) { set_error("more than 27 Jacobian entries in a row"); return fail(TDYHIP_ERR_ARG); }
     ctx->jell_w = W;
-    std::vector<int32_t> ecols((size_t)W * nc);
-    for (int c = 0; c < nc; c++)
-      for (int k = 0; k < W; k++) {
-        const int p = topo.jrp[c] + k;
-        ecols[(size_t)k * nc + c] = p < topo.jrp[c + 1] ? topo.jcols[p] : c;
-      }
     if ((rc = dupload(ctx, &ctx->d_jdslot, dslot.data(), dslot.size()))) return fail(rc);
-    if ((rc = dupload(ctx, &ctx->d_ecols, ecols.data(), ecols.size()))) return fail(rc);
   }
   if ((rc = dalloc(ctx, &ctx->d_T, (size_t)kMaxCols * nrows))) return fail(rc);
   if ((rc = dalloc(ctx, &ctx->d_G, (size_t)nrows))) return fail(rc);

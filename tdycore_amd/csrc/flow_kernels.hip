@@ -869,41 +869,6 @@ __global__ void __launch_bounds__(kCellJacBlock) k_seg_cell_jac(const SegProblem
   cell_jac_block<false>(ra, ga, cj, blockIdx.x - sb.start[s]);
 }
 
-// ELL SpMV over the slot-major layout: slot s of row i at s*n + i.
-template <class TV>
-__device__ inline TV ell_row(int n, int W, int i, const int32_t *__restrict__ ecol, const TV *__restrict__ a,
-                            const TV *__restrict__ x) {
-  TV s = 0;
-  // FP32 rows of a hexahedral mesh: the whole row's loads issued at once (in
-  // FP64 the 81 extra registers cost more occupancy than they gain)
-  if (sizeof(TV) == 4 && W == kJacSlots) {
-    int c[kJacSlots];
-    TV v[kJacSlots];
-#pragma unroll
-    for (int k = 0; k < kJacSlots; k++) {
-      c[k] = ecol[(int64_t)k * n + i];
-      v[k] = a[(int64_t)k * n + i];
-    }
-#pragma unroll
-    for (int k = 0; k < kJacSlots; k++) s += v[k] * x[c[k]];
-  } else {
-    for (int k = 0; k < W; k++) {
-      const int64_t p = (int64_t)k * n + i;
-      s += a[p] * x[ecol[p]];
-    }
-  }
-  return s;
-}
-
-template <class TV>
-__global__ void __launch_bounds__(256) k_spmv_ell(int n, int W, const int32_t *__restrict__ ecol,
-                                                  const TV *__restrict__ a, const TV *__restrict__ x,
-                                                  TV *__restrict__ y) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  y[i] = ell_row<TV>(n, W, i, ecol, a, x);
-}
-
 __global__ void k_fill(int64_t n, double *__restrict__ x, double val) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) x[i] = val;

@@ -851,33 +851,6 @@ __global__ void k_convert(int64_t n, const TA *__restrict__ a, TB *__restrict__ 
   if (i < n) b[i] = (TB)a[i];
 }
 
-// out = a - b
-template <class TV>
-__global__ void k_sub(int64_t n, const TV *__restrict__ a, const TV *__restrict__ b, TV *__restrict__ out) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) out[i] = a[i] - b[i];
-}
-
-
-
-template <class TV>
-__global__ void __launch_bounds__(256) k_spmv_ell_stop(int n, int W, const int32_t *__restrict__ ecol,
-                                                       const TV *__restrict__ a, const TV *__restrict__ x,
-                                                       TV *__restrict__ y, const GmresDev *__restrict__ gd) {
-  if (gd->done) return;
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  y[i] = ell_row<TV>(n, W, i, ecol, a, x);
-}
-
-// y = s * x with s read on the device (1/beta or 1/h(j+1,j))
-template <class TV>
-__global__ void k_scale_dev(int64_t n, const TV *__restrict__ x, TV *__restrict__ y, const GmresDev *__restrict__ gd) {
-  if (gd->done) return;
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) y[i] = (TV)gd->inv_h * x[i];
-}
-
 __global__ void k_gmres_init(GmresDev *gd, int *status, int maxit) {
   gd->its = 0;
   gd->done = 0;

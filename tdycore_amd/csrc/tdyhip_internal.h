@@ -169,7 +169,6 @@ struct tdyhip_ctx {
   int32_t *d_jrp = nullptr, *d_jcols = nullptr;
   uint8_t *d_jdslot = nullptr;      // nc: slot of the diagonal within its row
   int jell_w = 0;                   // ELL width (longest Jacobian row)
-  int32_t *d_ecols = nullptr;       // jell_w*nc slot-major ELL columns (padding = own row)
 
   // device: state
   double *d_rho = nullptr, *d_ukvr = nullptr, *d_drho = nullptr, *d_dukvr = nullptr;
