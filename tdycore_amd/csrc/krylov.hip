@@ -276,20 +276,106 @@ __device__ inline TV block_sum_n(TV v, TV *sh) {
   return s;
 }
 
-// Restriction of the block's right-hand side to one value (the coarse
-// correction's R1^T r), written by thread 0; all threads call it.
-template <class TV, int BS>
-__device__ inline void restrict_block(const TV *x, double *rc1, int b, int t) {
-  __shared__ TV sh[BS / 64];
-  const TV s = block_sum_n<BS>(x[t], sh);
-  if (t == 0) rc1[b] = (double)s;
+// ---------------------------------------------------------------- coarse right-hand side
+// The coarse correction acts on what the block-Jacobi sweeps leave:
+//   w = w_bj + P z,  z = Ac^-1 R (r - A w_bj)   (w_bj = BJ^-1 r)
+// with R the block sums and P the blocks' constant prolongation (coarse.hip).
+// R A w_bj needs no second matvec: row j of block b meets R A only in the
+// few blocks its column of A reaches, C[q][j] = sum of A_ij over the rows i of
+// neighbour block q, so the workgroup that has just swept block b sums its
+// contributions C[q][.] w_bj to every neighbour q and stores each in a slot of
+// the receiving block that nobody else writes (no atomics, a fixed order).
+// A block's own column sums (q = itself, all its rows) are one coalesced value
+// per row; the others are listed by neighbour, each neighbour's list padded to
+// teams of 8 lanes (kCoarsePad).
+constexpr int kCQ = 32;  // neighbour blocks of a block (itself included)
+constexpr uint16_t kCoarsePad = 0xffff;
+struct CoarseRestrict {
+  const double *cown = nullptr;    // nblocks*bs: the own block's column sums
+  const int32_t *eptr = nullptr;   // nblocks+1: first list entry of each block (multiples of 8)
+  const uint16_t *cent = nullptr;  // list entries: row of the block | neighbour << 9
+  const double *cval = nullptr;    // their column sums
+  const uint16_t *tq = nullptr;    // nblocks*(kCQ+1): first 8-entry team of each neighbour
+  const uint8_t *ownq = nullptr;   // nblocks: the own block's place among the neighbours
+  const int32_t *wdst = nullptr;   // nblocks*kCQ: where the contribution to neighbour q goes in rcs (-1 none)
+  const uint8_t *gsl = nullptr;    // nblocks*kCQ: which of the groups the block reaches neighbour q is in (255 none)
+  const int32_t *w2dst = nullptr;  // nblocks*kCQ: where the sum over its s-th group goes in r2c (-1 none)
+  double *rcs = nullptr;           // nblocks*kCQ: received contributions; nullptr: no coarse correction
+  double *r2c = nullptr;           // received contributions by group
+};
+
+// Per-neighbour sums of block b: thread q < kCQ returns the sum of neighbour q
+// (the own block's: of `own` over the workgroup; another's: of value(e) over
+// its list).  Every thread calls it; one barrier inside.
+template <int BS, class F>
+__device__ inline double coarse_block_sums(const CoarseRestrict &R, int b, int t, double own, F &&value) {
+  constexpr int kTeams = BS * 27 / 8 + kCQ;  // every row in 27 lists, each list's last team short
+  __shared__ double tm[kTeams];
+  __shared__ double ow[BS / 64];
+  const int e0 = R.eptr[b], ne = R.eptr[b + 1] - e0;
+  for (int off = 32; off > 0; off >>= 1) own += __shfl_down(own, off, 64);
+  if ((t & 63) == 0) ow[t >> 6] = own;
+  for (int e = t; e < ne; e += BS) {  // ne is a multiple of 8: a team's lanes stay together
+    double v = value(e0 + e);
+    v += __shfl_xor(v, 1, 64);
+    v += __shfl_xor(v, 2, 64);
+    v += __shfl_xor(v, 4, 64);
+    if ((t & 7) == 0) tm[e >> 3] = v;
+  }
+  __syncthreads();
+  double s = 0.0;
+  if (t < kCQ) {
+    const int i0 = R.tq[b * (kCQ + 1) + t], i1 = R.tq[b * (kCQ + 1) + t + 1];
+    for (int i = i0; i < i1; i++) s += tm[i];
+    if (t == R.ownq[b]) {
+#pragma unroll
+      for (int w = 0; w < BS / 64; w++) s += ow[w];
+    }
+  }
+  return s;
 }
 
-// The same restriction, and in the same pass the block sum of v (this
-// thread's entry of the basis vector) into rv[b]; rc1[b] is the value
-// restrict_block gives.
+// After the sweeps (x: w_bj of the block, rr: the block sum of its right-hand
+// side): the block's contributions to R (r - A w_bj), per neighbour block and
+// summed per neighbour group.  Every thread calls it.
 template <class TV, int BS>
-__device__ inline void restrict_block2(const TV *x, double *rc1, TV v, double *rv, int b, int t) {
+__device__ inline void coarse_scatter(const CoarseRestrict &R, const TV *x, const double &rr, int b, int t) {
+  __shared__ double qv[kCQ];
+  __shared__ uint8_t qg[kCQ];
+  const double s = coarse_block_sums<BS>(R, b, t, R.cown[(int64_t)b * BS + t] * (double)x[t],
+                                         [&](int e) {
+                                           const unsigned w = R.cent[e];
+                                           return R.cval[e] * (double)x[w == kCoarsePad ? BS : w & 511];  // x[BS] is 0
+                                         });
+  if (t < kCQ) {
+    const double v = (t == R.ownq[b] ? rr : 0.0) - s;
+    const int d = R.wdst[b * kCQ + t], d2 = R.w2dst[b * kCQ + t];
+    if (d >= 0) R.rcs[d] = v;
+    qv[t] = v;
+    qg[t] = R.gsl[b * kCQ + t];
+    __builtin_amdgcn_wave_barrier();  // one wavefront: its LDS operations run in program order
+    if (d2 >= 0) {
+      double g = 0.0;
+#pragma unroll
+      for (int q = 0; q < kCQ; q++) g += qg[q] == t ? qv[q] : 0.0;
+      R.r2c[d2] = g;
+    }
+  }
+}
+
+// Block sum of the right-hand side x, left in LDS (rr) by thread 0; the
+// sweeps' barriers come before its use.
+template <class TV, int BS>
+__device__ inline void restrict_block(const TV *x, double &rr, int t) {
+  __shared__ TV sh[BS / 64];
+  const TV s = block_sum_n<BS>(x[t], sh);
+  if (t == 0) rr = (double)s;
+}
+
+// The same, and in the same pass the block sum of v (this thread's entry of
+// the basis vector) into rv[b].
+template <class TV, int BS>
+__device__ inline void restrict_block2(const TV *x, double &rr, TV v, double *rv, int b, int t) {
   __shared__ TV sh[2][BS / 64];
   TV a = x[t];
   for (int off = 32; off > 0; off >>= 1) {
@@ -308,7 +394,7 @@ __device__ inline void restrict_block2(const TV *x, double *rc1, TV v, double *r
       s += sh[0][w];
       q += sh[1][w];
     }
-    rc1[b] = (double)s;
+    rr = (double)s;
     rv[b] = (double)q;
   }
   __syncthreads();
@@ -364,16 +450,18 @@ __device__ inline void bj_sweeps(const BJLayout &L, const TV *__restrict__ fac, 
 template <class TV, int BS>
 __global__ void __launch_bounds__(BS) k_bj_apply(BJLayout L, const TV *__restrict__ fac, const TV *__restrict__ r,
                                                  TV *__restrict__ y, const int *__restrict__ stop = nullptr,
-                                                 double *__restrict__ rc1 = nullptr) {
+                                                 CoarseRestrict cr = CoarseRestrict{}) {
   __shared__ TV x[BS + 1];
+  __shared__ double rr;
   if (stop && *stop) return;  // uniform over the workgroup
   const int b = blockIdx.x, t = threadIdx.x;
   const int row = L.d_row[(int64_t)b * BS + t];
   x[t] = row >= 0 ? r[row] : (TV)0;
   if (t == 0) x[BS] = (TV)0;
-  if (rc1) restrict_block<TV, BS>(x, rc1, b, t);  // rc1 is uniform
+  if (cr.rcs) restrict_block<TV, BS>(x, rr, t);  // cr is uniform
   bj_sweeps<TV, BS>(L, fac, x, b, t);
   if (row >= 0) y[row] = x[t];
+  if (cr.rcs) coarse_scatter<TV, BS>(cr, x, rr, b, t);
 }
 
 // ---------------------------------------------------------------- block-ordered SpMV
@@ -519,9 +607,10 @@ __global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(4))) k_
                                                       const TV *__restrict__ a, const TV *__restrict__ u,
                                                       GmresDev *__restrict__ gd, TV *__restrict__ vj,
                                                       const TV *__restrict__ fac, TV *__restrict__ out,
-                                                      const int *__restrict__ stop, double *__restrict__ rc1,
+                                                      const int *__restrict__ stop, CoarseRestrict cr,
                                                       NormArgs na, double *__restrict__ rv) {
   __shared__ TV x[BS + 1];
+  __shared__ double rr;
   __shared__ TV shn[BS / 64];
   __shared__ int stop_s;
   const int b = blockIdx.x, t = threadIdx.x;
@@ -555,24 +644,26 @@ __global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(4))) k_
   const TV vv = row >= 0 ? sc * u[row] : (TV)0;
   if (row >= 0) vj[row] = vv;
   if (t == 0) x[BS] = (TV)0;
-  // rc1 and rv are uniform; rv: the block sums of V_j, for the coarse terms of the multi-dot
-  if (rc1 && rv) restrict_block2<TV, BS>(x, rc1, vv, rv, b, t);
-  else if (rc1) restrict_block<TV, BS>(x, rc1, b, t);
+  // cr is uniform; rv: the block sums of V_j, for the coarse terms of the multi-dot
+  if (cr.rcs) restrict_block2<TV, BS>(x, rr, vv, rv, b, t);
   bj_sweeps<TV, BS>(L, fac, x, b, t);
   if (row >= 0) out[row] = x[t];
+  if (cr.rcs) coarse_scatter<TV, BS>(cr, x, rr, b, t);
 }
 
 // A restart's preconditioned residual out = M_BJ^-1 (b - J y) in one pass:
 // the block's rows of b - J y (FP64, the difference taken in FP64 and then
 // rounded to TV, as a separate product and difference would give) go into
-// LDS, restricted for the coarse level when rc1 is set, and the sweeps follow.
+// LDS, the sweeps follow, and the block's part of the coarse right-hand side
+// when the coarse correction is on.
 template <class TV, int BS, class TI>
 __global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(4))) k_bj_resid_apply(BJLayout L, int W, const TI *__restrict__ ecol,
                                                        const double *__restrict__ J, const double *__restrict__ y,
                                                        const double *__restrict__ bvec, const TV *__restrict__ fac,
                                                        TV *__restrict__ out, const int *__restrict__ stop,
-                                                       double *__restrict__ rc1) {
+                                                       CoarseRestrict cr) {
   __shared__ TV x[BS + 1];
+  __shared__ double rr;
   if (stop && *stop) return;  // uniform over the workgroup
   const int b = blockIdx.x, t = threadIdx.x;
   const int64_t p = (int64_t)b * BS + t;
@@ -583,9 +674,10 @@ __global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(4))) k_
   x[t] = row >= 0 ? (TV)(bvec[row] - blk_row<double, TI, true>(((int64_t)b * W) * BS + t, BS, wb, row, ecol, eb, es, J, y))
                   : (TV)0;
   if (t == 0) x[BS] = (TV)0;
-  if (rc1) restrict_block<TV, BS>(x, rc1, b, t);  // rc1 is uniform
+  if (cr.rcs) restrict_block<TV, BS>(x, rr, t);  // cr is uniform
   bj_sweeps<TV, BS>(L, fac, x, b, t);
   if (row >= 0) out[row] = x[t];
+  if (cr.rcs) coarse_scatter<TV, BS>(cr, x, rr, b, t);
 }
 
 // ---------------------------------------------------------------- BLAS-1 with deterministic reductions
@@ -647,19 +739,23 @@ __device__ inline TV wave_reduce_scatter(TV (&v)[32]) {
   return r;
 }
 
-// The coarse correction's level-1/2 solve run by the first ng workgroups of
-// a multi-dot launch (ng = 0: none), with the group's terms of the dots.
+// The coarse solve run by the first `parts` workgroups of a multi-dot launch
+// (0: none), with their terms of the dots.
 struct CoarseDot {
-  int ng = 0, gsz = 0;
+  int parts = 0;                                // parts of the groups, in group order
+  int ng = 0, gsz = 0, g2max = 0;               // groups, blocks of a group, entries of r2c of a group (at most)
+  int nov = 0;                                  // columns of G1 (0: level 2 alone)
   const int32_t *gmem = nullptr;                // ng*gsz blocks of each group (-1 pad)
-  const double *G1 = nullptr, *A2 = nullptr;    // group inverses, inverted level-2 operator
-  const double *rc1 = nullptr;                  // restricted vector (one value per block)
+  const int32_t *gov = nullptr;                 // ng*nov blocks of each group with its overlap (-1 pad)
+  const double *G1 = nullptr, *M = nullptr;     // group and level-2 parts of the coarse inverse (coarse.hip)
+  const double *rcs = nullptr, *r2c = nullptr;  // contributions to the restricted residual, by block and by group
+  const int32_t *g2ptr = nullptr;               // ng+1: each group's entries of r2c
   const double *RV = nullptr;                   // block sums of the basis vectors, rv_ld per vector
   int64_t rv_ld = 0;
   double *z1 = nullptr;                         // coarse correction per block (out)
 };
 template <class TV>
-__device__ void coarse_level1_dots(const CoarseDot &cd, int g, int nv, TV *partial, int pstride);
+__device__ void coarse_level1_dots(const CoarseDot &cd, int part, int nv, TV *partial, int pstride);
 
 // Coarse prolongation applied on the fly: w[i] += z1[pos[i] >> bs_log2]
 // (pos = block-layout position of row i).  z1 == nullptr: none.
@@ -710,20 +806,24 @@ __device__ inline void load_pairs(const TV *__restrict__ V, int64_t ldv, int64_t
 // one reduce-scatter per wavefront and one barrier per group of NS vectors
 // finish the chunk.  With pro.z1 set, w first receives the coarse
 // prolongation (written back).
-template <class TV, int NS>
-__global__ void __launch_bounds__(kRedBlock) k_mdot(int64_t n, int nv, const TV *__restrict__ V, int64_t ldv,
+//
+// COARSE: the launch's first cd.parts workgroups run the coarse solve; its
+// registers would set the occupancy of the row chunks at NS <= 16 (74), so
+// the budget is held to 7 waves per SIMD there.
+template <class TV, int NS, bool COARSE>
+__global__ void __launch_bounds__(kRedBlock) __attribute__((amdgpu_waves_per_eu(COARSE && NS <= 16 ? 7 : 1))) k_mdot(int64_t n, int nv, const TV *__restrict__ V, int64_t ldv,
                                                     TV *__restrict__ w, TV *__restrict__ partial, int nchunk,
                                                     Prolong pro, const int *__restrict__ stop = nullptr,
                                                     CoarseDot cd = CoarseDot{}) {
   static_assert(Red<TV>::E == 2, "two rows per thread");
   __shared__ TV red[kRedBlock / 64][NS];
   if (stop && *stop) return;
-  // partial[j*nchunk + c]: c < cd.ng the coarse workgroups' terms, then one per row chunk
-  if ((int)blockIdx.x < cd.ng) {
+  // partial[j*nchunk + c]: c < cd.parts the coarse workgroups' terms, then one per row chunk
+  if (COARSE && (int)blockIdx.x < cd.parts) {
     coarse_level1_dots<TV>(cd, blockIdx.x, nv, partial, nchunk);
     return;
   }
-  const int chunk = blockIdx.x - cd.ng;
+  const int chunk = blockIdx.x - cd.parts;
   const int t = threadIdx.x, lane = t & 63, wv_id = t >> 6;
   const int64_t r0 = (int64_t)chunk * Red<TV>::chunk + 2 * t;
   const bool vec = (ldv & 1) == 0;
@@ -765,7 +865,7 @@ __global__ void __launch_bounds__(kRedBlock) k_mdot(int64_t n, int nv, const TV 
       TV s = 0;
 #pragma unroll
       for (int q = 0; q < kRedBlock / 64; q++) s += red[q][t];
-      partial[(int64_t)(j0 + t) * nchunk + cd.ng + chunk] = s;
+      partial[(int64_t)(j0 + t) * nchunk + cd.parts + chunk] = s;
     }
     __syncthreads();
   }

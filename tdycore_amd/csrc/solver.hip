@@ -276,16 +276,21 @@ static std::string build_bj(const std::vector<int32_t> &jrp, const std::vector<i
 }
 
 struct HostCoarse {
-  int nb = 0, ng = 0, gsz = 0;
-  std::vector<int32_t> nbr, grp, gmem;
-  std::vector<uint8_t> cq;
+  int nb = 0, ng = 0, gsz = 0, nov = 0;
+  std::vector<int32_t> nbr, grp, gmem, gov, g2ptr;
+  std::vector<uint8_t> cq, gpos;
+  // CoarseRestrict: entry lists, teams and destinations
+  std::vector<int32_t> eptr, wdst, w2dst;
+  std::vector<uint16_t> cent, tq, gent, gep;
+  std::vector<uint8_t> ownq, gsl;
 };
 
-// Level-1 / level-2 structure of the coarse correction: neighbour blocks of
-// each block, the slot -> neighbour map, and groups of blocks built by
-// breadth-first aggregation over block adjacency (group size grown until at
-// most kNG groups remain).  Returns an empty string when the mesh is outside
-// the correction's limits (then it is not used).
+// Structure of the coarse correction (coarse.hip): neighbour blocks of each
+// block, the slot -> neighbour map, groups of blocks built by breadth-first
+// aggregation over block adjacency (group size grown until at most kNG groups
+// remain), each group's overlap, and the lists by which a block's sweeps pass
+// on their part of the restricted residual.  Returns an empty string when the
+// mesh is within the correction's limits (otherwise it is not used).
 static std::string build_coarse(const HostBJ &hb, const std::vector<int32_t> &jrp, const std::vector<int32_t> &jcols,
                                 int nc, int W, HostCoarse &out) {
   const int S = hb.bs, nb = hb.nblocks;
@@ -294,33 +299,66 @@ static std::string build_coarse(const HostBJ &hb, const std::vector<int32_t> &jr
   for (int c = 0; c < nc; c++) blk[c] = hb.perm[c] / S;
   out.nb = nb;
   out.nbr.assign((size_t)nb * kCQ, -1);
-  std::vector<int32_t> tmp;
+  out.cq.assign((size_t)W * NB, 255);
+  out.ownq.assign(nb, 0);
+  out.eptr.assign(nb + 1, 0);
+  out.tq.assign((size_t)nb * (kCQ + 1), 0);
+  std::vector<int32_t> tmp, place(nb, -1);
+  std::vector<uint32_t> rowmask(S);
   for (int b = 0; b < nb; b++) {
     tmp.clear();
     for (int i = 0; i < S; i++) {
       const int r = hb.row[(size_t)b * S + i];
       if (r < 0) continue;
-      for (int k = jrp[r]; k < jrp[r + 1]; k++) tmp.push_back(blk[jcols[k]]);
+      for (int k = jrp[r]; k < jrp[r + 1]; k++) {
+        const int cb = blk[jcols[k]];
+        if (place[cb] < 0) { place[cb] = 0; tmp.push_back(cb); }
+      }
     }
-    std::sort(tmp.begin(), tmp.end());
-    tmp.erase(std::unique(tmp.begin(), tmp.end()), tmp.end());
     if ((int)tmp.size() > kCQ) return "a block has more than 32 neighbour blocks";
-    for (size_t q = 0; q < tmp.size(); q++) out.nbr[(size_t)b * kCQ + q] = tmp[q];
-  }
-  out.cq.assign((size_t)W * NB, 255);
-  for (int64_t p = 0; p < NB; p++) {
-    const int r = hb.row[p];
-    if (r < 0) continue;
-    const int b = (int)(p / S);
-    const int32_t *nl = &out.nbr[(size_t)b * kCQ];
-    for (int k = 0; k < jrp[r + 1] - jrp[r]; k++) {
-      const int cb = blk[jcols[jrp[r] + k]];
-      for (int q = 0; q < kCQ && nl[q] >= 0; q++)
-        if (nl[q] == cb) { out.cq[(size_t)k * NB + p] = (uint8_t)q; break; }
+    std::sort(tmp.begin(), tmp.end());
+    for (size_t q = 0; q < tmp.size(); q++) {
+      out.nbr[(size_t)b * kCQ + q] = tmp[q];
+      place[tmp[q]] = (int32_t)q;
+      if (tmp[q] == b) out.ownq[b] = (uint8_t)q;
     }
+    // each row's slots by neighbour, and the rows that reach each other block
+    const uint32_t own = 1u << out.ownq[b];
+    int cnt[kCQ] = {};
+    for (int i = 0; i < S; i++) {
+      const int64_t p = (int64_t)b * S + i;
+      const int r = hb.row[p];
+      uint32_t mask = 0;
+      if (r >= 0)
+        for (int k = 0; k < jrp[r + 1] - jrp[r]; k++) {
+          const int q = place[blk[jcols[jrp[r] + k]]];
+          out.cq[(size_t)k * NB + p] = (uint8_t)q;
+          mask |= 1u << q;
+        }
+      rowmask[i] = mask & ~own;
+      for (uint32_t w = rowmask[i]; w; w &= w - 1) cnt[__builtin_ctz(w)]++;
+    }
+    int team = 0, at[kCQ];
+    const size_t e0 = out.cent.size();
+    for (int q = 0; q < kCQ; q++) {
+      out.tq[(size_t)b * (kCQ + 1) + q] = (uint16_t)team;
+      at[q] = 8 * team;
+      team += (cnt[q] + 7) / 8;
+    }
+    out.tq[(size_t)b * (kCQ + 1) + kCQ] = (uint16_t)team;
+    out.cent.resize(e0 + (size_t)8 * team, kCoarsePad);
+    for (int i = 0; i < S; i++)
+      for (uint32_t w = rowmask[i]; w; w &= w - 1) {
+        const int q = __builtin_ctz(w);
+        out.cent[e0 + at[q]++] = (uint16_t)(i | q << 9);
+      }
+    if (out.cent.size() > (size_t)INT32_MAX) return "too many coarse entries";
+    out.eptr[b + 1] = (int32_t)out.cent.size();
+    for (int32_t cb : tmp) place[cb] = -1;
   }
   // groups
-  for (int G = std::max(1, (nb + kNG - 1) / kNG); G <= kGMax; G++) {
+  bool grouped = false;
+  for (int G = std::max(1, (nb + kNG - 1) / kNG); G <= kGMax && !grouped; G++) {
     std::vector<int32_t> grp(nb, -1), mem;
     std::vector<std::vector<int32_t>> groups;
     std::vector<int32_t> queue;
@@ -346,15 +384,101 @@ static std::string build_coarse(const HostBJ &hb, const std::vector<int32_t> &jr
       }
     }
     if ((int)groups.size() > kNG) continue;
+    grouped = true;
     out.ng = (int)groups.size();
     out.gsz = G;
     out.grp = grp;
     out.gmem.assign((size_t)out.ng * G, -1);
     for (int g = 0; g < out.ng; g++)
       for (size_t i = 0; i < groups[g].size(); i++) out.gmem[(size_t)g * G + i] = groups[g][i];
-    return std::string();
   }
-  return "too many blocks for the coarse correction";
+  if (!grouped) return "too many blocks for the coarse correction";
+  // groups with overlap: the members, then their neighbours in other groups (ascending), at most kOV
+  if (out.gsz > 1) {
+    std::vector<std::vector<int32_t>> ov(out.ng);
+    for (int g = 0; g < out.ng; g++) {
+      std::vector<int32_t> &o = ov[g], ext;
+      for (int i = 0; i < out.gsz; i++) {
+        const int b = out.gmem[(size_t)g * out.gsz + i];
+        if (b < 0) break;
+        o.push_back(b);
+        for (int q = 0; q < kCQ && out.nbr[(size_t)b * kCQ + q] >= 0; q++) {
+          const int nbk = out.nbr[(size_t)b * kCQ + q];
+          if (out.grp[nbk] != g && place[nbk] < 0) { place[nbk] = 0; ext.push_back(nbk); }
+        }
+      }
+      for (int32_t b : ext) place[b] = -1;
+      std::sort(ext.begin(), ext.end());
+      if (ext.size() + o.size() > (size_t)kOV) ext.resize(kOV - o.size());
+      o.insert(o.end(), ext.begin(), ext.end());
+      out.nov = std::max(out.nov, (int)o.size());
+    }
+    out.gov.assign((size_t)out.ng * out.nov, -1);
+    out.gpos.assign((size_t)out.ng * out.nov * kCQ, 255);
+    for (int g = 0; g < out.ng; g++) {
+      const std::vector<int32_t> &o = ov[g];
+      for (size_t c = 0; c < o.size(); c++) place[o[c]] = (int32_t)c;
+      for (size_t c = 0; c < o.size(); c++) {
+        out.gov[(size_t)g * out.nov + c] = o[c];
+        for (int q = 0; q < kCQ && out.nbr[(size_t)o[c] * kCQ + q] >= 0; q++) {
+          const int at = place[out.nbr[(size_t)o[c] * kCQ + q]];
+          if (at >= 0) out.gpos[((size_t)g * out.nov + c) * kCQ + q] = (uint8_t)at;
+        }
+      }
+      for (int32_t b : o) place[b] = -1;
+    }
+  }
+  // the entries of the members' A1 rows by the neighbour's group
+  const int nm = out.nov ? out.nov : out.gsz;
+  const std::vector<int32_t> &gm = out.nov ? out.gov : out.gmem;
+  out.gent.assign((size_t)out.ng * nm * kCQ, 0);
+  out.gep.assign((size_t)out.ng * (out.ng + 1), 0);
+  for (int g = 0; g < out.ng; g++) {
+    uint16_t *ep = &out.gep[(size_t)g * (out.ng + 1)], *en = &out.gent[(size_t)g * nm * kCQ];
+    for (int pass = 0; pass < 2; pass++) {
+      std::vector<int> at(ep, ep + out.ng);
+      for (int c = 0; c < nm; c++) {
+        const int b = gm[(size_t)g * nm + c];
+        if (b < 0) break;
+        for (int q = 0; q < kCQ && out.nbr[(size_t)b * kCQ + q] >= 0; q++) {
+          const int h = out.grp[out.nbr[(size_t)b * kCQ + q]];
+          if (pass == 0) ep[h + 1]++;
+          else en[at[h]++] = (uint16_t)(c * kCQ + q);
+        }
+      }
+      if (pass == 0)
+        for (int h = 0; h < out.ng; h++) ep[h + 1] += ep[h];
+    }
+  }
+  // where each block's contributions go: the receiving block's slot of this
+  // block, and the receiving group's list
+  out.wdst.assign((size_t)nb * kCQ, -1);
+  out.w2dst.assign((size_t)nb * kCQ, -1);
+  out.gsl.assign((size_t)nb * kCQ, 255);
+  std::vector<int32_t> reach((size_t)nb * kCQ, -1);
+  out.g2ptr.assign(out.ng + 1, 0);
+  for (int b = 0; b < nb; b++) {
+    const int32_t *nl = &out.nbr[(size_t)b * kCQ];
+    int ns = 0;
+    for (int q = 0; q < kCQ && nl[q] >= 0; q++) {
+      const int32_t *ml = &out.nbr[(size_t)nl[q] * kCQ];
+      int m = 0;
+      while (m < kCQ && ml[m] != b) m++;
+      if (m == kCQ) return "the block adjacency is not symmetric";
+      out.wdst[(size_t)b * kCQ + q] = nl[q] * kCQ + m;
+      const int h = out.grp[nl[q]];
+      int s = 0;
+      while (s < ns && reach[(size_t)b * kCQ + s] != h) s++;
+      if (s == ns) { reach[(size_t)b * kCQ + ns++] = h; out.g2ptr[h + 1]++; }
+      out.gsl[(size_t)b * kCQ + q] = (uint8_t)s;
+    }
+  }
+  for (int h = 0; h < out.ng; h++) out.g2ptr[h + 1] += out.g2ptr[h];
+  std::vector<int32_t> fill(out.g2ptr.begin(), out.g2ptr.end() - 1);
+  for (int b = 0; b < nb; b++)
+    for (int s = 0; s < kCQ && reach[(size_t)b * kCQ + s] >= 0; s++)
+      out.w2dst[(size_t)b * kCQ + s] = fill[reach[(size_t)b * kCQ + s]]++;
+  return std::string();
 }
 
 struct SolverWS {
@@ -527,7 +651,7 @@ static int ensure_ws(tdyhip_ctx *ctx, const tdyhip_solver_opts &o) {
   char **cp[] = {(char **)&ws.V, (char **)&ws.w, (char **)&ws.z, (char **)&ws.b, (char **)&ws.x, (char **)&ws.fac,
                  (char **)&ws.partial};
   size_t cnt[] = {(size_t)(o.ksp_restart + 1) * n, (size_t)n, (size_t)n, (size_t)n, (size_t)n,
-                  (size_t)hb.nblocks * kW * hb.bs, (size_t)(o.ksp_restart + 2) * (ws.nchunk + kNG)};
+                  (size_t)hb.nblocks * kW * hb.bs, (size_t)(o.ksp_restart + 2) * (ws.nchunk + kNG * coarse_parts(kGMax))};
   for (int i = 0; i < 7; i++)
     if ((rc = ws_alloc(ws, cp[i], cnt[i] * tv))) return rc;
   if ((rc = ws_alloc(ws, (float **)&ws.Jk, nnz))) return rc;  // FP32 copy of the Jacobian
@@ -545,18 +669,39 @@ static int ensure_ws(tdyhip_ctx *ctx, const tdyhip_solver_opts &o) {
     // (the Galerkin row kernel handles up to 32 slots per row)
     if (ctx->jell_w <= 32 && build_coarse(hb, ctx->h_jrp, ctx->h_jcols, ctx->nc, ctx->jell_w, hc).empty()) {
       CoarseLayout &C = ws.cl;
-      C.nb = hc.nb; C.ng = hc.ng; C.gsz = hc.gsz;
+      CoarseRestrict &R = C.R;
+      C.nb = hc.nb; C.ng = hc.ng; C.gsz = hc.gsz; C.nov = hc.nov;
+      for (int h = 0; h < hc.ng; h++) C.g2max = std::max(C.g2max, hc.g2ptr[h + 1] - hc.g2ptr[h]);
+      const size_t nq = (size_t)hc.nb * kCQ, nel = (size_t)ctx->jell_w * ws.NB;
+      int32_t *eptr, *wdst, *w2dst;
+      uint16_t *cent, *tq;
+      uint8_t *ownq, *gsl;
       if ((rc = up(&C.nbr, hc.nbr)) || (rc = up(&C.cq, block_contiguous(hc.cq, ctx->jell_w, hb.bs, hb.nblocks))) ||
-          (rc = up(&C.grp, hc.grp)) ||
-          (rc = up(&C.gmem, hc.gmem)))
+          (rc = up(&C.grp, hc.grp)) || (rc = up(&C.gmem, hc.gmem)) || (rc = up(&C.gov, hc.gov)) ||
+          (rc = up(&C.gpos, hc.gpos)) || (rc = up(&C.gent, hc.gent)) || (rc = up(&C.gep, hc.gep)) || (rc = up(&C.g2ptr, hc.g2ptr)) || (rc = up(&eptr, hc.eptr)) ||
+          (rc = up(&cent, hc.cent)) || (rc = up(&tq, hc.tq)) || (rc = up(&ownq, hc.ownq)) || (rc = up(&gsl, hc.gsl)) ||
+          (rc = up(&wdst, hc.wdst)) || (rc = up(&w2dst, hc.w2dst)))
         return rc;
-      if ((rc = ws_alloc(ws, &C.A1, (size_t)hc.nb * kCQ)) ||
-          (rc = ws_alloc(ws, &C.G1, (size_t)hc.ng * hc.gsz * hc.gsz)) ||
-          (rc = ws_alloc(ws, &C.A2, (size_t)hc.ng * hc.ng)) || (rc = ws_alloc(ws, &C.rc1, (size_t)hc.nb)) ||
-          (rc = ws_alloc(ws, &C.z1, (size_t)hc.nb)) ||
+      if ((rc = ws_alloc(ws, &C.tslot, nel)) || (rc = ws_alloc(ws, &C.cown, (size_t)ws.NB)) ||
+          (rc = ws_alloc(ws, &C.cval, hc.cent.size())) || (rc = ws_alloc(ws, &C.A1, nq)) ||
+          (rc = ws_alloc(ws, &C.G1, (size_t)hc.ng * hc.nov * hc.gsz)) ||
+          (rc = ws_alloc(ws, &C.A2, (size_t)hc.ng * hc.ng)) ||
+          (rc = ws_alloc(ws, &C.M, (size_t)hc.ng * hc.ng * hc.gsz)) || (rc = ws_alloc(ws, &C.z1, (size_t)hc.nb)) ||
+          (rc = ws_alloc(ws, &R.rcs, nq)) || (rc = ws_alloc(ws, &R.r2c, (size_t)hc.g2ptr.back())) ||
           (rc = ws_alloc(ws, &ws.RV, (size_t)(o.ksp_restart + 1) * hc.nb)))
         return rc;
+      R.cown = C.cown; R.eptr = eptr; R.cent = cent; R.cval = C.cval; R.tq = tq; R.ownq = ownq;
+      R.wdst = wdst; R.gsl = gsl; R.w2dst = w2dst;
       C.status = ws.status;
+      // slots of rcs and A1 that no neighbour writes stay 0
+      k_fill<<<nblk((int64_t)nq, 256), 256, 0, ctx->stream>>>((int64_t)nq, R.rcs, 0.0);
+      k_fill<<<nblk((int64_t)nq, 256), 256, 0, ctx->stream>>>((int64_t)nq, C.A1, 0.0);
+      k_coarse_tslot<<<nblk((int64_t)nel, 256), 256, 0, ctx->stream>>>(ws.NB, ctx->jell_w, hb.bs, ws.bj.d_row,
+                                                                       ctx->d_jrp, ctx->d_jcols, C.tslot);
+      if (hipGetLastError() != hipSuccess || hipStreamSynchronize(ctx->stream) != hipSuccess) {
+        set_error("coarse correction set-up failed");
+        return TDYHIP_ERR_HIP;
+      }
       if (hipStreamCreateWithFlags(&ws.side, hipStreamNonBlocking) != hipSuccess) ws.side = nullptr;
       if (!ws.side || hipEventCreateWithFlags(&ws.fork_ev, hipEventDisableTiming) != hipSuccess ||
           hipEventCreateWithFlags(&ws.join_ev, hipEventDisableTiming) != hipSuccess) {
@@ -640,7 +785,8 @@ static double bytes_factor(const SolverWS &ws, size_t tv) {
 template <class TV>
 struct KBufs {
   TV *V, *w, *z, *b, *fac, *Jk, *part;
-  double *dH, *dcs, *dsn, *dg, *dy, *rc1;
+  double *dH, *dcs, *dsn, *dg, *dy;
+  CoarseRestrict cr;  // rcs null without the coarse correction
   GmresDev *gd;
   int m, nch;
   int64_t N;
@@ -654,7 +800,7 @@ static KBufs<TV> kbufs(tdyhip_ctx *ctx, int m) {
   k.Jk = std::is_same<TV, double>::value ? (TV *)ws.J : (TV *)ws.Jk;
   k.part = (TV *)ws.partial;
   k.dH = ws.hs; k.dcs = k.dH + (size_t)(m + 1) * m; k.dsn = k.dcs + m; k.dg = k.dsn + m; k.dy = k.dg + (m + 1);
-  k.rc1 = ws.coarse ? ws.cl.rc1 : nullptr;
+  if (ws.coarse) k.cr = ws.cl.R;
   k.gd = ws.gdev;
   k.m = m;
   k.N = ws.n;
@@ -662,28 +808,30 @@ static KBufs<TV> kbufs(tdyhip_ctx *ctx, int m) {
   return k;
 }
 
-// level-1/2 solve of the coarse correction: z1 per block
+// the coarse solve: z1 per block
 static CoarseDot coarse_dot(const SolverWS &ws) {
   const CoarseLayout &C = ws.cl;
   CoarseDot cd;
-  cd.ng = C.ng; cd.gsz = C.gsz; cd.gmem = C.gmem; cd.G1 = C.G1; cd.A2 = C.A2; cd.rc1 = C.rc1; cd.z1 = C.z1;
+  cd.parts = C.ng * coarse_parts(C.gsz); cd.g2max = C.g2max;
+  cd.ng = C.ng; cd.gsz = C.gsz; cd.nov = C.nov; cd.gmem = C.gmem; cd.gov = C.gov; cd.G1 = C.G1; cd.M = C.M;
+  cd.rcs = C.R.rcs; cd.r2c = C.R.r2c; cd.g2ptr = C.g2ptr; cd.z1 = C.z1;
   cd.RV = ws.RV; cd.rv_ld = C.nb;
   return cd;
 }
 
 static void coarse_solve(tdyhip_ctx *ctx, const int *stp, hipStream_t st) {
   const CoarseLayout &C = ctx->ws->cl;
-  KT(ctx, st, "k_coarse_level1", (double)C.ng * C.gsz * C.gsz * 8 + (double)C.nb * 24 + (double)C.ng * C.ng * 8,
-     k_coarse_level1<<<C.ng, kL1Threads, 0, st>>>(coarse_dot(*ctx->ws), stp));
+  KT(ctx, st, "k_coarse_level1", (double)C.ng * C.gsz * (C.nov + C.ng) * 8 + (double)C.nb * 24,
+     k_coarse_level1<<<C.ng * coarse_parts(C.gsz), kL1Threads, 0, st>>>(coarse_dot(*ctx->ws), stp));
 }
 
 // out = M^-1 in (block-Jacobi ILU(0), plus the coarse correction when on)
 template <class TV>
 static void pc_apply(tdyhip_ctx *ctx, const KBufs<TV> &k, const TV *in, TV *out, const int *stp, hipStream_t st) {
   SolverWS &ws = *ctx->ws;
-  if (ws.bj.bs == 64) KT(ctx, st, "k_bj_apply", bytes_apply(ws, sizeof(TV)), k_bj_apply<TV, 64><<<ws.bj.nblocks, 64, 0, st>>>(ws.bj, k.fac, in, out, stp, k.rc1));
-  else if (ws.bj.bs == 256) KT(ctx, st, "k_bj_apply", bytes_apply(ws, sizeof(TV)), k_bj_apply<TV, 256><<<ws.bj.nblocks, 256, 0, st>>>(ws.bj, k.fac, in, out, stp, k.rc1));
-  else KT(ctx, st, "k_bj_apply", bytes_apply(ws, sizeof(TV)), k_bj_apply<TV, 512><<<ws.bj.nblocks, 512, 0, st>>>(ws.bj, k.fac, in, out, stp, k.rc1));
+  if (ws.bj.bs == 64) KT(ctx, st, "k_bj_apply", bytes_apply(ws, sizeof(TV)), k_bj_apply<TV, 64><<<ws.bj.nblocks, 64, 0, st>>>(ws.bj, k.fac, in, out, stp, k.cr));
+  else if (ws.bj.bs == 256) KT(ctx, st, "k_bj_apply", bytes_apply(ws, sizeof(TV)), k_bj_apply<TV, 256><<<ws.bj.nblocks, 256, 0, st>>>(ws.bj, k.fac, in, out, stp, k.cr));
+  else KT(ctx, st, "k_bj_apply", bytes_apply(ws, sizeof(TV)), k_bj_apply<TV, 512><<<ws.bj.nblocks, 512, 0, st>>>(ws.bj, k.fac, in, out, stp, k.cr));
   if (!ws.coarse) return;
   const CoarseLayout &C = ws.cl;
   coarse_solve(ctx, stp, st);
@@ -706,11 +854,11 @@ static void resid_pc_apply(tdyhip_ctx *ctx, const KBufs<TV> &k, const double *bv
 #define TDY_RESID(TI, EC)                                                                                           \
   do {                                                                                                             \
     if (ws.bj.bs == 64)                                                                                            \
-      KT(ctx, st, "k_bj_resid_apply", by, k_bj_resid_apply<TV, 64, TI><<<nb, 64, 0, st>>>(ws.bj, W, EC, ws.J, y, bvec, k.fac, out, stp, k.rc1)); \
+      KT(ctx, st, "k_bj_resid_apply", by, k_bj_resid_apply<TV, 64, TI><<<nb, 64, 0, st>>>(ws.bj, W, EC, ws.J, y, bvec, k.fac, out, stp, k.cr)); \
     else if (ws.bj.bs == 256)                                                                                      \
-      KT(ctx, st, "k_bj_resid_apply", by, k_bj_resid_apply<TV, 256, TI><<<nb, 256, 0, st>>>(ws.bj, W, EC, ws.J, y, bvec, k.fac, out, stp, k.rc1)); \
+      KT(ctx, st, "k_bj_resid_apply", by, k_bj_resid_apply<TV, 256, TI><<<nb, 256, 0, st>>>(ws.bj, W, EC, ws.J, y, bvec, k.fac, out, stp, k.cr)); \
     else                                                                                                           \
-      KT(ctx, st, "k_bj_resid_apply", by, k_bj_resid_apply<TV, 512, TI><<<nb, 512, 0, st>>>(ws.bj, W, EC, ws.J, y, bvec, k.fac, out, stp, k.rc1)); \
+      KT(ctx, st, "k_bj_resid_apply", by, k_bj_resid_apply<TV, 512, TI><<<nb, 512, 0, st>>>(ws.bj, W, EC, ws.J, y, bvec, k.fac, out, stp, k.cr)); \
   } while (0)
   if (i16) TDY_RESID(int16_t, ws.d_ecol16);
   else TDY_RESID(int32_t, ws.d_ecol);
@@ -737,15 +885,15 @@ static void spmv_apply(tdyhip_ctx *ctx, const KBufs<TV> &k, const TV *u, TV *vj,
   const NormArgs nv = na ? *na : NormArgs{};
   GmresDev *gd = k.gd;
   const TV *Jk = k.Jk, *fac = k.fac;
-  double *rc1 = k.rc1;
+  const CoarseRestrict cr = k.cr;
 #define TDY_SPMV(TI, EC, NRM)                                                                                      \
   do {                                                                                                             \
     if (ws.bj.bs == 64)                                                                                            \
-      KT(ctx, st, "k_bj_spmv_apply", by, k_bj_spmv_apply<TV, 64, TI, NRM><<<nb, 64, 0, st>>>(ws.bj, ws.NB, W, EC, Jk, u, gd, vj, fac, out, stp, rc1, nv, rv)); \
+      KT(ctx, st, "k_bj_spmv_apply", by, k_bj_spmv_apply<TV, 64, TI, NRM><<<nb, 64, 0, st>>>(ws.bj, ws.NB, W, EC, Jk, u, gd, vj, fac, out, stp, cr, nv, rv)); \
     else if (ws.bj.bs == 256)                                                                                      \
-      KT(ctx, st, "k_bj_spmv_apply", by, k_bj_spmv_apply<TV, 256, TI, NRM><<<nb, 256, 0, st>>>(ws.bj, ws.NB, W, EC, Jk, u, gd, vj, fac, out, stp, rc1, nv, rv)); \
+      KT(ctx, st, "k_bj_spmv_apply", by, k_bj_spmv_apply<TV, 256, TI, NRM><<<nb, 256, 0, st>>>(ws.bj, ws.NB, W, EC, Jk, u, gd, vj, fac, out, stp, cr, nv, rv)); \
     else                                                                                                           \
-      KT(ctx, st, "k_bj_spmv_apply", by, k_bj_spmv_apply<TV, 512, TI, NRM><<<nb, 512, 0, st>>>(ws.bj, ws.NB, W, EC, Jk, u, gd, vj, fac, out, stp, rc1, nv, rv)); \
+      KT(ctx, st, "k_bj_spmv_apply", by, k_bj_spmv_apply<TV, 512, TI, NRM><<<nb, 512, 0, st>>>(ws.bj, ws.NB, W, EC, Jk, u, gd, vj, fac, out, stp, cr, nv, rv)); \
   } while (0)
   if (ws.d_ecol16) {
     if (na) TDY_SPMV(int16_t, ws.d_ecol16, true);
@@ -777,31 +925,42 @@ static void gmres_prep(tdyhip_ctx *ctx, const tdyhip_solver_opts &o, const doubl
     KT(ctx, st, "k_convert_J", (double)ws.nnz * (8 + sizeof(TV)),
        k_convert<double, TV><<<(unsigned)((ws.nnz + 255) / 256), 256, 0, st>>>(ws.nnz, ws.J, k.Jk));
   k_gmres_init<<<1, 1, 0, st>>>(k.gd, ws.status, o.ksp_max_it);
-  // coarse correction: Galerkin rows, group inverses and the level-2 inverse
-  // for this Jacobian; each application then adds its prolongation to the
-  // block-Jacobi result (the restriction is fused into the ILU sweeps).  Its
-  // latency-bound kernels run on the side stream, beside the factor, and
-  // join before the first preconditioner application.  With the FP64
-  // factor, whose workgroups leave no CU room for the group inverses' LDS,
-  // the rows and group inverses run first and only the one-workgroup level-2
-  // inverse goes beside it.
+  // coarse correction: column sums and Galerkin rows, the groups' overlapped
+  // inverses, the level-2 inverse and its product with them for this
+  // Jacobian.  The column sums and group inverses run first (the factor's
+  // workgroups fill the wavefront slots, so beside it they would start as it
+  // drains: 1223 against 390 us at 442,368 rows in FP32); the one-workgroup
+  // level-2 inverse and the product go beside the factor on the side stream
+  // and join before the first preconditioner application.
   const CoarseLayout &C = ws.cl;
   auto rows_groups = [&](hipStream_t cs) {
     const int W = ctx->jell_w;
-    const double brows = (double)ws.NB * W * (8 + 1) + (double)C.nb * kCQ * (4 + 8);
-    if (ws.bj.bs == 64) KT(ctx, cs, "k_coarse_rows", brows, k_coarse_rows<64><<<C.nb, 64, 0, cs>>>(C, ws.NB, W, ws.J));
-    else if (ws.bj.bs == 256) KT(ctx, cs, "k_coarse_rows", brows, k_coarse_rows<256><<<C.nb, 256, 0, cs>>>(C, ws.NB, W, ws.J));
-    else KT(ctx, cs, "k_coarse_rows", brows, k_coarse_rows<512><<<C.nb, 512, 0, cs>>>(C, ws.NB, W, ws.J));
-    KT(ctx, cs, "k_coarse_groups", (double)C.nb * kCQ * 16, k_coarse_groups<<<C.ng, kGroupThreads, 0, cs>>>(C));
+    const double brows = (double)ws.NB * W * (8 + 4) + (double)C.nb * kCQ * (4 + 8);
+#define TDY_COLS(BS)                                                                                                \
+  do {                                                                                                             \
+    if (ws.d_ecol16)                                                                                               \
+      KT(ctx, cs, "k_coarse_cols", brows, k_coarse_cols<BS, int16_t><<<C.nb, BS, 0, cs>>>(C, W, ws.bj.bs == 64 ? 6 : ws.bj.bs == 256 ? 8 : 9, ws.bj.d_row, ws.d_perm, ws.d_ecol16, ws.bj.d_pat, ws.J)); \
+    else                                                                                                           \
+      KT(ctx, cs, "k_coarse_cols", brows, k_coarse_cols<BS, int32_t><<<C.nb, BS, 0, cs>>>(C, W, ws.bj.bs == 64 ? 6 : ws.bj.bs == 256 ? 8 : 9, ws.bj.d_row, ws.d_perm, ws.d_ecol, ws.bj.d_pat, ws.J)); \
+  } while (0)
+    if (ws.bj.bs == 64) TDY_COLS(64);
+    else if (ws.bj.bs == 256) TDY_COLS(256);
+    else TDY_COLS(512);
+#undef TDY_COLS
+    if (C.nov <= 64) KT(ctx, cs, "k_coarse_groups", (double)C.nb * kCQ * 16, k_coarse_groups<64><<<C.ng, TiledGJ<64>::NT, 0, cs>>>(C));
+    else KT(ctx, cs, "k_coarse_groups", (double)C.nb * kCQ * 16, k_coarse_groups<kOV><<<C.ng, TiledGJ<kOV>::NT, 0, cs>>>(C));
   };
-  const bool early = ws.coarse && sizeof(TV) == 8;
-  if (early) rows_groups(st);
+  if (ws.coarse) rows_groups(st);
   const bool side = ws.coarse && hipEventRecord(ws.fork_ev, st) == hipSuccess &&
                     hipStreamWaitEvent(ws.side, ws.fork_ev, 0) == hipSuccess;
   if (ws.coarse) {
     const hipStream_t cs = side ? ws.side : st;
-    if (!early) rows_groups(cs);
-    KT(ctx, cs, "k_coarse_invert", (double)C.ng * C.ng * 16, k_coarse_invert<<<1, 1024, 0, cs>>>(C));
+    if (C.ng <= 64) KT(ctx, cs, "k_coarse_invert", (double)C.ng * C.ng * 16, k_coarse_invert<64><<<1, TiledGJ<64>::NT, 0, cs>>>(C));
+    else KT(ctx, cs, "k_coarse_invert", (double)C.ng * C.ng * 16, k_coarse_invert<kNG><<<1, TiledGJ<kNG>::NT, 0, cs>>>(C));
+const double bfold = (double)C.ng * C.ng * C.gsz * 8;
+    if (C.gsz <= 4) KT(ctx, cs, "k_coarse_fold", bfold, k_coarse_fold<2, 32><<<C.ng, kFoldThreads, 0, cs>>>(C));
+    else if (C.gsz <= 16) KT(ctx, cs, "k_coarse_fold", bfold, k_coarse_fold<8, 32><<<C.ng, kFoldThreads, 0, cs>>>(C));
+    else KT(ctx, cs, "k_coarse_fold", bfold, k_coarse_fold<32, 16><<<C.ng, kFoldThreads, 0, cs>>>(C));
   }
   if (ws.bj.bs == 64) KT(ctx, st, "k_bj_factor", bytes_factor(ws, sizeof(TV)), k_bj_factor<TV, 64><<<ws.bj.nblocks, FactorLanes<64>::NT, 0, st>>>(ws.bj, ws.J, k.fac, ws.status));
   else if (ws.bj.bs == 256) KT(ctx, st, "k_bj_factor", bytes_factor(ws, sizeof(TV)), k_bj_factor<TV, 256><<<ws.bj.nblocks, FactorLanes<256>::NT, 0, st>>>(ws.bj, ws.J, k.fac, ws.status));
@@ -839,8 +998,8 @@ static void gmres_cycle(tdyhip_ctx *ctx, const tdyhip_solver_opts &o, const doub
   GmresDev *gd = k.gd;
   const int *stop = &gd->done;
   // With the coarse correction, w = w_bj + P z1 (w_bj the block-Jacobi part
-  // the fused matvec leaves): the multi-dot's first cd.ng workgroups solve for
-  // z1 and add the coarse terms RV_i . z1 of h_i = V_i . w (RV_i the block sums
+  // the fused matvec leaves, which also forms the coarse right-hand side): the
+  // multi-dot's first cd.parts workgroups solve for z1 and add the coarse terms RV_i . z1 of h_i = V_i . w (RV_i the block sums
   // of V_i, formed by the matvec that formed V_i), the other workgroups the
   // terms V_i . w_bj; the update kernel adds the prolongation P z1 to w.
   Prolong pro;
@@ -851,7 +1010,7 @@ static void gmres_cycle(tdyhip_ctx *ctx, const tdyhip_solver_opts &o, const doub
     pro.bs_log2 = ws.bj.bs == 64 ? 6 : ws.bj.bs == 256 ? 8 : 9;
     cd = coarse_dot(ws);
   }
-  const int pst = nch + cd.ng;  // partials per vector: the coarse groups', then the row chunks'
+  const int pst = nch + cd.parts;  // partials per vector: the coarse parts', then the row chunks'
   const unsigned gmd = (unsigned)pst;
   // The unnormalised Arnoldi vector alternates between w and z: step j reads
   // it from one and leaves the next in the other.
@@ -871,9 +1030,15 @@ static void gmres_cycle(tdyhip_ctx *ctx, const tdyhip_solver_opts &o, const doub
     const Prolong none;
     const double bmd = (double)(j + 2) * N * sizeof(TV);
     // FP32: two passes of 16 beyond 16 vectors (67 VGPRs against 83 for one of 32)
-    if (j < 8) KT(ctx, st, "k_mdot", bmd, k_mdot<TV, 8><<<gmd, kRedBlock, 0, st>>>(N, j + 1, k.V, N, ov, k.part, pst, none, stop, cd));
-    else if (j < 16 || sizeof(TV) == 4) KT(ctx, st, "k_mdot", bmd, k_mdot<TV, 16><<<gmd, kRedBlock, 0, st>>>(N, j + 1, k.V, N, ov, k.part, pst, none, stop, cd));
-    else KT(ctx, st, "k_mdot", bmd, k_mdot<TV, 32><<<gmd, kRedBlock, 0, st>>>(N, j + 1, k.V, N, ov, k.part, pst, none, stop, cd));
+#define TDY_MDOT(NS)                                                                                                 \
+  do {                                                                                                             \
+    if (cd.parts) KT(ctx, st, "k_mdot", bmd, k_mdot<TV, NS, true><<<gmd, kRedBlock, 0, st>>>(N, j + 1, k.V, N, ov, k.part, pst, none, stop, cd)); \
+    else KT(ctx, st, "k_mdot", bmd, k_mdot<TV, NS, false><<<gmd, kRedBlock, 0, st>>>(N, j + 1, k.V, N, ov, k.part, pst, none, stop, cd)); \
+  } while (0)
+    if (j < 8) TDY_MDOT(8);
+    else if (j < 16 || sizeof(TV) == 4) TDY_MDOT(16);
+    else TDY_MDOT(32);
+#undef TDY_MDOT
     k_reduce_partials<TV><<<j + 1, kRedBlock, 0, st>>>(j + 1, pst, k.part, ws.h, stop);
     const double bmx = (double)(j + 3) * N * sizeof(TV) + (pro.z1 ? (double)N * 4 : 0.0);
     KT(ctx, st, "k_maxpy_norm", bmx, k_maxpy_norm<TV><<<nch, kRedBlock, 0, st>>>(N, j + 1, k.V, N, ws.h, ov, k.part, stop, pro));

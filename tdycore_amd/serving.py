@@ -114,6 +114,9 @@ def footprint_bytes(nc, nf, nv, nbnd, rows, krylov_fp32=True, restart=30):
     # block-Jacobi tables and factor (rows = the block layout's row count)
     ws = 64 * nc + 4 * nc + rows * 27 * (8 + 4) + (restart + 5) * nc * tv + rows * (548 + 27 * tv)
     ws += rows * 27 * 4  # FP32 copy of the Jacobian (kept in both precisions)
+    # coarse correction: slot maps, column sums and their lists per row; lists,
+    # basis sums and inverses per block (a server's blocks hold 256 rows); tables
+    ws += rows * (27 + 27 + 8 + 24) + -(-rows // 256) * (3600 + 8 * (restart + 1)) + (2 << 20)
     return int(ctx + max(setup_tmp, ws) + (1 << 20))
 
 

@@ -1,0 +1,125 @@
+"""The coarse correction of the block-Jacobi preconditioner (pc_coarse) by what
+it is for: GMRES iterations.  The first Newton system of a layered box is
+solved on the device with one Newton iteration allowed, and on the CPU by
+left-preconditioned GMRES(30) with block ILU(0) followed by an exact solve of
+the Galerkin operator A1 on what block Jacobi leaves,
+
+    w = BJ^-1 r,   M^-1 r = w + P A1^-1 P^T (r - A w).
+
+Up to 128 blocks the device's coarse solve is A1^-1 too, so the counts agree
+to the rounding at the stop test (one iteration, two in FP32).  Beyond, groups
+of blocks with one layer of overlap stand in for A1^-1; a wrong entry in one
+of its lists costs far more than the quarter allowed here.  Blocks: whole and
+cut bricks, a single block, a group of one block, overlaps within 64 blocks
+and beyond, and the default breadth-first partition."""
+import numpy as np
+import pytest
+
+from tdycore_amd import meshgen as mg
+from tdycore_amd import workloads
+
+pytestmark = pytest.mark.gpu
+
+DAY = 86400.0
+
+
+def _ilu0(A, part):
+    """Block ILU(0) factors: per block its rows and the dense LU on the pattern."""
+    out = []
+    for b in range(part.max() + 1):
+        rows = np.nonzero(part == b)[0]
+        M = A[rows][:, rows].toarray()
+        pat = A[rows][:, rows].copy()
+        pat.data[:] = 1.0
+        pat = pat.toarray() != 0
+        for i in range(len(rows)):
+            for k in np.nonzero(pat[i, :i])[0]:
+                M[i, k] /= M[k, k]
+                q = pat[i, k + 1:] & pat[k, k + 1:]
+                M[i, k + 1:][q] -= M[i, k] * M[k, k + 1:][q]
+        out.append((rows, np.linalg.inv(np.tril(M, -1) + np.eye(len(rows))), np.linalg.inv(np.triu(M))))
+    return out
+
+
+def _iterations(A, F, part, rtol=1e-5, restart=30):
+    import scipy.sparse as sp
+    n, nb = A.shape[0], int(part.max()) + 1
+    fac = _ilu0(A, part)
+    R = sp.csr_matrix((np.ones(n), (part, np.arange(n))), shape=(nb, n))
+    A1 = np.linalg.inv((R @ A @ R.T).toarray())
+
+    def M(r):
+        w = np.empty(n)
+        for rows, L, U in fac:
+            w[rows] = U @ (L @ r[rows])
+        return w + R.T @ (A1 @ (R @ (r - A @ w)))
+
+    x, its, tol = np.zeros(n), 0, None
+    while True:
+        r = M(F - A @ x)
+        beta = np.linalg.norm(r)
+        tol = rtol * beta if tol is None else tol
+        if beta <= tol:
+            return its
+        V, H = [r / beta], np.zeros((restart + 1, restart))
+        for j in range(restart):
+            w = M(A @ V[j])
+            H[:j + 1, j] = [v @ w for v in V]
+            w = w - np.array(V).T @ H[:j + 1, j]
+            H[j + 1, j] = np.linalg.norm(w)
+            V.append(w / H[j + 1, j])
+            its += 1
+            e1 = np.zeros(j + 2)
+            e1[0] = beta
+            y, *_ = np.linalg.lstsq(H[:j + 2, :j + 1], e1, rcond=None)
+            if np.linalg.norm(e1 - H[:j + 2, :j + 1] @ y) <= tol:
+                break
+        x = x + np.array(V[:len(y)]).T @ y
+        if np.linalg.norm(e1 - H[:j + 2, :j + 1] @ y) <= tol:
+            return its
+
+
+@pytest.mark.parametrize("n,brick,block,fp32", [
+    ((5, 4, 3), (8, 8, 4), 256, 0),      # one cut block
+    ((16, 16, 8), (4, 4, 4), 64, 0),     # 32 blocks: a group per block
+    ((13, 11, 9), (4, 4, 4), 64, 1),     # cut bricks
+    ((24, 20, 12), (8, 8, 4), 256, 0),
+    ((17, 18, 9), (8, 8, 8), 512, 0),
+    ((32, 32, 8), (4, 4, 4), 64, 0),     # 128 blocks: the last size with a group per block
+    ((33, 32, 8), (4, 4, 4), 64, 0),     # 144 blocks: groups of two
+    ((24, 24, 16), (2, 2, 2), 64, 0),    # 1152 blocks: overlaps of more than 64 blocks
+    ((24, 24, 16), (2, 2, 2), 64, 1),
+    ((12, 12, 10), None, 64, 0),         # breadth-first blocks
+])
+def test_iterations_match_an_exact_coarse_solve(n, brick, block, fp32):
+    import torch
+    from pyoracle import Oracle
+    from tdycore_amd.mpfao import MPFAO
+    print(f"[case] coarse correction {n} brick={brick} fp32={fp32}", flush=True)
+    P = workloads.layered_box_problem(*n)
+    args = (P["mesh"], P["face_bc"], P["K"], P["porosity"], P["Sr"])
+    o = Oracle(*args, **P["kw"])
+    o.set_dtime(DAY)
+    o.snes_presolve(P["U0"])
+    F = o.snes_function(P["U0"])
+    A = o.jac_to_csr(o.snes_jacobian(P["U0"])).tocsr()
+    g = MPFAO(*args, **P["kw"])
+    if brick:
+        g.set_pc_partition(mg.brick_partition(P["mesh"], *brick))
+    U = torch.tensor(P["U0"], device="cuda", dtype=torch.float64)
+    g.SetDtime(DAY)
+    g.SNESPreSolve(U)
+    st = {c: g.newton_snes(U.clone(), g.solver_options(snes_max_it=1, pc_block=block, krylov_fp32=fp32, pc_coarse=c))
+          for c in (0, 1)}
+    g.close()
+    got = st[1]["linear_its"]
+    if brick is None:  # the partition is the library's own: fewer iterations than without the correction
+        assert 0 < got < st[0]["linear_its"]
+        return
+    part = np.unique(mg.brick_partition(P["mesh"], *brick), return_inverse=True)[1].ravel()
+    want = _iterations(A, F, part)
+    print(f"  {got} iterations, exact coarse solve {want}, one level {st[0]['linear_its']}", flush=True)
+    if part.max() < 128:
+        assert abs(got - want) <= (2 if fp32 else 1)
+    else:
+        assert want - 2 <= got <= 1.25 * want + 2
