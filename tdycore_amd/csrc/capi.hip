@@ -1186,7 +1186,7 @@ int tdyhip_recover_velocity(tdyhip_ctx *ctx, const double *U, double *vel, int32
   a.ccell = ctx->d_ccell; a.vdcol = ctx->d_vdcol; a.Tgen = ctx->d_Tgen;
   a.bnd_cell = ctx->d_bnd_cell; a.U = U; a.cell_z = ctx->d_cell_z; a.pbnd_fn = ctx->d_pbnd_fn;
   a.face_area = ctx->d_face_area; a.vel = vel; a.count = count;
-  k_velocity<<<nblk(ctx->nf, 256), 256, 0, st>>>(a);
+  k_velocity<<<nblk(a.nrows, 256), 256, 0, st>>>(a);
   HIPCHK(hipGetLastError());
   return 0;
 }
