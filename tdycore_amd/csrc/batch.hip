@@ -68,8 +68,8 @@ static int fused_eval(tdyhip_batch *b, int table, std::vector<BatchMember *> &ms
   const int n = (int)ms.size();
   if (n == 0) return 0;
   SegProblem *hp = b->h_prob[table];
-  SegBlocks s_state{}, s_bnd{}, s_rows{}, s_gather{}, s_jac{};
-  s_state.nseg = s_bnd.nseg = s_rows.nseg = s_gather.nseg = s_jac.nseg = n;
+  SegBlocks s_state{}, s_rows{}, s_gather{}, s_jac{};
+  s_state.nseg = s_rows.nseg = s_gather.nseg = s_jac.nseg = n;
   for (int i = 0; i < n; i++) {
     tdyhip_ctx *ctx = ms[i]->ctx;
     SolverWS &ws = *ctx->ws;
@@ -82,8 +82,7 @@ static int fused_eval(tdyhip_batch *b, int table, std::vector<BatchMember *> &ms
                : gather_args(ctx, 1, 0.0, nullptr, rof(ms[i]), nullptr, false, nullptr, 0);
     p.cj = cell_jac_args(ctx, ws.bj.d_row, ws.NB);
     p.stop = stopof(ms[i]);
-    s_state.start[i + 1] = s_state.start[i] + nblk(ctx->nc, 256);
-    s_bnd.start[i + 1] = s_bnd.start[i] + nblk(ctx->nbnd, 256);
+    s_state.start[i + 1] = s_state.start[i] + nblk(ctx->nc + ctx->nbnd, 256);
     s_rows.start[i + 1] = s_rows.start[i] + nblk((int64_t)4 * ctx->nf, kRowBlock);
     s_gather.start[i + 1] = s_gather.start[i] + nblk(ctx->nc, kGatherBlock);
     s_jac.start[i + 1] = s_jac.start[i] + nblk(ws.NB, kCellJacCells);
@@ -97,7 +96,6 @@ static int fused_eval(tdyhip_batch *b, int table, std::vector<BatchMember *> &ms
     k_seg_cell_jac<<<(unsigned)s_jac.start[n], kCellJacBlock, 0, b->st>>>(dp, s_jac);
   } else {
     k_seg_state<<<(unsigned)s_state.start[n], 256, 0, b->st>>>(dp, s_state);
-    if (s_bnd.start[n] > 0) k_seg_bnd_state<<<(unsigned)s_bnd.start[n], 256, 0, b->st>>>(dp, s_bnd);
     k_seg_rows<<<(unsigned)s_rows.start[n], kRowBlock, 0, b->st>>>(dp, s_rows);
     k_seg_cell_gather<<<(unsigned)s_gather.start[n], kGatherBlock, 0, b->st>>>(dp, s_gather);
   }

@@ -240,8 +240,7 @@ static RowArgs row_args(tdyhip_ctx *ctx, const double *U) {
   a.nc = ctx->nc; a.nrows = (int64_t)4 * ctx->nf; a.pref = ctx->pref;
   a.face_cells = ctx->d_face_cells; a.face_verts = ctx->d_face_verts; a.face_flags = ctx->d_face_flags;
   a.vcols = ctx->d_vcols; a.T = ctx->d_T; a.G = ctx->d_G; a.U = U; a.Pbnd = ctx->d_Pbnd;
-  a.rho = ctx->d_rho; a.ukvr = ctx->d_ukvr; a.drho = ctx->d_drho; a.dukvr = ctx->d_dukvr;
-  a.rho_bnd = ctx->d_rho_bnd; a.ukvr_bnd = ctx->d_ukvr_bnd;
+  a.st = ctx->d_st;
   a.flux = ctx->launch_flux ? ctx->launch_flux : ctx->d_flux;
   a.stop = ctx->launch_stop;
   return a;
@@ -268,7 +267,7 @@ static CellStateArgs cell_state_args(tdyhip_ctx *ctx, int form, const double *U,
   CellStateArgs a;
   a.nc = ctx->nc; a.sp = state_params(ctx, form, 0.0);
   a.U = U; a.Udot = Udot; a.phi = ctx->d_phi; a.Sr = ctx->d_Sr; a.vol = ctx->d_cell_vol; a.accum_prev = ctx->d_accum_prev;
-  a.rho = ctx->d_rho; a.ukvr = ctx->d_ukvr; a.drho = ctx->d_drho; a.dukvr = ctx->d_dukvr;
+  a.st = ctx->d_st;
   a.dM = ctx->d_dM; a.d2M = ctx->d_d2M; a.acc = ctx->d_acc;
   return a;
 }
@@ -276,15 +275,14 @@ static BndStateArgs bnd_state_args(tdyhip_ctx *ctx, int form, const double *U) {
   BndStateArgs a;
   a.nbnd = ctx->nbnd; a.sp = state_params(ctx, form, 0.0);
   a.U = U; a.bnd_cell = ctx->d_bnd_cell; a.Sr = ctx->d_Sr; a.pbnd_fn = ctx->d_pbnd_fn;
-  a.Pbnd = ctx->d_Pbnd; a.ukvr_bnd = ctx->d_ukvr_bnd;
+  a.Pbnd = ctx->d_Pbnd; a.st = ctx->d_st + ctx->nc;
   return a;
 }
 
 // state (+boundary) at U
 static int launch_state(tdyhip_ctx *ctx, int form, const double *U, const double *Udot, hipStream_t st) {
   KT(ctx, st, "k_cell_state", bytes_state(ctx),
-     k_cell_state<<<nblk(ctx->nc, 256), 256, 0, st>>>(cell_state_args(ctx, form, U, Udot)));
-  if (ctx->nbnd > 0) k_bnd_state<<<nblk(ctx->nbnd, 256), 256, 0, st>>>(bnd_state_args(ctx, form, U));
+     k_cell_state<<<nblk(ctx->nc + ctx->nbnd, 256), 256, 0, st>>>(cell_state_args(ctx, form, U, Udot), bnd_state_args(ctx, form, U)));
   HIPCHK(hipGetLastError());
   return 0;
 }
@@ -639,15 +637,14 @@ static int setup_general(tdyhip_ctx *ctx, const tdyhip_mesh *m, const tdyhip_mat
     ctx->has_pbnd_fn = true;
     if ((rc = dupload(ctx, &ctx->d_pbnd_fn, mat->p_bnd_fn, nbnd))) return done(rc);
   }
-  for (double **q : {&ctx->d_rho, &ctx->d_ukvr, &ctx->d_drho, &ctx->d_dukvr, &ctx->d_dM, &ctx->d_d2M, &ctx->d_acc,
-                     &ctx->d_accum_prev})
+  if ((rc = dalloc(ctx, &ctx->d_st, (size_t)nc + nbnd))) return done(rc);
+  for (double **q : {&ctx->d_dM, &ctx->d_d2M, &ctx->d_acc, &ctx->d_accum_prev})
     if ((rc = dalloc(ctx, q, nc))) return done(rc);
-  for (double **q : {&ctx->d_Pbnd, &ctx->d_ukvr_bnd, &ctx->d_rho_bnd})
-    if ((rc = dalloc(ctx, q, std::max(nbnd, 1)))) return done(rc);
+  if ((rc = dalloc(ctx, &ctx->d_Pbnd, (size_t)std::max(nbnd, 1)))) return done(rc);
   {
     double rb, d1, d2;  // boundary rho frozen at (Pref, Tref) (tdympfao.c:297-336)
     water_density(ctx->density_type, ctx->pref, rb, d1, d2);
-    if (nbnd > 0) k_fill<<<nblk(nbnd, 256), 256, 0, st>>>(nbnd, ctx->d_rho_bnd, rb);
+    if (nbnd > 0) k_bnd_init<<<nblk(nbnd, 256), 256, 0, st>>>(nbnd, ctx->d_st + nc, rb);
   }
   if (hipStreamSynchronize(st) != hipSuccess) { set_error("general setup failed"); return done(TDYHIP_ERR_HIP); }
   ctx->jnnz = g->jrp[nc];
@@ -669,16 +666,14 @@ static int launch_flux_general(tdyhip_ctx *ctx, int form, double shift, const do
   a.face_cells = ctx->d_face_cells; a.face_flags = ctx->d_face_flags;
   a.rtoff = ctx->d_rtoff; a.rinfo = ctx->d_rinfo; a.roc = ctx->d_roc; a.rdc = ctx->d_rdc;
   a.ccell = ctx->d_ccell; a.vdcol = ctx->d_vdcol;
-  a.T = ctx->d_Tgen; a.G = ctx->d_G; a.U = U; a.Pbnd = ctx->d_Pbnd; a.rho = ctx->d_rho; a.ukvr = ctx->d_ukvr;
-  a.drho = ctx->d_drho; a.dukvr = ctx->d_dukvr; a.rho_bnd = ctx->d_rho_bnd; a.ukvr_bnd = ctx->d_ukvr_bnd;
+  a.T = ctx->d_Tgen; a.G = ctx->d_G; a.U = U; a.Pbnd = ctx->d_Pbnd; a.st = ctx->d_st;
   a.flux = ctx->launch_flux ? ctx->launch_flux : ctx->d_flux; a.D = ctx->d_Dgen;
   a.stop = ctx->launch_stop;
   if (ctx->d_vblk) {
     GenBlkArgs b;
     b.pref = ctx->pref; b.vblk = ctx->d_vblk; b.brow = ctx->d_brow;
     b.face_cells = ctx->d_face_cells; b.face_flags = ctx->d_face_flags; b.ccell = ctx->d_ccell; b.vdcol = ctx->d_vdcol;
-    b.T = ctx->d_Tgen; b.G = ctx->d_G; b.U = U; b.Pbnd = ctx->d_Pbnd; b.rho = ctx->d_rho; b.ukvr = ctx->d_ukvr;
-    b.drho = ctx->d_drho; b.dukvr = ctx->d_dukvr; b.rho_bnd = ctx->d_rho_bnd; b.ukvr_bnd = ctx->d_ukvr_bnd;
+    b.T = ctx->d_Tgen; b.G = ctx->d_G; b.U = U; b.Pbnd = ctx->d_Pbnd; b.st = ctx->d_st; b.nc = ctx->nc;
     b.flux = ctx->launch_flux ? ctx->launch_flux : ctx->d_flux; b.D = ctx->d_Dgen;
     b.stop = ctx->launch_stop;
     const unsigned gv = (unsigned)ctx->nv;
@@ -887,7 +882,14 @@ int tdyhip_create(const tdyhip_mesh *m, const tdyhip_materials *mat, tdyhip_ctx 
           if (j == 8 || cnt[j] == 3) { set_error("hexahedron with a corner not on exactly three of its faces"); return fail(TDYHIP_ERR_ARG); }
           uint32_t &w = crow[(size_t)c * 8 + j];
           w |= (uint32_t)(lf * 4 + q) << (5 * cnt[j]);
-          if (m->face_cells[(size_t)2 * f] == c) w |= 1u << (18 + cnt[j]);
+          const int up = m->face_cells[(size_t)2 * f], dn = m->face_cells[(size_t)2 * f + 1];
+          if (up == c) w |= 1u << (18 + cnt[j]);
+          const int o = up == c ? dn : up;
+          if (o >= 0) {
+            int oi = 0;
+            while (oi < 7 && topo.vcols[(size_t)v * kMaxCols + oi] != o) oi++;
+            w |= (uint32_t)oi << (21 + 3 * cnt[j]);
+          }
           cnt[j]++;
         }
       }
@@ -917,11 +919,10 @@ int tdyhip_create(const tdyhip_mesh *m, const tdyhip_materials *mat, tdyhip_ctx 
   }
   if ((rc = dalloc(ctx, &ctx->d_T, (size_t)kMaxCols * nrows))) return fail(rc);
   if ((rc = dalloc(ctx, &ctx->d_G, (size_t)nrows))) return fail(rc);
-  for (double **p : {&ctx->d_rho, &ctx->d_ukvr, &ctx->d_drho, &ctx->d_dukvr, &ctx->d_dM, &ctx->d_d2M, &ctx->d_acc,
-                     &ctx->d_accum_prev})
+  if ((rc = dalloc(ctx, &ctx->d_st, (size_t)nc + nbnd))) return fail(rc);
+  for (double **p : {&ctx->d_dM, &ctx->d_d2M, &ctx->d_acc, &ctx->d_accum_prev})
     if ((rc = dalloc(ctx, p, nc))) return fail(rc);
-  for (double **p : {&ctx->d_Pbnd, &ctx->d_ukvr_bnd, &ctx->d_rho_bnd})
-    if ((rc = dalloc(ctx, p, nbnd))) return fail(rc);
+  if ((rc = dalloc(ctx, &ctx->d_Pbnd, (size_t)nbnd))) return fail(rc);
   if ((rc = dalloc(ctx, &ctx->d_flux, (size_t)nrows))) return fail(rc);
 
   // setup temporaries
@@ -975,7 +976,7 @@ int tdyhip_create(const tdyhip_mesh *m, const tdyhip_materials *mat, tdyhip_ctx 
   {
     double rb, d1, d2;
     water_density(ctx->density_type, ctx->pref, rb, d1, d2);
-    if (nbnd > 0) k_fill<<<nblk(nbnd, 256), 256, 0, st>>>(nbnd, ctx->d_rho_bnd, rb);
+    if (nbnd > 0) k_bnd_init<<<nblk(nbnd, 256), 256, 0, st>>>(nbnd, ctx->d_st + nc, rb);
   }
   if (hipGetLastError() != hipSuccess || hipStreamSynchronize(st) != hipSuccess) {
     set_error("setup kernels failed");
@@ -1233,7 +1234,7 @@ int tdyhip_trans_csr(const tdyhip_ctx *ctx, int32_t *rowptr, int32_t *cols, doub
       for (int k = 0; k < kMaxCols; k++) {
         const int col = ctx->h_vcols[(size_t)v * kMaxCols + k];
         if (col < 0) continue;
-        const double val = T[(size_t)k * nrows + r];
+        const double val = T[(size_t)trans_index(nrows, k, r)];
         int64_t p = n;
         while (p > base && cols[p - 1] > col) { cols[p] = cols[p - 1]; vals[p] = vals[p - 1]; p--; }
         cols[p] = col; vals[p] = val; n++;

@@ -3,8 +3,8 @@
 //  k_cell_state   per cell: van Genuchten / Mualem / EOS state, rho, Kr/mu and their
 //                 pressure derivatives, and the accumulation term (TS or SNES form)
 //                 (TDyUpdateState_Richards_MPFAO, src/fv/mpfao/tdympfao.c:2527-2594;
-//                  tdympfao_ts.c:191-212; tdympfao_snes.c:19-30, 112-123)
-//  k_bnd_state    per boundary face: P_bnd and Kr/mu on the boundary
+//                  tdympfao_ts.c:191-212; tdympfao_snes.c:19-30, 112-123);
+//                 per boundary face: P_bnd and Kr/mu on the boundary
 //                 (tdympfao_utils.c:24-99, 690-759)
 //  k_rows         per flux row (face*4 + subface): T.P from the vertex's columns,
 //                 upwinded rho^2 kr/mu flux (TDyMPFAOIFunction_Vertices, tdympfao_ts.c:12-150)
@@ -15,8 +15,8 @@
 //                 accumulation diagonal, optionally the residual as well
 //
 // Flux rows are stored face-major (row = face*4 + subface), the reference's
-// Trans_mat row numbering; T is an 8-wide ELL block stored column-major so that
-// consecutive lanes read consecutive addresses.
+// Trans_mat row numbering; T is an 8-wide ELL block stored by pairs of columns
+// (trans_index) so that consecutive lanes read consecutive 16-byte pairs.
 #include "tdyhip_internal.h"
 #include "tdyhip_math.h"
 
@@ -38,7 +38,8 @@ struct CellStateArgs {
   int nc;
   StateParams sp;
   const double *U, *Udot, *phi, *Sr, *vol, *accum_prev;
-  double *rho, *ukvr, *drho, *dukvr, *dM, *d2M, *acc;
+  FlowState *st;
+  double *dM, *d2M, *acc;
 };
 
 __device__ inline void cell_state(const CellStateArgs &a, int c) {
@@ -55,10 +56,7 @@ __device__ inline void cell_state(const CellStateArgs &a, int c) {
   double rho, drho, d2rho;
   water_density(sp.density_type, p, rho, drho, d2rho);
   const double vis = kViscosity, dvis = 0.0;
-  a.rho[c] = rho;
-  a.ukvr[c] = Kr / vis;
-  a.drho[c] = drho;
-  a.dukvr[c] = dKr * dS / vis - Kr / (vis * vis) * dvis;
+  a.st[c] = FlowState{rho, Kr / vis, drho, dKr * dS / vis - Kr / (vis * vis) * dvis};
   const double ph = a.phi[c];
   const double dM = drho * ph * S + rho * ph * dS;
   const double d2M = 2.0 * dS * drho * ph + S * d2rho * ph + d2S * rho * ph;
@@ -69,12 +67,6 @@ __device__ inline void cell_state(const CellStateArgs &a, int c) {
   } else {
     a.acc[c] = rho * ph * S * a.vol[c] / (sp.dyn ? sp.dyn[0] : sp.dtime) - a.accum_prev[c];
   }
-}
-
-__global__ void k_cell_state(CellStateArgs a) {
-  if (a.sp.stop && *a.sp.stop) return;
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c < a.nc) cell_state(a, c);
 }
 
 // rho phi S V / dt at Uprev (TDyMPFAOSNESPreSolve, tdympfao_snes.c:32-64)
@@ -113,7 +105,8 @@ struct BndStateArgs {
   const double *U;
   const int32_t *bnd_cell;
   const double *Sr, *pbnd_fn;
-  double *Pbnd, *ukvr_bnd;
+  double *Pbnd;
+  FlowState *st;  // boundary entries; rho and the zero derivatives are written at setup
 };
 
 __device__ inline void bnd_state(const BndStateArgs &a, int b) {
@@ -128,13 +121,24 @@ __device__ inline void bnd_state(const BndStateArgs &a, int b) {
   double Kr, dKr;
   const double cc[4] = {sp.c0, sp.c1, sp.c2, sp.c3};
   mualem_kr(sp.vg_m, sp.x0, sp.x1, sp.dx, cc, Se, Kr, dKr);
-  a.ukvr_bnd[b] = Kr / kViscosity;
+  a.st[b].ukvr = Kr / kViscosity;
 }
 
-__global__ void k_bnd_state(BndStateArgs a) {
+// State of cell i < nc, or of boundary face i - nc (which depends on U alone,
+// so both share a launch).
+__device__ inline void state_entry(const CellStateArgs &a, const BndStateArgs &b, int i) {
+  if (i < a.nc) cell_state(a, i);
+  else if (i - a.nc < b.nbnd) bnd_state(b, i - a.nc);
+}
+__global__ void k_cell_state(CellStateArgs a, BndStateArgs b) {
   if (a.sp.stop && *a.sp.stop) return;
+  state_entry(a, b, blockIdx.x * blockDim.x + threadIdx.x);
+}
+
+// boundary rho frozen at (Pref, Tref) (tdympfao.c:297-336)
+__global__ void k_bnd_init(int nbnd, FlowState *__restrict__ st, double rho) {
   const int b = blockIdx.x * blockDim.x + threadIdx.x;
-  if (b < a.nbnd) bnd_state(a, b);
+  if (b < nbnd) st[b] = FlowState{rho, 0.0, 0.0, 0.0};
 }
 
 struct RowArgs {
@@ -149,8 +153,7 @@ struct RowArgs {
   const double *G;
   const double *U;
   const double *Pbnd;
-  const double *rho, *ukvr, *drho, *dukvr;
-  const double *rho_bnd, *ukvr_bnd;
+  const FlowState *st;
   double *flux;
   const int *stop;
 };
@@ -182,29 +185,11 @@ __device__ inline double row_flux(double TP, double den, double G, double ukvr, 
   fluxm += -(den * den) * ukvr * G;
   return zero ? 0.0 : fluxm;
 }
-// d(flux)/d(p of column k), negated (the up cell's residual gets -Jac, the
-// down cell's +Jac, tdympfao_ts.c:439-444); 0 for padding and boundary-pressure
-// columns, which never enter J, and for a row that carries no flux
-__device__ inline void row_derivs(int nc, const double (&T)[kMaxCols], const int (&ck)[kMaxCols], int up, int dn,
-                                  double TP, double den, double G, double ukvr, bool upwind_up, bool zero,
-                                  double dr_up, double dr_dn, double du, double (&jr)[kMaxCols]) {
-  const double dden_up = up >= 0 ? 0.5 * dr_up : 0.0;
-  const double dden_dn = dn >= 0 ? 0.5 * dr_dn : 0.0;
-  const double dukvr_up = (upwind_up && up >= 0) ? du : 0.0;
-  const double dukvr_dn = (!upwind_up && dn >= 0) ? du : 0.0;
-  // the up (down) cell's column adds the derivatives of rho_bar and kr/mu
-  const double Aup = dden_up * ukvr * TP + den * dukvr_up * TP;
-  const double Dup = 2 * den * dden_up * ukvr * G, Eup = (den * den) * dukvr_up * G;
-  const double Adn = dden_dn * ukvr * TP + den * dukvr_dn * TP;
-  const double Ddn = 2 * den * dden_dn * ukvr * G, Edn = (den * den) * dukvr_dn * G;
-#pragma unroll
-  for (int k = 0; k < kMaxCols; k++) {
-    const int col = ck[k];
-    const double C = den * ukvr * T[k];
-    const double Ju = ((Aup + C) + Dup) + Eup, Jd = ((Adn + C) + Ddn) + Edn;
-    const double Jac = col == up ? Ju : (col == dn ? Jd : C);
-    jr[k] = (zero || col < 0 || col >= nc) ? 0.0 : -Jac;
-  }
+// what d(flux) adds in the column of one side of the row beyond rho_bar
+// lambda T: the derivatives dden of rho_bar and dl of kr/mu by that side's
+// pressure (0 for a boundary side), negated like the flux
+__device__ inline double side_extra(double TP, double den, double G, double ukvr, double dden, double dl) {
+  return (dden * ukvr + den * dl) * TP + (2.0 * dden * ukvr + den * dl) * (den * G);
 }
 
 // the columns of vertex v and their pressures (padding reads U[0], unused)
@@ -220,6 +205,24 @@ __device__ inline void vertex_columns(const RowArgs &a, int v, int (&ck)[kMaxCol
   }
 }
 
+// the row's transmissibilities, four 16-byte loads
+__device__ inline void row_trans(const double *__restrict__ T, int64_t nrows, int64_t r, double (&t)[kMaxCols]) {
+  const double2 *p = reinterpret_cast<const double2 *>(T) + r;
+#pragma unroll
+  for (int k = 0; k < kMaxCols / 2; k++) {
+    const double2 q = p[k * nrows];
+    t[2 * k] = q.x;
+    t[2 * k + 1] = q.y;
+  }
+}
+// rho and kr / mu of a face side
+__device__ inline double2 side_state(const FlowState *st, int i) {
+  return *reinterpret_cast<const double2 *>(&st[i].rho);
+}
+__device__ inline double2 side_derivs(const FlowState *st, int i) {
+  return *reinterpret_cast<const double2 *>(&st[i].drho);
+}
+
 // Thread per flux row: the residual's flux rows (the Jacobian is assembled by
 // k_cell_jac, one pass per cell).
 __device__ inline void flux_row(const RowArgs &a, int64_t r) {
@@ -232,15 +235,14 @@ __device__ inline void flux_row(const RowArgs &a, int64_t r) {
     int ck[kMaxCols];
     double P[kMaxCols], T[kMaxCols];
     vertex_columns(a, a.face_verts[r], ck, P);
-#pragma unroll
-    for (int k = 0; k < kMaxCols; k++) T[k] = a.T[(int64_t)k * a.nrows + r];
+    row_trans(a.T, a.nrows, r, T);
+    const double2 su = side_state(a.st, flow_index(a.nc, up)), sd = side_state(a.st, flow_index(a.nc, dn));
     const double G = a.G[r];
-    const double den = row_den(*(up >= 0 ? a.rho + up : a.rho_bnd + (-up - 1)),
-                               *(dn >= 0 ? a.rho + dn : a.rho_bnd + (-dn - 1)));
+    const double den = row_den(su.x, sd.x);
     const double TP = row_tp(T, ck, P);
     const bool upwind_up = row_upwind_up(TP, den, G);
     const int uw = upwind_up ? up : dn;
-    const double ukvr = *(uw >= 0 ? a.ukvr + uw : a.ukvr_bnd + (-uw - 1));
+    const double ukvr = upwind_up ? su.y : sd.y;
     // a seepage face's boundary side carries no flux while its pressure is at
     // or below the reference pressure
     const bool zero = uw < 0 && (fl & kFaceSeepage) && a.Pbnd[-uw - 1] <= a.pref;
@@ -267,7 +269,8 @@ struct GenRowArgs {
   const int32_t *face_cells;
   const uint8_t *face_flags;
   const int32_t *rtoff, *rinfo, *roc, *rdc, *ccell, *vdcol;
-  const double *T, *G, *U, *Pbnd, *rho, *ukvr, *drho, *dukvr, *rho_bnd, *ukvr_bnd;
+  const double *T, *G, *U, *Pbnd;
+  const FlowState *st;
   double *flux, *D;
   const int *stop;
 };
@@ -294,20 +297,15 @@ __global__ void __launch_bounds__(256) k_rows_general(GenRowArgs a) {
   for (int j = 0; j < ndir; j++) TP += Tr[ncell + j] * a.Pbnd[dcols[j]];
   const int up = a.face_cells[2 * f], dn = a.face_cells[2 * f + 1];
   double den = 0.0;
-  den += up >= 0 ? a.rho[up] : a.rho_bnd[-up - 1];
-  den += dn >= 0 ? a.rho[dn] : a.rho_bnd[-dn - 1];
+  const FlowState su = a.st[flow_index(a.nc, up)], sd = a.st[flow_index(a.nc, dn)];
+  den += su.rho;
+  den += sd.rho;
   den *= 0.5;
   const double G = a.G[r];
   const bool upwind_up = (TP + den * G < 0.0);
   const int uw = upwind_up ? up : dn;
-  double ukvr;
-  bool zero = false;
-  if (uw >= 0) {
-    ukvr = a.ukvr[uw];
-  } else {
-    ukvr = a.ukvr_bnd[-uw - 1];
-    if ((fl & kFaceSeepage) && a.Pbnd[-uw - 1] <= a.pref) zero = true;
-  }
+  const double ukvr = upwind_up ? su.ukvr : sd.ukvr;
+  const bool zero = uw < 0 && (fl & kFaceSeepage) && a.Pbnd[-uw - 1] <= a.pref;
   if (WITH_R) {
     double fluxm = 0.0;
     if (!zero) {
@@ -317,11 +315,8 @@ __global__ void __launch_bounds__(256) k_rows_general(GenRowArgs a) {
     a.flux[r] = fluxm;
   }
   if (WITH_J) {
-    const double dden_up = up >= 0 ? 0.5 * a.drho[up] : 0.0;
-    const double dden_dn = dn >= 0 ? 0.5 * a.drho[dn] : 0.0;
-    double dukvr_up = 0.0, dukvr_dn = 0.0;
-    if (upwind_up) { if (up >= 0) dukvr_up = a.dukvr[up]; }
-    else { if (dn >= 0) dukvr_dn = a.dukvr[dn]; }
+    const double dden_up = 0.5 * su.drho, dden_dn = 0.5 * sd.drho;
+    const double dukvr_up = upwind_up ? su.dukvr : 0.0, dukvr_dn = upwind_up ? 0.0 : sd.dukvr;
 #pragma unroll 4
     for (int j = 0; j < ncell; j++) {
       const int col = cols[j];
@@ -373,13 +368,15 @@ struct GenGatherArgs {
 // arithmetic as k_rows_general, entry by entry.
 constexpr int kBlkRows = 64;  // most flux rows of one vertex block (checked at setup)
 struct GenBlkArgs {
+  int nc;
   double pref;
   const int32_t *vblk;  // per vertex: T offset, rows, cells, Dirichlet columns, cell offset, Dirichlet offset, row offset
   const int32_t *brow;  // flux row of each block row, blocks in vertex order
   const int32_t *face_cells;
   const uint8_t *face_flags;
   const int32_t *ccell, *vdcol;
-  const double *T, *G, *U, *Pbnd, *rho, *ukvr, *drho, *dukvr, *rho_bnd, *ukvr_bnd;
+  const double *T, *G, *U, *Pbnd;
+  const FlowState *st;
   double *flux, *D;
   const int *stop;
 };
@@ -412,20 +409,15 @@ __global__ void __launch_bounds__(64) k_rows_general_blk(GenBlkArgs a) {
       for (int j = 0; j < ndir; j++) TP += Tr[ncell + j] * a.Pbnd[dcols[j]];
       const int up = a.face_cells[2 * f], dn = a.face_cells[2 * f + 1];
       double den = 0.0;
-      den += up >= 0 ? a.rho[up] : a.rho_bnd[-up - 1];
-      den += dn >= 0 ? a.rho[dn] : a.rho_bnd[-dn - 1];
+      const FlowState su = a.st[flow_index(a.nc, up)], sd = a.st[flow_index(a.nc, dn)];
+      den += su.rho;
+      den += sd.rho;
       den *= 0.5;
       const double G = a.G[r];
       const bool upwind_up = (TP + den * G < 0.0);
       const int uw = upwind_up ? up : dn;
-      double ukvr;
-      bool zero = false;
-      if (uw >= 0) {
-        ukvr = a.ukvr[uw];
-      } else {
-        ukvr = a.ukvr_bnd[-uw - 1];
-        if ((fl & kFaceSeepage) && a.Pbnd[-uw - 1] <= a.pref) zero = true;
-      }
+      const double ukvr = upwind_up ? su.ukvr : sd.ukvr;
+      const bool zero = uw < 0 && (fl & kFaceSeepage) && a.Pbnd[-uw - 1] <= a.pref;
       if (WITH_R) {
         double fluxm = 0.0;
         if (!zero) {
@@ -435,12 +427,10 @@ __global__ void __launch_bounds__(64) k_rows_general_blk(GenBlkArgs a) {
         a.flux[r] = fluxm;
       }
       if (WITH_J) {
-        double dukvr_up = 0.0, dukvr_dn = 0.0;
-        if (upwind_up) { if (up >= 0) dukvr_up = a.dukvr[up]; }
-        else { if (dn >= 0) dukvr_dn = a.dukvr[dn]; }
+        const double dukvr_up = upwind_up ? su.dukvr : 0.0, dukvr_dn = upwind_up ? 0.0 : sd.dukvr;
         s_tp[t] = TP; s_den[t] = den; s_ukvr[t] = ukvr; s_G[t] = G;
-        s_ddu[t] = up >= 0 ? 0.5 * a.drho[up] : 0.0;
-        s_ddd[t] = dn >= 0 ? 0.5 * a.drho[dn] : 0.0;
+        s_ddu[t] = 0.5 * su.drho;
+        s_ddd[t] = 0.5 * sd.drho;
         s_dku[t] = dukvr_up; s_dkd[t] = dukvr_dn;
         s_up[t] = up; s_dn[t] = dn;
       }
@@ -659,8 +649,9 @@ __global__ void __launch_bounds__(kGatherBlock) k_cell_gather(GatherArgs a) {
 // padding) and the XCD-grouped workgroup numbering arrange.
 //   crow[c*8 + j]: the corner's three rows as 5-bit (face slot * 4 + sub-face)
 //                  codes in face order (bits 0-4, 5-9, 10-14), the cell's index
-//                  in the region of the corner's vertex (bits 15-17), and
-//                  whether the cell is each row's up cell (bits 18, 19, 20)
+//                  in the region of the corner's vertex (bits 15-17),
+//                  whether the cell is each row's up cell (bits 18, 19, 20),
+//                  and the index of each row's other cell there (bits 21-29)
 //   cell_verts[c*8 + j]: the corner's vertex
 //   jslot[v*64 + li*8 + k]: slot of column k of vertex v's region in the row
 //                  of the region's cell li (255: not a cell column)
@@ -716,12 +707,12 @@ __device__ inline void cell_jac_block(const RowArgs &ra, const GatherArgs &a, co
     double P[kMaxCols];
     vertex_columns(ra, v, ck, P);
     const uint64_t w = *reinterpret_cast<const uint64_t *>(cj.jslot + (int64_t)v * 64 + li * 8);
-    // the three rows' loads in two batches: what the faces fix, then what the
-    // upwind side fixes (a no-flow face's row runs at the cell on both sides,
-    // every read in range, and is dropped)
+    // the three rows' loads together, both sides' states (a no-flow face's row
+    // runs at the cell on both sides, every read in range, and is dropped)
     int up[3], dn[3];
     bool noflow[3], seep[3];
-    double T[3][kMaxCols], G[3], rup[3], rdn[3], drup[3], drdn[3];
+    double T[3][kMaxCols], G[3];
+    double2 su[3], sd2[3], du2[3], dd2[3];  // rho and kr / mu, and their derivatives, of the two sides
 #pragma unroll
     for (int m = 0; m < 3; m++) {
       const int f = fr[m];
@@ -732,13 +723,13 @@ __device__ inline void cell_jac_block(const RowArgs &ra, const GatherArgs &a, co
       seep[m] = (fl & kFaceSeepage) != 0;
       up[m] = noflow[m] ? c : ud.x;
       dn[m] = noflow[m] ? c : ud.y;
-#pragma unroll
-      for (int k = 0; k < kMaxCols; k++) T[m][k] = ra.T[(int64_t)k * ra.nrows + r];
+      row_trans(ra.T, ra.nrows, r, T[m]);
       G[m] = ra.G[r];
-      rup[m] = *(up[m] >= 0 ? ra.rho + up[m] : ra.rho_bnd + (-up[m] - 1));
-      rdn[m] = *(dn[m] >= 0 ? ra.rho + dn[m] : ra.rho_bnd + (-dn[m] - 1));
-      drup[m] = ra.drho[up[m] >= 0 ? up[m] : 0];
-      drdn[m] = ra.drho[dn[m] >= 0 ? dn[m] : 0];
+      const int iu = flow_index(ra.nc, up[m]), id = flow_index(ra.nc, dn[m]);
+      su[m] = side_state(ra.st, iu);
+      sd2[m] = side_state(ra.st, id);
+      du2[m] = side_derivs(ra.st, iu);
+      dd2[m] = side_derivs(ra.st, id);
     }
     double TP[3], den[3], ukvr[3], du[3], pb[3];
     bool upw[3];
@@ -746,31 +737,45 @@ __device__ inline void cell_jac_block(const RowArgs &ra, const GatherArgs &a, co
 #pragma unroll
     for (int m = 0; m < 3; m++) {
       TP[m] = row_tp(T[m], ck, P);
-      den[m] = row_den(rup[m], rdn[m]);
+      den[m] = row_den(su[m].x, sd2[m].x);
       upw[m] = row_upwind_up(TP[m], den[m], G[m]);
       uw[m] = upw[m] ? up[m] : dn[m];
     }
 #pragma unroll
     for (int m = 0; m < 3; m++) {
-      ukvr[m] = *(uw[m] >= 0 ? ra.ukvr + uw[m] : ra.ukvr_bnd + (-uw[m] - 1));
-      du[m] = ra.dukvr[uw[m] >= 0 ? uw[m] : 0];
+      ukvr[m] = upw[m] ? su[m].y : sd2[m].y;
+      du[m] = upw[m] ? du2[m].y : dd2[m].y;
       pb[m] = ra.Pbnd[uw[m] < 0 ? -uw[m] - 1 : 0];  // Pbnd always holds at least one entry
     }
-    double sum[kMaxCols];
+    // Row m adds s (rho_bar lambda) T to the corner's columns, s the sign of
+    // its flux in this cell's residual (0 for a row that carries none); the
+    // derivatives of rho_bar and kr/mu go to the columns of its two sides, this
+    // cell's own (column li) and the other cell's (tdympfao_ts.c:439-444).
+    // Boundary-pressure and padding columns gather values nobody reads.
+    double sum[kMaxCols], self = 0.0, other[3];
 #pragma unroll
     for (int k = 0; k < kMaxCols; k++) sum[k] = 0.0;
 #pragma unroll
     for (int m = 0; m < 3; m++) {
-      const bool zero = (uw[m] < 0) & seep[m] & (pb[m] <= ra.pref);
-      double jr[kMaxCols];
-      row_derivs(ra.nc, T[m], ck, up[m], dn[m], TP[m], den[m], G[m], ukvr[m], upw[m], zero, drup[m], drdn[m], du[m], jr);
+      const bool zero = noflow[m] | ((uw[m] < 0) & seep[m] & (pb[m] <= ra.pref));
       const bool is_up = (code >> (18 + m)) & 1;
+      const double s = zero ? 0.0 : is_up ? -1.0 : 1.0;
+      const double sl = s * (den[m] * ukvr[m]);
 #pragma unroll
-      for (int k = 0; k < kMaxCols; k++) sum[k] = noflow[m] ? sum[k] : (is_up ? sum[k] + jr[k] : sum[k] - jr[k]);
+      for (int k = 0; k < kMaxCols; k++) sum[k] = fma(sl, T[m][k], sum[k]);
+      const double xu = side_extra(TP[m], den[m], G[m], ukvr[m], 0.5 * du2[m].x, upw[m] ? du2[m].y : 0.0);
+      const double xd = side_extra(TP[m], den[m], G[m], ukvr[m], 0.5 * dd2[m].x, upw[m] ? 0.0 : dd2[m].y);
+      self += s * (is_up ? xu : xd);
+      other[m] = s * (is_up ? xd : xu);
       if (WITH_R) sf[lfq[m]][cl] = noflow[m] ? 0.0 : row_flux(TP[m], den[m], G[m], ukvr[m], zero);
     }
 #pragma unroll
     for (int k = 0; k < kMaxCols; k++) sd[k][t] = sum[k];
+    // (each lane adds to its own entries: plain LDS adds, in order)
+    atomicAdd(&sd[li][t], self);
+#pragma unroll
+    for (int m = 0; m < 3; m++)
+      if (((code >> (18 + m)) & 1 ? dn[m] : up[m]) >= 0) atomicAdd(&sd[(code >> (21 + 3 * m)) & 7][t], other[m]);
     sw[t] = w;
   }
   // A cell's eight lanes share a wavefront, whose LDS operations run in
@@ -848,14 +853,7 @@ struct SegProblem {  // one request's arguments of every fused launch
 __global__ void __launch_bounds__(256) k_seg_state(const SegProblem *__restrict__ P, SegBlocks sb) {
   const int s = seg_find(sb, blockIdx.x);
   if (P[s].stop && *P[s].stop) return;
-  const int c = (int)((blockIdx.x - sb.start[s]) * 256 + threadIdx.x);
-  if (c < P[s].cs.nc) cell_state(P[s].cs, c);
-}
-__global__ void __launch_bounds__(256) k_seg_bnd_state(const SegProblem *__restrict__ P, SegBlocks sb) {
-  const int s = seg_find(sb, blockIdx.x);
-  if (P[s].stop && *P[s].stop) return;
-  const int b = (int)((blockIdx.x - sb.start[s]) * 256 + threadIdx.x);
-  if (b < P[s].bs.nbnd) bnd_state(P[s].bs, b);
+  state_entry(P[s].cs, P[s].bs, (int)((blockIdx.x - sb.start[s]) * 256 + threadIdx.x));
 }
 __global__ void __launch_bounds__(kRowBlock) k_seg_rows(const SegProblem *__restrict__ P, SegBlocks sb) {
   const int s = seg_find(sb, blockIdx.x);
@@ -948,10 +946,10 @@ __global__ void __launch_bounds__(256) k_velocity(VelArgs a) {
       const int4 c0 = vc[0], c1 = vc[1];
       const int ck[kMaxCols] = {c0.x, c0.y, c0.z, c0.w, c1.x, c1.y, c1.z, c1.w};
       double T[kMaxCols], P[kMaxCols], z[kMaxCols];
+      row_trans(a.T, a.nrows, r, T);
 #pragma unroll
       for (int k = 0; k < kMaxCols; k++) {
         const int c = ck[k] < 0 || ck[k] >= a.nc ? 0 : ck[k];
-        T[k] = a.T[(int64_t)k * a.nrows + r];
         P[k] = a.U[c];
         z[k] = a.cell_z[c];
       }

@@ -45,8 +45,8 @@ static int fuser_launch(tdyhip_fuser *fz, std::vector<tdyhip_fuser::Req *> &rs) 
   SCHK(hipEventSynchronize(fz->ring_ev[slot]));  // the slot's previous launch has read its table
   SegProblem *hp = fz->h_tab[slot];
   const bool jac = rs[0]->kind == 1;
-  SegBlocks s_state{}, s_bnd{}, s_rows{}, s_gather{}, s_jac{};
-  s_state.nseg = s_bnd.nseg = s_rows.nseg = s_gather.nseg = s_jac.nseg = n;
+  SegBlocks s_state{}, s_rows{}, s_gather{}, s_jac{};
+  s_state.nseg = s_rows.nseg = s_gather.nseg = s_jac.nseg = n;
   for (int i = 0; i < n; i++) {
     tdyhip_ctx *ctx = rs[i]->ctx;
     SolverWS &ws = *ctx->ws;
@@ -59,8 +59,7 @@ static int fuser_launch(tdyhip_fuser *fz, std::vector<tdyhip_fuser::Req *> &rs) 
                : gather_args(ctx, 1, 0.0, nullptr, rs[i]->out, nullptr, false, nullptr, 0);
     p.cj = cell_jac_args(ctx, ws.bj.d_row, ws.NB);
     p.stop = rs[i]->stop;
-    s_state.start[i + 1] = s_state.start[i] + nblk(ctx->nc, 256);
-    s_bnd.start[i + 1] = s_bnd.start[i] + nblk(ctx->nbnd, 256);
+    s_state.start[i + 1] = s_state.start[i] + nblk(ctx->nc + ctx->nbnd, 256);
     s_rows.start[i + 1] = s_rows.start[i] + nblk((int64_t)4 * ctx->nf, kRowBlock);
     s_gather.start[i + 1] = s_gather.start[i] + nblk(ctx->nc, kGatherBlock);
     s_jac.start[i + 1] = s_jac.start[i] + nblk(ws.NB, kCellJacCells);
@@ -72,7 +71,6 @@ static int fuser_launch(tdyhip_fuser *fz, std::vector<tdyhip_fuser::Req *> &rs) 
     k_seg_cell_jac<<<(unsigned)s_jac.start[n], kCellJacBlock, 0, fz->st>>>(dp, s_jac);
   } else {
     k_seg_state<<<(unsigned)s_state.start[n], 256, 0, fz->st>>>(dp, s_state);
-    if (s_bnd.start[n] > 0) k_seg_bnd_state<<<(unsigned)s_bnd.start[n], 256, 0, fz->st>>>(dp, s_bnd);
     k_seg_rows<<<(unsigned)s_rows.start[n], kRowBlock, 0, fz->st>>>(dp, s_rows);
     k_seg_cell_gather<<<(unsigned)s_gather.start[n], kGatherBlock, 0, fz->st>>>(dp, s_gather);
   }

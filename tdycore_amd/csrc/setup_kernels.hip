@@ -264,7 +264,7 @@ __global__ void __launch_bounds__(kTeam * kTeamsPerBlock)
         for (int m = 0; m < 3; m++) cdir -= (cu[m] == nU + j - ncell) ? gu[m] : 0.0;
         t = s + cdir;
       }
-      T[(int64_t)j * nrows + r] = t;
+      T[trans_index(nrows, j, r)] = t;
     }
   }
 }

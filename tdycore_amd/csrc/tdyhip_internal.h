@@ -50,6 +50,21 @@ struct HostTopology {
   bool over_limit = false;        // set with the error when a vertex exceeds the fixed-size limits above
 };
 
+// Flow state of a cell or boundary face, read together by the flux rows: one
+// entry per cell, then one per boundary face (whose derivatives stay 0).
+struct alignas(32) FlowState {
+  double rho, ukvr, drho, dukvr;  // density, kr / mu and their pressure derivatives
+};
+// Place of face side `side` (a cell, or -(b+1) for boundary face b) in it.
+__host__ __device__ inline int flow_index(int nc, int side) { return side >= 0 ? side : nc - side - 1; }
+
+// Transmissibilities of a hexahedral mesh: pairs of columns per flux row, so
+// that a row's 8 columns are four 16-byte loads, each coalesced over rows.
+// Place of column k of row r:
+__host__ __device__ inline int64_t trans_index(int64_t nrows, int k, int64_t r) {
+  return ((k >> 1) * nrows + r) * 2 + (k & 1);
+}
+
 // Builds the host topology; returns an error message or empty string.  A mesh
 // that only exceeds the hexahedral kernels' fixed limits (over_limit) is
 // valid: it takes the general path.
@@ -160,7 +175,7 @@ struct tdyhip_ctx {
 
   // device: discretisation
   int32_t *d_vcols = nullptr;       // nv*kMaxCols
-  double *d_T = nullptr;            // kMaxCols * 4nf (column-major ELL over face-major rows)
+  double *d_T = nullptr;            // kMaxCols * 4nf: trans_index over face-major rows
   double *d_G = nullptr;            // 4nf gravity term
   uint8_t *d_jslot = nullptr;       // nv*64: Jacobian-row slot of (region cell i, column k)
   uint32_t *d_crow = nullptr;       // nc*8: a corner's three flux rows, the cell's region index, its sides
@@ -171,9 +186,9 @@ struct tdyhip_ctx {
   int jell_w = 0;                   // ELL width (longest Jacobian row)
 
   // device: state
-  double *d_rho = nullptr, *d_ukvr = nullptr, *d_drho = nullptr, *d_dukvr = nullptr;
+  tdyhip::FlowState *d_st = nullptr;  // nc + nbnd
   double *d_dM = nullptr, *d_d2M = nullptr, *d_acc = nullptr;
-  double *d_Pbnd = nullptr, *d_ukvr_bnd = nullptr, *d_rho_bnd = nullptr;
+  double *d_Pbnd = nullptr;
   double *d_flux = nullptr;         // 4nf
   double *d_accum_prev = nullptr;   // nc
   double *d_source = nullptr;       // nc source_sink (tdyhip_set_source_sink)
