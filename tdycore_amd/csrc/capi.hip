@@ -598,37 +598,63 @@ static int setup_general(tdyhip_ctx *ctx, const tdyhip_mesh *m, const tdyhip_mat
       (rc = dupload(ctx, &ctx->d_jrp, g->jrp.data(), g->jrp.size())) ||
       (rc = dupload(ctx, &ctx->d_jcols, g->jcols.data(), g->jcols.size())) ||
       (rc = dupload(ctx, &ctx->d_jdiag, g->jdiag.data(), g->jdiag.size())) ||
-      (rc = dalloc(ctx, &ctx->d_Dgen, (size_t)std::max<int64_t>(g->tsize, 1))) ||
+      (rc = dalloc(ctx, &ctx->d_rlam, (size_t)4 * nf)) || (rc = dalloc(ctx, &ctx->d_rside, (size_t)4 * nf)) ||
+      (rc = dalloc(ctx, &ctx->d_nslot, (size_t)6 * nc)) ||
       (rc = dalloc(ctx, &ctx->d_gslot, (size_t)2 * std::max<int64_t>(g->tsize, 1))) ||
       (rc = dalloc(ctx, &ctx->d_flux, (size_t)4 * nf)))
     return done(rc);
   {
-    // vertex blocks for the flux-row kernel: T offset, rows, cells, Dirichlet
-    // columns, cell offset, Dirichlet-column offset, first block row
+    // the flux rows with a block, blocks in vertex order, and the runs of
+    // vertices the row kernel's workgroups take
     const int nv = m->nv;
-    std::vector<int32_t> vb((size_t)nv * 7), br;
+    std::vector<int32_t> br;
+    std::vector<GenRow> bd;
+    std::vector<GenGroup> gr;
+    GenGroup cur{};
     int32_t od = 0;
-    bool fits = true;
-    for (int v = 0; v < nv && fits; v++) {
+    for (int v = 0; v < nv; v++) {
       const int32_t *d = g->vdesc.data() + (size_t)v * 8;
-      const int nface = d[1], of = d[5], nrow = d[7];
-      int32_t *o = vb.data() + (size_t)v * 7;
-      o[0] = d[6]; o[1] = nrow; o[2] = d[0]; o[3] = d[3]; o[4] = d[4]; o[5] = od; o[6] = (int32_t)br.size();
-      if (nrow > kBlkRows || br.size() + (size_t)nrow > (size_t)INT32_MAX) fits = false;
-      br.resize(br.size() + nrow, -1);
+      const int ncell = d[0], nface = d[1], ndir = d[3], of = d[5], nrow = d[7], nB = ncell + ndir;
+      if (nrow > kGrpRows || nrow * nB > kGrpTMax || nB > kGrpCols) {
+        set_error("interaction region too large for the flux-row kernel");
+        return done(TDYHIP_ERR_ARG);
+      }
+      if (cur.nrow + nrow > kGrpRows || cur.nt + nrow * nB > kGrpT || cur.ncell + cur.ndir + nB > kGrpCols) {
+        if (cur.nrow) gr.push_back(cur);
+        cur = GenGroup{};
+      }
+      if (cur.ncell == 0) {
+        cur.row = (int32_t)br.size();
+        cur.t = d[6]; cur.cell = d[4]; cur.dir = od;
+      }
+      const size_t at = br.size();
+      br.resize(at + nrow, -1);
       for (int k = 0; k < nface; k++) {
         const int trow = (g->fb[of + k] >> 16) - 1;
-        if (trow >= 0 && trow < nrow) br[o[6] + trow] = g->frow[of + k];
+        if (trow >= 0 && trow < nrow) br[at + trow] = g->frow[of + k];
       }
-      od += d[3];
+      for (int k = 0; k < nrow; k++)
+        bd.push_back(GenRow{(uint16_t)(cur.nt + k * nB), (uint16_t)cur.ncell, (uint16_t)cur.ndir, (uint8_t)ncell, (uint8_t)ndir});
+      cur.nrow += nrow; cur.nt += nrow * nB; cur.ncell += ncell; cur.ndir += ndir;
+      od += ndir;
     }
-    if (fits && !br.empty() && std::find(br.begin(), br.end(), -1) == br.end() && od == (int32_t)g->vdcol.size()) {
-      if ((rc = dupload(ctx, &ctx->d_vblk, vb.data(), vb.size())) ||
-          (rc = dupload(ctx, &ctx->d_brow, br.data(), br.size())))
-        return done(rc);
-      // rows without a block are never written by the block kernel: their flux stays 0
-      k_fill<<<nblk((int64_t)4 * nf, 256), 256, 0, st>>>((int64_t)4 * nf, ctx->d_flux, 0.0);
+    if (cur.nrow) gr.push_back(cur);
+    for (const GenGroup &q : gr) ctx->grp_nt = std::max(ctx->grp_nt, q.nt);
+    if (std::find(br.begin(), br.end(), -1) != br.end() || od != (int32_t)g->vdcol.size()) {
+      set_error("flux rows of the vertex blocks are incomplete");
+      return done(TDYHIP_ERR_ARG);
     }
+    ctx->ngrp = (int)gr.size();
+    if ((rc = dupload(ctx, &ctx->d_brow, br.data(), br.size())) || (rc = dupload(ctx, &ctx->d_brd, bd.data(), bd.size())) ||
+        (rc = dupload(ctx, &ctx->d_grp, gr.data(), gr.size())))
+      return done(rc);
+    // rows without a block are never written: their flux and factors stay 0
+    const int64_t nr = (int64_t)4 * nf;
+    k_fill<<<nblk(nr, 256), 256, 0, st>>>(nr, ctx->d_flux, 0.0);
+    k_fill<<<nblk(nr, 256), 256, 0, st>>>(nr, ctx->d_rlam, 0.0);
+    k_fill<<<nblk(2 * nr, 256), 256, 0, st>>>(2 * nr, reinterpret_cast<double *>(ctx->d_rside), 0.0);
+    k_gen_neighbour_slots<<<nblk((int64_t)6 * nc, 256), 256, 0, st>>>(nc, ctx->d_cell_faces, ctx->d_face_cells,
+                                                                      ctx->d_jrp, ctx->d_jcols, ctx->d_nslot);
   }
   k_gen_slot_table<<<nblk((int64_t)4 * nf, 256), 256, 0, st>>>((int64_t)4 * nf, ctx->d_face_cells, ctx->d_face_flags,
                                                                 ctx->d_rtoff, ctx->d_rinfo, ctx->d_roc, ctx->d_ccell,
@@ -662,29 +688,18 @@ static int setup_general(tdyhip_ctx *ctx, const tdyhip_mesh *m, const tdyhip_mat
 static int launch_flux_general(tdyhip_ctx *ctx, int form, double shift, const double *U, const double *Udot,
                                double *R, double *J, hipStream_t st, const int32_t *perm, int ell_bs) {
   GenRowArgs a;
-  a.nc = ctx->nc; a.nrows = (int64_t)4 * ctx->nf; a.pref = ctx->pref;
+  a.nc = ctx->nc; a.pref = ctx->pref; a.grp = ctx->d_grp; a.brow = ctx->d_brow; a.brd = ctx->d_brd;
   a.face_cells = ctx->d_face_cells; a.face_flags = ctx->d_face_flags;
-  a.rtoff = ctx->d_rtoff; a.rinfo = ctx->d_rinfo; a.roc = ctx->d_roc; a.rdc = ctx->d_rdc;
   a.ccell = ctx->d_ccell; a.vdcol = ctx->d_vdcol;
   a.T = ctx->d_Tgen; a.G = ctx->d_G; a.U = U; a.Pbnd = ctx->d_Pbnd; a.st = ctx->d_st;
-  a.flux = ctx->launch_flux ? ctx->launch_flux : ctx->d_flux; a.D = ctx->d_Dgen;
+  a.flux = ctx->launch_flux ? ctx->launch_flux : ctx->d_flux; a.lam = ctx->d_rlam; a.side = ctx->d_rside;
   a.stop = ctx->launch_stop;
-  if (ctx->d_vblk) {
-    GenBlkArgs b;
-    b.pref = ctx->pref; b.vblk = ctx->d_vblk; b.brow = ctx->d_brow;
-    b.face_cells = ctx->d_face_cells; b.face_flags = ctx->d_face_flags; b.ccell = ctx->d_ccell; b.vdcol = ctx->d_vdcol;
-    b.T = ctx->d_Tgen; b.G = ctx->d_G; b.U = U; b.Pbnd = ctx->d_Pbnd; b.st = ctx->d_st; b.nc = ctx->nc;
-    b.flux = ctx->launch_flux ? ctx->launch_flux : ctx->d_flux; b.D = ctx->d_Dgen;
-    b.stop = ctx->launch_stop;
-    const unsigned gv = (unsigned)ctx->nv;
-    if (R && J) k_rows_general_blk<true, true><<<gv, 64, 0, st>>>(b);
-    else if (R) k_rows_general_blk<true, false><<<gv, 64, 0, st>>>(b);
-    else k_rows_general_blk<false, true><<<gv, 64, 0, st>>>(b);
-  } else {
-    const unsigned gr = nblk(a.nrows, 256);
-    if (R && J) k_rows_general<true, true><<<gr, 256, 0, st>>>(a);
-    else if (R) k_rows_general<true, false><<<gr, 256, 0, st>>>(a);
-    else k_rows_general<false, true><<<gr, 256, 0, st>>>(a);
+  if (ctx->ngrp > 0) {
+    const unsigned ng = (unsigned)ctx->ngrp;
+    const size_t lds = sizeof(double) * (size_t)(kGrpCols + ctx->grp_nt);
+    if (R && J) k_rows_general<true, true><<<ng, kGrpRows, lds, st>>>(a);
+    else if (R) k_rows_general<true, false><<<ng, kGrpRows, lds, st>>>(a);
+    else k_rows_general<false, true><<<ng, kGrpRows, lds, st>>>(a);
   }
   if (R) {
     GatherArgs ga = gather_args(ctx, form, shift, Udot, R, nullptr, false, nullptr, 0);
@@ -695,9 +710,9 @@ static int launch_flux_general(tdyhip_ctx *ctx, int form, double shift, const do
     gg.nc = ctx->nc; gg.form = form; gg.shift = shift; gg.dtime = ctx->dtime;
     gg.ell_w = ctx->jell_w; gg.perm = perm; gg.jbs = perm ? ell_bs : 1;
     gg.cell_faces = ctx->d_cell_faces; gg.face_cells = ctx->d_face_cells; gg.rtoff = ctx->d_rtoff;
-    gg.rinfo = ctx->d_rinfo; gg.roc = ctx->d_roc; gg.ccell = ctx->d_ccell; gg.jrp = ctx->d_jrp;
-    gg.jcols = ctx->d_jcols; gg.jdiag = ctx->d_jdiag; gg.face_flags = ctx->d_face_flags; gg.gslot = ctx->d_gslot;
-    gg.D = ctx->d_Dgen; gg.dM = ctx->d_dM; gg.d2M = ctx->d_d2M; gg.Udot = Udot; gg.vol = ctx->d_cell_vol; gg.J = J;
+    gg.rinfo = ctx->d_rinfo; gg.jrp = ctx->d_jrp; gg.jdiag = ctx->d_jdiag; gg.face_flags = ctx->d_face_flags;
+    gg.gslot = ctx->d_gslot; gg.nslot = ctx->d_nslot; gg.T = ctx->d_Tgen; gg.lam = ctx->d_rlam; gg.side = ctx->d_rside;
+    gg.dM = ctx->d_dM; gg.d2M = ctx->d_d2M; gg.Udot = Udot; gg.vol = ctx->d_cell_vol; gg.J = J;
     gg.dyn = ctx->launch_dyn; gg.stop = ctx->launch_stop;
     k_gather_general_J<<<nblk(ctx->nc, kGenJBlock / kGenJLanes), kGenJBlock, 0, st>>>(gg);  // kGenJLanes lanes per cell
   }

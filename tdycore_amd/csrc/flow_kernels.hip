@@ -7,7 +7,8 @@
 //                 per boundary face: P_bnd and Kr/mu on the boundary
 //                 (tdympfao_utils.c:24-99, 690-759)
 //  k_rows         per flux row (face*4 + subface): T.P from the vertex's columns,
-//                 upwinded rho^2 kr/mu flux (TDyMPFAOIFunction_Vertices, tdympfao_ts.c:12-150)
+//                 upwinded rho^2 kr/mu flux (TDyMPFAOIFunction_Vertices, tdympfao_ts.c:12-150);
+//                 k_rows_general where a vertex has any number of columns
 //  k_cell_gather  per cell: R = sum over its 6 faces x 4 subfaces (+/- by orientation)
 //                 + accumulation
 //  k_cell_jac     per cell, one pass: the Jacobian row from its 24 flux rows'
@@ -260,207 +261,162 @@ __global__ void __launch_bounds__(kRowBlock) k_rows(RowArgs a) {
 // ---------------------------------------------------------------- general (prism) meshes
 // Flux rows whose vertex has any number of columns: the row's T entries sit in
 // its vertex's block (row-major, columns = the region's cells, then its
-// Dirichlet faces), and its derivatives D in the same place for the cell
-// columns.  The physics is k_rows' (tdympfao_ts.c:12-150, 235-456).
+// Dirichlet faces).  The physics is k_rows' (tdympfao_ts.c:12-150, 235-456).
+//
+// A workgroup per run of consecutive vertices (at most kGrpRows rows, kGrpT
+// entries, kGrpCols columns): their T blocks, one contiguous run, and their
+// columns' pressures go to LDS first, all loads coalesced or gathered once per
+// vertex, then a thread per row sums its own.  Bound by reading T.  The
+// Jacobian needs three numbers of a row beside T itself: rho_bar lambda (0 for
+// a row that carries no flux) and what each side adds in its own column
+// (side_extra); k_gather_general_J forms the derivatives from T again.
+// 200k prisms, residual rows 106 -> 66 us, the Jacobian's 202 -> 84 us against a
+// wavefront per vertex, whose rows strode over T and gathered every pressure
+// themselves (18 of 64 lanes busy), and which wrote every entry's derivative.
+// Rows without a block (a triangle's fourth sub-face, no-flow faces) keep the
+// zeros written at setup.
+// (a single vertex may hold up to 80 x 64 entries: 48 cells, 16 Dirichlet faces)
+constexpr int kGrpRows = 256, kGrpT = 4096, kGrpTMax = 5120, kGrpCols = 512;
+struct GenGroup {       // a run of vertices
+  int32_t row, nrow;    // block rows
+  int32_t t, nt;        // T entries
+  int32_t cell, ncell;  // columns: cells (ccell), then Dirichlet faces (vdcol)
+  int32_t dir, ndir;
+};
+struct GenRow {           // a block row, relative to its group
+  uint16_t t, cell, dir;  // first T entry, first cell, first Dirichlet column
+  uint8_t ncell, ndir;
+};
 struct GenRowArgs {
   int nc;
-  int64_t nrows;
   double pref;
-  const int32_t *face_cells;
-  const uint8_t *face_flags;
-  const int32_t *rtoff, *rinfo, *roc, *rdc, *ccell, *vdcol;
-  const double *T, *G, *U, *Pbnd;
-  const FlowState *st;
-  double *flux, *D;
-  const int *stop;
-};
-
-template <bool WITH_R, bool WITH_J>
-__global__ void __launch_bounds__(256) k_rows_general(GenRowArgs a) {
-  if (a.stop && *a.stop) return;
-  const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (r >= a.nrows) return;
-  const int f = (int)(r >> 2);
-  const uint8_t fl = a.face_flags[f];
-  const int to = a.rtoff[r];
-  if (to < 0 || (fl & kFaceNoFlow)) {
-    if (WITH_R) a.flux[r] = 0.0;
-    return;
-  }
-  const int ncell = a.rinfo[r] & 0xff, ndir = (a.rinfo[r] >> 8) & 0xff;
-  const int32_t *cols = a.ccell + a.roc[r];
-  const int32_t *dcols = a.vdcol + a.rdc[r];
-  const double *Tr = a.T + to;
-  double TP = 0.0;
-#pragma unroll 4
-  for (int j = 0; j < ncell; j++) TP += Tr[j] * a.U[cols[j]];
-  for (int j = 0; j < ndir; j++) TP += Tr[ncell + j] * a.Pbnd[dcols[j]];
-  const int up = a.face_cells[2 * f], dn = a.face_cells[2 * f + 1];
-  double den = 0.0;
-  const FlowState su = a.st[flow_index(a.nc, up)], sd = a.st[flow_index(a.nc, dn)];
-  den += su.rho;
-  den += sd.rho;
-  den *= 0.5;
-  const double G = a.G[r];
-  const bool upwind_up = (TP + den * G < 0.0);
-  const int uw = upwind_up ? up : dn;
-  const double ukvr = upwind_up ? su.ukvr : sd.ukvr;
-  const bool zero = uw < 0 && (fl & kFaceSeepage) && a.Pbnd[-uw - 1] <= a.pref;
-  if (WITH_R) {
-    double fluxm = 0.0;
-    if (!zero) {
-      fluxm = den * ukvr * (-TP);
-      fluxm += -(den * den) * ukvr * G;
-    }
-    a.flux[r] = fluxm;
-  }
-  if (WITH_J) {
-    const double dden_up = 0.5 * su.drho, dden_dn = 0.5 * sd.drho;
-    const double dukvr_up = upwind_up ? su.dukvr : 0.0, dukvr_dn = upwind_up ? 0.0 : sd.dukvr;
-#pragma unroll 4
-    for (int j = 0; j < ncell; j++) {
-      const int col = cols[j];
-      double Jac;
-      if (zero) Jac = 0.0;
-      else if (up >= 0 && col == up)
-        Jac = dden_up * ukvr * TP + den * dukvr_up * TP + den * ukvr * Tr[j] + 2 * den * dden_up * ukvr * G +
-              (den * den) * dukvr_up * G;
-      else if (dn >= 0 && col == dn)
-        Jac = dden_dn * ukvr * TP + den * dukvr_dn * TP + den * ukvr * Tr[j] + 2 * den * dden_dn * ukvr * G +
-              (den * den) * dukvr_dn * G;
-      else
-        Jac = den * ukvr * Tr[j];
-      a.D[to + j] = -Jac;  // the up cell's residual gets -Jac, the down cell's +Jac (tdympfao_ts.c:439-444)
-    }
-  }
-}
-
-// Jacobian row of each cell (CSR in the vertex-adjacency pattern, or the
-// solver's ELL): the derivatives of its faces' flux rows in a fixed (face,
-// sub-face) row order, then the accumulation diagonal.  kGenJLanes lanes own
-// one row, summed in LDS (up to kGenJSlots entries), every slot written once.
-// Lane l first reads row l's metadata (face lf = l/4, sub-face l%4); then a
-// lane per column loads the rows' derivatives eight rows at a time and adds
-// them row by row.  A flux row adds to each slot at most once (its columns
-// are distinct cells), so every slot is summed in row order.
-constexpr int kGenJBlock = 256;
-constexpr int kGenJLanes = 32;  // lanes per cell: columns of a flux row (a row of more loops)
-constexpr int kGenJSlots = 64;
-struct GenGatherArgs {
-  int nc, form, ell_w;
-  int jbs;               // ELL: block size of the block-contiguous layout (see jac_row_addr)
-  const int32_t *perm;   // ELL: position of row c (nullptr: CSR at jrp[c])
-  double shift, dtime;
-  const int32_t *cell_faces, *face_cells, *rtoff, *rinfo, *roc, *ccell, *jrp, *jcols, *jdiag;
-  const uint8_t *face_flags, *gslot;
-  const double *D, *dM, *d2M, *Udot, *vol;
-  double *J;
-  const double *dyn;  // device dtime / shift (see StateParams), or nullptr
-  const int *stop;
-};
-
-// The same flux rows, one wavefront per vertex block: first a lane per block
-// row computes the row's flux and its scalars (T.P, mean density, upwind
-// mobility and their derivatives) into LDS, then the lanes sweep the block's
-// cell entries in memory order and write the derivatives D, so T and D are
-// read and written in contiguous runs.  Rows without a block (a triangle's
-// fourth sub-face, no-flow faces) keep the zero flux written at setup.  Same
-// arithmetic as k_rows_general, entry by entry.
-constexpr int kBlkRows = 64;  // most flux rows of one vertex block (checked at setup)
-struct GenBlkArgs {
-  int nc;
-  double pref;
-  const int32_t *vblk;  // per vertex: T offset, rows, cells, Dirichlet columns, cell offset, Dirichlet offset, row offset
+  const GenGroup *grp;
+  const GenRow *brd;
   const int32_t *brow;  // flux row of each block row, blocks in vertex order
   const int32_t *face_cells;
   const uint8_t *face_flags;
   const int32_t *ccell, *vdcol;
   const double *T, *G, *U, *Pbnd;
   const FlowState *st;
-  double *flux, *D;
+  double *flux, *lam;
+  double2 *side;
   const int *stop;
 };
 
 template <bool WITH_R, bool WITH_J>
-__global__ void __launch_bounds__(64) k_rows_general_blk(GenBlkArgs a) {
-  if (a.stop && *a.stop) return;  // uniform over the workgroup
-  __shared__ double s_tp[kBlkRows], s_den[kBlkRows], s_ukvr[kBlkRows], s_G[kBlkRows];
-  __shared__ double s_ddu[kBlkRows], s_ddd[kBlkRows], s_dku[kBlkRows], s_dkd[kBlkRows];
-  __shared__ int s_up[kBlkRows], s_dn[kBlkRows], s_flag[kBlkRows];  // flag: 1 no D, 2 zero D
-  const int v = blockIdx.x, t = threadIdx.x;
-  const int32_t *d = a.vblk + (int64_t)v * 7;
-  const int ot = d[0], nrow = d[1], ncell = d[2], ndir = d[3];
-  const int32_t *cols = a.ccell + d[4];
-  const int32_t *dcols = a.vdcol + d[5];
-  const int nB = ncell + ndir;
-  if (t < nrow) {
-    const int64_t r = a.brow[d[6] + t];
-    const int f = (int)(r >> 2);
-    const uint8_t fl = a.face_flags[f];
-    int flag = 0;
-    if (fl & kFaceNoFlow) {
-      if (WITH_R) a.flux[r] = 0.0;
-      flag = 1;
-    } else {
-      const double *Tr = a.T + ot + (int64_t)t * nB;
-      double TP = 0.0;
-#pragma unroll 4
-      for (int j = 0; j < ncell; j++) TP += Tr[j] * a.U[cols[j]];
-      for (int j = 0; j < ndir; j++) TP += Tr[ncell + j] * a.Pbnd[dcols[j]];
-      const int up = a.face_cells[2 * f], dn = a.face_cells[2 * f + 1];
-      double den = 0.0;
-      const FlowState su = a.st[flow_index(a.nc, up)], sd = a.st[flow_index(a.nc, dn)];
-      den += su.rho;
-      den += sd.rho;
-      den *= 0.5;
-      const double G = a.G[r];
-      const bool upwind_up = (TP + den * G < 0.0);
-      const int uw = upwind_up ? up : dn;
-      const double ukvr = upwind_up ? su.ukvr : sd.ukvr;
-      const bool zero = uw < 0 && (fl & kFaceSeepage) && a.Pbnd[-uw - 1] <= a.pref;
-      if (WITH_R) {
-        double fluxm = 0.0;
-        if (!zero) {
-          fluxm = den * ukvr * (-TP);
-          fluxm += -(den * den) * ukvr * G;
-        }
-        a.flux[r] = fluxm;
-      }
-      if (WITH_J) {
-        const double dukvr_up = upwind_up ? su.dukvr : 0.0, dukvr_dn = upwind_up ? 0.0 : sd.dukvr;
-        s_tp[t] = TP; s_den[t] = den; s_ukvr[t] = ukvr; s_G[t] = G;
-        s_ddu[t] = 0.5 * su.drho;
-        s_ddd[t] = 0.5 * sd.drho;
-        s_dku[t] = dukvr_up; s_dkd[t] = dukvr_dn;
-        s_up[t] = up; s_dn[t] = dn;
-      }
-      flag = zero ? 2 : 0;
+__global__ void __launch_bounds__(kGrpRows) k_rows_general(GenRowArgs a) {
+  extern __shared__ double gen_lds[];  // the columns' pressures, then the run's T entries
+  double *Ps = gen_lds, *Ts = gen_lds + kGrpCols;
+  if (a.stop && *a.stop) return;
+  const GenGroup g = a.grp[blockIdx.x];
+  const int t = threadIdx.x;
+  // the row's own data beside the staging
+  const bool live = t < g.nrow;
+  const int r = live ? a.brow[g.row + t] : 0, f = r >> 2;
+  const GenRow d = live ? a.brd[g.row + t] : GenRow{};
+  {
+    double v[kGrpT / kGrpRows];
+    int col[kGrpCols / kGrpRows];
+#pragma unroll
+    for (int i = 0; i < kGrpCols / kGrpRows; i++) {
+      const int e = t + i * kGrpRows;
+      col[i] = e < g.ncell ? a.ccell[g.cell + e] : e < g.ncell + g.ndir ? a.vdcol[g.dir + e - g.ncell] : 0;
     }
-    if (WITH_J) s_flag[t] = flag;
+#pragma unroll
+    for (int i = 0; i < kGrpT / kGrpRows; i++) {
+      const int e = t + i * kGrpRows;
+      v[i] = e < g.nt ? a.T[(int64_t)g.t + e] : 0.0;
+    }
+#pragma unroll
+    for (int i = 0; i < kGrpCols / kGrpRows; i++) {
+      const int e = t + i * kGrpRows;
+      if (e < g.ncell + g.ndir) Ps[e] = e < g.ncell ? a.U[col[i]] : a.Pbnd[col[i]];
+    }
+#pragma unroll
+    for (int i = 0; i < kGrpT / kGrpRows; i++) {
+      const int e = t + i * kGrpRows;
+      if (e < g.nt) Ts[e] = v[i];
+    }
+    for (int e = t + kGrpT; e < g.nt; e += kGrpRows) Ts[e] = a.T[(int64_t)g.t + e];
   }
-  if (!WITH_J) return;
+  const int2 ud = *reinterpret_cast<const int2 *>(a.face_cells + 2 * f);
+  const uint8_t fl = a.face_flags[f];
+  const double G = a.G[r];
+  const int up = ud.x, dn = ud.y;
+  const FlowState su = a.st[flow_index(a.nc, up)], sd = a.st[flow_index(a.nc, dn)];
   __syncthreads();
-  const int ne = nrow * ncell;
-  for (int e = t; e < ne; e += 64) {
-    const int i = e / ncell, j = e - i * ncell;
-    const int flag = s_flag[i];
-    if (flag & 1) continue;
-    const int64_t q = (int64_t)ot + (int64_t)i * nB + j;
-    const int col = cols[j];
-    const int up = s_up[i], dn = s_dn[i];
-    const double TP = s_tp[i], den = s_den[i], ukvr = s_ukvr[i], G = s_G[i];
-    double Jac;
-    if (flag & 2) Jac = 0.0;
-    else if (up >= 0 && col == up)
-      Jac = s_ddu[i] * ukvr * TP + den * s_dku[i] * TP + den * ukvr * a.T[q] + 2 * den * s_ddu[i] * ukvr * G +
-            (den * den) * s_dku[i] * G;
-    else if (dn >= 0 && col == dn)
-      Jac = s_ddd[i] * ukvr * TP + den * s_dkd[i] * TP + den * ukvr * a.T[q] + 2 * den * s_ddd[i] * ukvr * G +
-            (den * den) * s_dkd[i] * G;
-    else
-      Jac = den * ukvr * a.T[q];
-    a.D[q] = -Jac;  // the up cell's residual gets -Jac, the down cell's +Jac (tdympfao_ts.c:439-444)
+  if (!live) return;
+  double TP = 0.0;
+#pragma unroll 4
+  for (int j = 0; j < d.ncell; j++) TP += Ts[d.t + j] * Ps[d.cell + j];
+  for (int j = 0; j < d.ndir; j++) TP += Ts[d.t + d.ncell + j] * Ps[g.ncell + d.dir + j];
+  const double den = row_den(su.rho, sd.rho);
+  const bool upwind_up = (TP + den * G < 0.0);
+  const int uw = upwind_up ? up : dn;
+  const double ukvr = upwind_up ? su.ukvr : sd.ukvr;
+  const bool zero = uw < 0 && (fl & kFaceSeepage) && a.Pbnd[-uw - 1] <= a.pref;
+  if (WITH_R) a.flux[r] = row_flux(TP, den, G, ukvr, zero);
+  if (WITH_J) {
+    a.lam[r] = zero ? 0.0 : den * ukvr;
+    a.side[r] = zero ? double2{0.0, 0.0}
+                     : double2{side_extra(TP, den, G, ukvr, 0.5 * su.drho, upwind_up ? su.dukvr : 0.0),
+                               side_extra(TP, den, G, ukvr, 0.5 * sd.drho, upwind_up ? 0.0 : sd.dukvr)};
   }
+}
+
+// Jacobian row of each cell (CSR in the vertex-adjacency pattern, or the
+// solver's ELL): its faces' flux rows in a fixed (face, sub-face) order, then
+// the sides' terms and the accumulation diagonal.  kGenJLanes lanes own one
+// row, summed in LDS (up to kGenJSlots entries), every slot written once.
+// Lanes l and l + 16 of the 24 rows first read the rows' metadata and factors
+// (face lf = i/4, sub-face i%4); then a lane per column loads T and its slot
+// eight rows at a time and adds factor * T row by row with LDS adds, which
+// need no answer (200k prisms 218 -> 171 us against read, add and write back,
+// 32 lanes per cell): a wavefront's LDS operations run in program order and a
+// flux row reaches each slot at most once (its columns are distinct cells),
+// so every slot is summed in row order.  The rows' terms in the cell's own
+// column and, per face, in the other cell's are reduced over the lanes first.
+constexpr int kGenJBlock = 256;
+constexpr int kGenJLanes = 16;  // lanes per cell: columns of a flux row (a row of more loops)
+constexpr int kGenJSlots = 64;
+struct GenGatherArgs {
+  int nc, form, ell_w;
+  int jbs;               // ELL: block size of the block-contiguous layout (see jac_row_addr)
+  const int32_t *perm;   // ELL: position of row c (nullptr: CSR at jrp[c])
+  double shift, dtime;
+  const int32_t *cell_faces, *face_cells, *rtoff, *rinfo, *jrp, *jdiag;
+  const uint8_t *face_flags, *gslot, *nslot;
+  const double *T, *lam, *dM, *d2M, *Udot, *vol;
+  const double2 *side;
+  double *J;
+  const double *dyn;  // device dtime / shift (see StateParams), or nullptr
+  const int *stop;
+};
+
+// Slot of each face's other cell in the cell's Jacobian row (0xff for a
+// boundary or absent face), built once at setup: one thread per cell and face.
+__global__ void __launch_bounds__(256) k_gen_neighbour_slots(int nc, const int32_t *__restrict__ cell_faces,
+                                                             const int32_t *__restrict__ face_cells,
+                                                             const int32_t *__restrict__ jrp,
+                                                             const int32_t *__restrict__ jcols,
+                                                             uint8_t *__restrict__ nslot) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= (int64_t)nc * 6) return;
+  const int c = (int)(i / 6), f = cell_faces[i];
+  uint8_t s = 0xff;
+  if (f >= 0) {
+    const int o = face_cells[2 * f] == c ? face_cells[2 * f + 1] : face_cells[2 * f];
+    if (o >= 0) {
+      const int r0 = jrp[c];
+      int lo = r0, hi = jrp[c + 1] - 1;
+      while (lo < hi) {
+        const int mid = (lo + hi) >> 1;
+        if (jcols[mid] < o) lo = mid + 1; else hi = mid;
+      }
+      s = (uint8_t)(lo - r0);
+    }
+  }
+  nslot[i] = s;
 }
 
 // Slot table of the general Jacobian gather, built once at setup: entry
@@ -507,58 +463,83 @@ __global__ void __launch_bounds__(kGenJBlock) k_gather_general_J(GenGatherArgs a
   constexpr int CPB = kGenJBlock / kGenJLanes;  // cells per workgroup
   constexpr int NR = 24;                        // flux rows of a cell: 6 faces x 4 sub-faces
   constexpr int RB = 8;                         // rows whose loads are in flight together
-  static_assert(kGenJLanes >= NR && 64 % kGenJLanes == 0, "a cell's lanes hold its rows and share a wavefront");
-  __shared__ double acc[CPB][kGenJSlots];
+  static_assert(2 * kGenJLanes >= NR && 64 % kGenJLanes == 0, "a cell's lanes hold its rows and share a wavefront");
+  __shared__ double acc[CPB][kGenJSlots + 1];
   if (a.stop && *a.stop) return;
   const int g = threadIdx.x / kGenJLanes, l = threadIdx.x % kGenJLanes;
   const int base = (threadIdx.x & 63) - l;  // the cell's first lane within the wavefront
   const int c = blockIdx.x * CPB + g;
-  if (c >= a.nc) return;  // uniform over the cell's lanes (the wavefront's other cell is independent)
+  if (c >= a.nc) return;  // uniform over the cell's lanes (the wavefront's other cells are independent)
   const int r0 = a.jrp[c], len = a.jrp[c + 1] - r0;
   for (int k = l; k < len; k += kGenJLanes) acc[g][k] = 0.0;
-  // row l's metadata: its derivatives at D[to ..], its slots, the sign by the cell's side
-  int to = -1, nce = 0, side = 0;
-  bool up = false;
-  if (l < NR) {
-    const int f = a.cell_faces[c * 6 + (l >> 2)];
+  // rows l and l + 16: T at T[to ..], the columns' slots, the signed factor,
+  // and the sums of the sides' terms (this cell's, the other cell's)
+  int to[2], ns[2];  // ns: columns | side << 8
+  double fac[2], self = 0.0, other[2];
+#pragma unroll
+  for (int h = 0; h < 2; h++) {
+    const int i = l + h * kGenJLanes;
+    to[h] = -1; ns[h] = 0; fac[h] = 0.0; other[h] = 0.0;
+    const int f = i < NR ? a.cell_faces[c * 6 + (i >> 2)] : -1;
     if (f >= 0 && !(a.face_flags[f] & kFaceNoFlow)) {
-      const int64_t r = (int64_t)f * 4 + (l & 3);
-      to = a.rtoff[r];
-      nce = to >= 0 ? (a.rinfo[r] & 0xff) : 0;
-      up = a.face_cells[2 * f] == c;
-      side = up ? 0 : 1;
+      const int64_t r = (int64_t)f * 4 + (i & 3);
+      to[h] = a.rtoff[r];
+      if (to[h] >= 0) {
+        const bool up = a.face_cells[2 * f] == c;
+        const double s = up ? -1.0 : 1.0;
+        const double2 x = a.side[r];
+        ns[h] = (a.rinfo[r] & 0xff) | (up ? 0 : 0x100);
+        fac[h] = s * a.lam[r];
+        self += s * (up ? x.x : x.y);
+        other[h] = s * (up ? x.y : x.x);
+      }
     }
   }
+#pragma unroll
+  for (int off = 1; off < kGenJLanes; off <<= 1) self += __shfl_xor(self, off, 64);
+#pragma unroll
+  for (int h = 0; h < 2; h++) {
+    other[h] += __shfl_xor(other[h], 1, 64);
+    other[h] += __shfl_xor(other[h], 2, 64);
+  }
+#pragma unroll
   for (int i0 = 0; i0 < NR; i0 += RB) {
-    double dv[RB];
+    double tv[RB], fv[RB];
     int sv[RB];
 #pragma unroll
     for (int k = 0; k < RB; k++) {
-      const int ti = __shfl(to, base + i0 + k, 64), ni = __shfl(nce, base + i0 + k, 64);
-      const int si = __shfl(side, base + i0 + k, 64);
-      const bool on = ti >= 0 && l < ni;
-      dv[k] = on ? a.D[ti + l] : 0.0;
-      sv[k] = on ? a.gslot[2 * ((int64_t)ti + l) + si] : -1;
+      const int h = (i0 + k) / kGenJLanes, src = base + (i0 + k) % kGenJLanes;
+      const int ti = __shfl(to[h], src, 64), ni = __shfl(ns[h], src, 64);
+      fv[k] = __shfl(fac[h], src, 64);
+      const bool on = ti >= 0 && l < (ni & 0xff);
+      tv[k] = on ? a.T[ti + l] : 0.0;
+      sv[k] = on ? a.gslot[2 * ((int64_t)ti + l) + (ni >> 8)] : -1;
     }
 #pragma unroll
     for (int k = 0; k < RB; k++) {
-      const int ti = __shfl(to, base + i0 + k, 64), ni = __shfl(nce, base + i0 + k, 64);
-      const int si = __shfl(side, base + i0 + k, 64);
-      const bool ui = __shfl((int)up, base + i0 + k, 64) != 0;
-      if (sv[k] >= 0) acc[g][sv[k]] += ui ? dv[k] : -dv[k];
+      if (sv[k] >= 0) atomicAdd(&acc[g][sv[k]], fv[k] * tv[k]);
       // columns past the lanes (regions of more than kGenJLanes cells): the rest of the same row
-      for (int j = l + kGenJLanes; ti >= 0 && j < ni; j += kGenJLanes) {
-        const double d = a.D[ti + j];
-        acc[g][a.gslot[2 * ((int64_t)ti + j) + si]] += ui ? d : -d;
-      }
+      const int h = (i0 + k) / kGenJLanes, src = base + (i0 + k) % kGenJLanes;
+      const int ti = __shfl(to[h], src, 64), ni = __shfl(ns[h], src, 64);
+      for (int j = l + kGenJLanes; ti >= 0 && j < (ni & 0xff); j += kGenJLanes)
+        atomicAdd(&acc[g][a.gslot[2 * ((int64_t)ti + j) + (ni >> 8)]], fv[k] * a.T[ti + j]);
+    }
+  }
+#pragma unroll
+  for (int h = 0; h < 2; h++) {
+    const int lf = (l + h * kGenJLanes) >> 2;
+    if ((l & 3) == 0 && lf < 6) {  // a face each: its other cell's slot is its own
+      const int s = a.nslot[(int64_t)c * 6 + lf];
+      if (s != 0xff) atomicAdd(&acc[g][s], other[h]);
     }
   }
   if (l == 0) {
     const double shift = a.dyn ? a.dyn[1] : a.shift, dtime = a.dyn ? a.dyn[0] : a.dtime;
     const double dvc = (a.form == 0) ? (shift * a.dM[c] + a.d2M[c] * a.Udot[c]) * a.vol[c]
                                      : a.dM[c] * a.vol[c] * (1.0 / dtime);
-    acc[g][a.jdiag[c]] += dvc;
+    atomicAdd(&acc[g][a.jdiag[c]], self + dvc);
   }
+  __builtin_amdgcn_wave_barrier();
   int64_t st = 1;
   double *row = a.J + r0;
   if (a.perm) {

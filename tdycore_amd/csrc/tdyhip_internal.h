@@ -145,6 +145,11 @@ struct KernelTimers {
 
 }  // namespace tdyhip
 
+namespace tdyhip {
+struct GenGroup;
+struct GenRow;
+}  // namespace tdyhip
+
 struct tdyhip_fuser;
 
 struct tdyhip_ctx {
@@ -217,12 +222,16 @@ struct tdyhip_ctx {
   // general (prism) meshes: transmissibility setup only, T as per-vertex blocks
   bool general = false;
   double *d_Tgen = nullptr;        // sum over vertices of rows x columns, row-major blocks
-  double *d_Dgen = nullptr;        // flux-row derivatives, same blocks (cell columns)
+  double *d_rlam = nullptr;        // 4nf: rho_bar lambda of each flux row (the Jacobian's)
+  double2 *d_rside = nullptr;      // 4nf: what each side adds in its own column
   int32_t *d_rtoff = nullptr, *d_rinfo = nullptr, *d_roc = nullptr, *d_rdc = nullptr;  // 4nf each
   int32_t *d_ccell = nullptr, *d_vdcol = nullptr, *d_jdiag = nullptr;
   uint8_t *d_gslot = nullptr;      // 2 per block entry: Jacobian slot in the up / down cell's row
-  int32_t *d_vblk = nullptr;       // nv*7 vertex blocks for the row kernel (nullptr: row per thread)
-  int32_t *d_brow = nullptr;       // flux row of each block row
+  uint8_t *d_nslot = nullptr;      // nc*6: slot of each face's other cell in the cell's row
+  int ngrp = 0, grp_nt = 0;        // runs of vertices of the flux-row kernel, the most T entries of one
+  tdyhip::GenGroup *d_grp = nullptr;
+  tdyhip::GenRow *d_brd = nullptr; // flux rows with a vertex block, in block order, and
+  int32_t *d_brow = nullptr;       // their flux rows
   tdyhip::HostGeneral *hgen = nullptr;
   double setup_ms[3] = {0, 0, 0};  // setup device times: G matrices, local systems, gravity term
   double ls_flops = 0.0, ls_bytes = 0.0;  // hexahedral local systems: algorithmic FP64 flops and bytes
