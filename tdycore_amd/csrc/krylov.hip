@@ -885,14 +885,20 @@ __global__ void k_reduce_partials(int nv, int nchunk, const TV *__restrict__ par
 }
 
 // w -= sum_j h[j] V_j ; partial[chunk] = ||w||^2 over the chunk (two
-// adjacent rows per thread, as k_mdot)
-template <class TV>
+// adjacent rows per thread, as k_mdot).  DOTS: h itself is still the
+// multi-dot's npart partials per vector; every workgroup sums them, eight
+// lanes a vector in a fixed order, and workgroup 0 stores them for the
+// Arnoldi update, so no launch of its own stands between the two kernels.
+constexpr int kMaxpyVecs = 200;  // basis vectors at most (the restart length)
+template <class TV, bool DOTS>
 __global__ void __launch_bounds__(kRedBlock) k_maxpy_norm(int64_t n, int nv, const TV *__restrict__ V, int64_t ldv,
-                                                          const double *__restrict__ h, TV *__restrict__ w,
+                                                          double *__restrict__ h, TV *__restrict__ w,
                                                           TV *__restrict__ partial,
                                                           const int *__restrict__ stop = nullptr,
-                                                          Prolong pro = Prolong{}) {
+                                                          Prolong pro = Prolong{}, const TV *__restrict__ dots = nullptr,
+                                                          int npart = 0) {
   __shared__ TV sh[kRedBlock / 64];
+  __shared__ double hs[DOTS ? kMaxpyVecs : 1];
   if (stop && *stop) return;
   const int64_t r0 = (int64_t)blockIdx.x * Red<TV>::chunk + 2 * threadIdx.x;
   const bool vec = (ldv & 1) == 0;
@@ -902,10 +908,32 @@ __global__ void __launch_bounds__(kRedBlock) k_maxpy_norm(int64_t n, int nv, con
     if (r0 < n) x0 += (TV)pro.z1[pro.pos[r0] >> pro.bs_log2];
     if (r0 + 1 < n) x1 += (TV)pro.z1[pro.pos[r0 + 1] >> pro.bs_log2];
   }
+  if (DOTS) {
+    const int l = threadIdx.x % 8;
+    for (int v = threadIdx.x / 8; v < nv; v += kRedBlock / 8) {
+      const TV *p = dots + (int64_t)v * npart;
+      TV s = 0;
+      for (int c = l; c < npart; c += 64) {
+        TV q[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++) q[u] = c + 8 * u < npart ? p[c + 8 * u] : (TV)0;
+#pragma unroll
+        for (int u = 0; u < 8; u++) s += q[u];
+      }
+      s += __shfl_xor(s, 1, 64);
+      s += __shfl_xor(s, 2, 64);
+      s += __shfl_xor(s, 4, 64);
+      if (l == 0) {
+        hs[v] = (double)s;
+        if (blockIdx.x == 0) h[v] = (double)s;
+      }
+    }
+    __syncthreads();
+  }
   for (int j = 0; j < nv; j++) {
     TV v0, v1;
     load2(V + (int64_t)j * ldv, r0, n, vec, v0, v1);
-    const TV hj = (TV)h[j];
+    const TV hj = (TV)(DOTS ? hs[j] : h[j]);
     x0 -= hj * v0;
     x1 -= hj * v1;
   }

@@ -987,6 +987,12 @@ const double bfold = (double)C.ng * C.ng * C.gsz * 8;
 // 1M rows, 2048 partials per workgroup cost as much as they save.)
 constexpr int kFuseNormChunks = 512;
 
+// With up to this many partials per dot, the update kernel sums them itself
+// (every workgroup, up to restart x 256 values from L2), which takes less than
+// the launch it saves: 4k cells 4.05 -> 3.34 ms a step, 46k one-level 20.7 -> 20.1,
+// 100k prisms 29.3 -> 27.5; at 246 partials (63k cells) the two are even.
+constexpr int kFuseDots = 256;
+
 template <class TV>
 static void gmres_cycle(tdyhip_ctx *ctx, const tdyhip_solver_opts &o, const double *bvec, double *yvec,
                         hipStream_t st) {
@@ -1012,11 +1018,12 @@ static void gmres_cycle(tdyhip_ctx *ctx, const tdyhip_solver_opts &o, const doub
   }
   const int pst = nch + cd.parts;  // partials per vector: the coarse parts', then the row chunks'
   const unsigned gmd = (unsigned)pst;
+  TV *npart = k.part + (int64_t)m * pst;  // the norm's partials, apart from the dots' that the same launch may read
   // The unnormalised Arnoldi vector alternates between w and z: step j reads
   // it from one and leaves the next in the other.
   for (int j = 0; j < m; j++) {
     TV *u = (j % 2 == 0) ? k.w : k.z, *ov = (j % 2 == 0) ? k.z : k.w;
-    const NormArgs na{k.part, nch, j - 1, m, ws.h, k.dH, k.dcs, k.dsn, k.dg};
+    const NormArgs na{npart, nch, j - 1, m, ws.h, k.dH, k.dcs, k.dsn, k.dg};
     const bool fuse_norm = nch <= kFuseNormChunks;
     // timer tags: the launches of step j work only if the cycle reached
     // column j; a fused matvec also finishes column j-1, so it counts with it
@@ -1039,10 +1046,14 @@ static void gmres_cycle(tdyhip_ctx *ctx, const tdyhip_solver_opts &o, const doub
     else if (j < 16 || sizeof(TV) == 4) TDY_MDOT(16);
     else TDY_MDOT(32);
 #undef TDY_MDOT
-    k_reduce_partials<TV><<<j + 1, kRedBlock, 0, st>>>(j + 1, pst, k.part, ws.h, stop);
     const double bmx = (double)(j + 3) * N * sizeof(TV) + (pro.z1 ? (double)N * 4 : 0.0);
-    KT(ctx, st, "k_maxpy_norm", bmx, k_maxpy_norm<TV><<<nch, kRedBlock, 0, st>>>(N, j + 1, k.V, N, ws.h, ov, k.part, stop, pro));
-    if (!fuse_norm || j == m - 1) k_norm_arnoldi<TV><<<1, kRedBlock, 0, st>>>(nch, k.part, gd, j, m, ws.h, k.dH, k.dcs, k.dsn, k.dg);
+    if (pst <= kFuseDots) {
+      KT(ctx, st, "k_maxpy_norm", bmx, k_maxpy_norm<TV, true><<<nch, kRedBlock, 0, st>>>(N, j + 1, k.V, N, ws.h, ov, npart, stop, pro, k.part, pst));
+    } else {
+      k_reduce_partials<TV><<<j + 1, kRedBlock, 0, st>>>(j + 1, pst, k.part, ws.h, stop);
+      KT(ctx, st, "k_maxpy_norm", bmx, k_maxpy_norm<TV, false><<<nch, kRedBlock, 0, st>>>(N, j + 1, k.V, N, ws.h, ov, npart, stop, pro));
+    }
+    if (!fuse_norm || j == m - 1) k_norm_arnoldi<TV><<<1, kRedBlock, 0, st>>>(nch, npart, gd, j, m, ws.h, k.dH, k.dcs, k.dsn, k.dg);
   }
   ctx->kt.tag = -1;
   if (m <= kHessLdsMaxM)
