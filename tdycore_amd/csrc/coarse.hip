@@ -127,10 +127,12 @@ __global__ void __launch_bounds__(BS) k_coarse_cols(CoarseLayout C, int W, int b
   const double own = acc[C.R.ownq[b]][t];
   C.cown[(int64_t)b * BS + t] = own;
   __syncthreads();
-  const double s = coarse_block_sums<BS>(C.R, b, t, own, [&](int e) {
-    const unsigned w = C.R.cent[e];
+  const int l0 = C.R.eptr[b], q = t < kCQ ? t : 0;
+  const double s = coarse_block_sums<BS>(C.R.eptr[b + 1] - l0, C.R.tq[b * (kCQ + 1) + q], C.R.tq[b * (kCQ + 1) + q + 1],
+                                         t == C.R.ownq[b], t, own, [&](int e) {
+    const unsigned w = C.R.cent[l0 + e];
     const double v = w == kCoarsePad ? 0.0 : acc[w >> 9][w & 511];
-    C.cval[e] = v;
+    C.cval[l0 + e] = v;
     return v;
   });
   if (t < kCQ) {

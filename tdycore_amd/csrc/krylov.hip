@@ -304,19 +304,19 @@ struct CoarseRestrict {
   double *r2c = nullptr;           // received contributions by group
 };
 
-// Per-neighbour sums of block b: thread q < kCQ returns the sum of neighbour q
+// Per-neighbour sums of a block: thread q < kCQ returns the sum of neighbour q
 // (the own block's: of `own` over the workgroup; another's: of value(e) over
-// its list).  Every thread calls it; one barrier inside.
+// its list of ne entries, teams i0 .. i1-1).  Every thread calls it; one
+// barrier inside.
 template <int BS, class F>
-__device__ inline double coarse_block_sums(const CoarseRestrict &R, int b, int t, double own, F &&value) {
+__device__ inline double coarse_block_sums(int ne, int i0, int i1, bool ownq, int t, double own, F &&value) {
   constexpr int kTeams = BS * 27 / 8 + kCQ;  // every row in 27 lists, each list's last team short
   __shared__ double tm[kTeams];
   __shared__ double ow[BS / 64];
-  const int e0 = R.eptr[b], ne = R.eptr[b + 1] - e0;
   for (int off = 32; off > 0; off >>= 1) own += __shfl_down(own, off, 64);
   if ((t & 63) == 0) ow[t >> 6] = own;
   for (int e = t; e < ne; e += BS) {  // ne is a multiple of 8: a team's lanes stay together
-    double v = value(e0 + e);
+    double v = value(e);
     v += __shfl_xor(v, 1, 64);
     v += __shfl_xor(v, 2, 64);
     v += __shfl_xor(v, 4, 64);
@@ -325,9 +325,8 @@ __device__ inline double coarse_block_sums(const CoarseRestrict &R, int b, int t
   __syncthreads();
   double s = 0.0;
   if (t < kCQ) {
-    const int i0 = R.tq[b * (kCQ + 1) + t], i1 = R.tq[b * (kCQ + 1) + t + 1];
     for (int i = i0; i < i1; i++) s += tm[i];
-    if (t == R.ownq[b]) {
+    if (ownq) {
 #pragma unroll
       for (int w = 0; w < BS / 64; w++) s += ow[w];
     }
@@ -335,30 +334,69 @@ __device__ inline double coarse_block_sums(const CoarseRestrict &R, int b, int t
   return s;
 }
 
+// What a thread of block b reads for its part of the coarse right-hand side:
+// its row's own column sum, its first list entries, and (thread q < kCQ)
+// neighbour q's teams and destinations.
+template <int BS>
+struct CoarseRegs {
+  static constexpr int PRE = BS == 64 ? 4 : 2;  // list entries held (a whole brick's has up to 5 or 2 per thread)
+  int e0, ne;
+  double own, val[PRE];
+  unsigned ent[PRE];
+  int i0 = 0, i1 = 0, dst = -1, dst2 = -1, grp = 255;
+  bool ownq = false;
+};
+template <int BS>
+__device__ inline void coarse_load(const CoarseRestrict &R, int b, int t, CoarseRegs<BS> &c) {
+  c.e0 = R.eptr[b];
+  c.ne = R.eptr[b + 1] - c.e0;
+  c.own = R.cown[(int64_t)b * BS + t];
+#pragma unroll
+  for (int k = 0; k < CoarseRegs<BS>::PRE; k++) {
+    const bool in = t + k * BS < c.ne;
+    c.val[k] = in ? R.cval[c.e0 + t + k * BS] : 0.0;
+    c.ent[k] = in ? R.cent[c.e0 + t + k * BS] : kCoarsePad;
+  }
+  if (t < kCQ) {
+    c.i0 = R.tq[b * (kCQ + 1) + t];
+    c.i1 = R.tq[b * (kCQ + 1) + t + 1];
+    c.ownq = t == R.ownq[b];
+    c.dst = R.wdst[b * kCQ + t];
+    c.dst2 = R.w2dst[b * kCQ + t];
+    c.grp = R.gsl[b * kCQ + t];
+  }
+}
+
 // After the sweeps (x: w_bj of the block, rr: the block sum of its right-hand
 // side): the block's contributions to R (r - A w_bj), per neighbour block and
 // summed per neighbour group.  Every thread calls it.
 template <class TV, int BS>
-__device__ inline void coarse_scatter(const CoarseRestrict &R, const TV *x, const double &rr, int b, int t) {
+__device__ inline void coarse_scatter(const CoarseRestrict &R, const CoarseRegs<BS> &c, const TV *x, const double &rr,
+                                      int b, int t) {
   __shared__ double qv[kCQ];
   __shared__ uint8_t qg[kCQ];
-  const double s = coarse_block_sums<BS>(R, b, t, R.cown[(int64_t)b * BS + t] * (double)x[t],
-                                         [&](int e) {
-                                           const unsigned w = R.cent[e];
-                                           return R.cval[e] * (double)x[w == kCoarsePad ? BS : w & 511];  // x[BS] is 0
-                                         });
+  constexpr int PRE = CoarseRegs<BS>::PRE;
+  const double s = coarse_block_sums<BS>(c.ne, c.i0, c.i1, c.ownq, t, c.own * (double)x[t], [&](int e) {
+    double v = 0.0;
+    unsigned w = kCoarsePad;
+    bool held = false;
+#pragma unroll
+    for (int k = 0; k < PRE; k++)
+      if (e == t + k * BS) { v = c.val[k]; w = c.ent[k]; held = true; }
+    if (!held) { v = R.cval[c.e0 + e]; w = R.cent[c.e0 + e]; }
+    return v * (double)x[w == kCoarsePad ? BS : w & 511];  // x[BS] is 0
+  });
   if (t < kCQ) {
-    const double v = (t == R.ownq[b] ? rr : 0.0) - s;
-    const int d = R.wdst[b * kCQ + t], d2 = R.w2dst[b * kCQ + t];
-    if (d >= 0) R.rcs[d] = v;
+    const double v = (c.ownq ? rr : 0.0) - s;
+    if (c.dst >= 0) R.rcs[c.dst] = v;
     qv[t] = v;
-    qg[t] = R.gsl[b * kCQ + t];
+    qg[t] = (uint8_t)c.grp;
     __builtin_amdgcn_wave_barrier();  // one wavefront: its LDS operations run in program order
-    if (d2 >= 0) {
+    if (c.dst2 >= 0) {
       double g = 0.0;
 #pragma unroll
       for (int q = 0; q < kCQ; q++) g += qg[q] == t ? qv[q] : 0.0;
-      R.r2c[d2] = g;
+      R.r2c[c.dst2] = g;
     }
   }
 }
@@ -405,46 +443,67 @@ __device__ inline void restrict_block2(const TV *x, double &rr, TV v, double *rv
 // x[BS] == 0 the target of padded slots) in LDS.  Every thread of the block
 // must call this; x[t] holds the right-hand side on entry and the solution on
 // return.
+//
+// Between two barriers of a level stand LDS reads, the row's products and one
+// LDS write: on grids too small to hide it, that chain is the kernel's time,
+// so the products go into four sums (levels of thirteen dependent
+// multiply-adds took 68 steps a brick: 1M cells 106.7 -> 101.4 us).
+template <class TV>
+struct SweepRegs {  // a thread's row: factor entries and their local columns
+  TV vl[kLU], vu[kLU], dinv;
+  uint16_t cl[kLU], cu[kLU];
+  int levL, levU, nL, nU;
+};
 template <class TV, int BS>
-__device__ inline void bj_sweeps(const BJLayout &L, const TV *__restrict__ fac, TV *x, int b, int t) {
+__device__ inline void bj_sweeps_load(const BJLayout &L, const TV *__restrict__ fac, int b, int t, SweepRegs<TV> &r) {
   const int pb = L.d_pat ? L.d_pat[b] : b;  // index tables of the block's pattern
   const int64_t base = (int64_t)pb * BS;
   const int64_t sbase = (int64_t)b * kW * BS;
   const int64_t cbase = (int64_t)pb * kLU * BS;
-  TV vl[kLU], vu[kLU];
-  uint16_t cl[kLU], cu[kLU];
   const int nlu = L.d_nlu ? L.d_nlu[pb] : kLU;  // slots past it hold 0 against the zero entry x[BS]
 #pragma unroll
   for (int p = 0; p < kLU; p++) {
     const bool in = p < nlu;
-    vl[p] = in ? fac[sbase + (int64_t)p * BS + t] : (TV)0;
-    vu[p] = in ? fac[sbase + (int64_t)(kLU + p) * BS + t] : (TV)0;
-    cl[p] = in ? L.d_cL[cbase + (int64_t)p * BS + t] : (uint16_t)BS;
-    cu[p] = in ? L.d_cU[cbase + (int64_t)p * BS + t] : (uint16_t)BS;
+    r.vl[p] = in ? fac[sbase + (int64_t)p * BS + t] : (TV)0;
+    r.vu[p] = in ? fac[sbase + (int64_t)(kLU + p) * BS + t] : (TV)0;
+    r.cl[p] = in ? L.d_cL[cbase + (int64_t)p * BS + t] : (uint16_t)BS;
+    r.cu[p] = in ? L.d_cU[cbase + (int64_t)p * BS + t] : (uint16_t)BS;
   }
-  const TV dinv = fac[sbase + (int64_t)(2 * kLU) * BS + t];
-  const int levL = L.d_levL[base + t], levU = L.d_levU[base + t];
-  const int nL = L.d_nlev[2 * pb], nU = L.d_nlev[2 * pb + 1];
+  r.dinv = fac[sbase + (int64_t)(2 * kLU) * BS + t];
+  r.levL = L.d_levL[base + t];
+  r.levU = L.d_levU[base + t];
+  r.nL = L.d_nlev[2 * pb];
+  r.nU = L.d_nlev[2 * pb + 1];
+}
+// x - sum v[p] x[c[p]], the products in four sums
+template <class TV>
+__device__ inline TV sweep_row(const TV *x, TV s, const TV (&v)[kLU], const uint16_t (&c)[kLU]) {
+  TV xv[kLU];
+#pragma unroll
+  for (int p = 0; p < kLU; p++) xv[p] = x[c[p]];
+  TV q[4] = {s, (TV)0, (TV)0, (TV)0};
+#pragma unroll
+  for (int p = 0; p < kLU; p++) q[p & 3] -= v[p] * xv[p];
+  return (q[0] + q[1]) + (q[2] + q[3]);
+}
+template <class TV, int BS>
+__device__ inline void bj_sweeps_run(const SweepRegs<TV> &r, TV *x, int t) {
   __syncthreads();
   // forward: branch-free inner loop, all LDS reads of a level in flight together
-  for (int l = 0; l < nL; l++) {
-    if (levL == l) {
-      TV s = x[t];
-#pragma unroll
-      for (int p = 0; p < kLU; p++) s -= vl[p] * x[cl[p]];
-      x[t] = s;
-    }
+  for (int l = 0; l < r.nL; l++) {
+    if (r.levL == l) x[t] = sweep_row(x, x[t], r.vl, r.cl);
     __syncthreads();
   }
-  for (int l = 0; l < nU; l++) {
-    if (levU == l) {
-      TV s = x[t];
-#pragma unroll
-      for (int p = 0; p < kLU; p++) s -= vu[p] * x[cu[p]];
-      x[t] = s * dinv;
-    }
+  for (int l = 0; l < r.nU; l++) {
+    if (r.levU == l) x[t] = sweep_row(x, x[t], r.vu, r.cu) * r.dinv;
     __syncthreads();
   }
+}
+template <class TV, int BS>
+__device__ inline void bj_sweeps(const BJLayout &L, const TV *__restrict__ fac, TV *x, int b, int t) {
+  SweepRegs<TV> r;
+  bj_sweeps_load<TV, BS>(L, fac, b, t, r);
+  bj_sweeps_run<TV, BS>(r, x, t);
 }
 
 template <class TV, int BS>
@@ -461,7 +520,11 @@ __global__ void __launch_bounds__(BS) k_bj_apply(BJLayout L, const TV *__restric
   if (cr.rcs) restrict_block<TV, BS>(x, rr, t);  // cr is uniform
   bj_sweeps<TV, BS>(L, fac, x, b, t);
   if (row >= 0) y[row] = x[t];
-  if (cr.rcs) coarse_scatter<TV, BS>(cr, x, rr, b, t);
+  if (cr.rcs) {
+    CoarseRegs<BS> cg;
+    coarse_load<BS>(cr, b, t, cg);
+    coarse_scatter<TV, BS>(cr, cg, x, rr, b, t);
+  }
 }
 
 // ---------------------------------------------------------------- block-ordered SpMV
@@ -602,8 +665,14 @@ struct NormArgs {
 // triangular sweeps follow, so neither A u nor a separate scaling pass
 // touches HBM; while some workgroups sweep their levels, others stream their
 // rows of A.  u and out must be different vectors.
-template <class TV, int BS, class TI, bool NORM>
-__global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(4))) k_bj_spmv_apply(BJLayout L, int64_t NB, int W, const TI *__restrict__ ecol,
+//
+// EARLY (grids of at most two waves per SIMD, kEarlyWaves): the factor, the
+// schedule and the coarse lists are loaded before the product instead of
+// after it, in registers a larger grid needs for its occupancy: 46k rows 20.0 ->
+// 19.0 us, 63k 20.9 -> 19.7, 4k in 64-row blocks 10.3 -> 9.5 (with the four sums).
+constexpr int kEarlyWaves = 2048;
+template <class TV, int BS, class TI, bool NORM, bool EARLY>
+__global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(EARLY ? 2 : 4))) k_bj_spmv_apply(BJLayout L, int64_t NB, int W, const TI *__restrict__ ecol,
                                                       const TV *__restrict__ a, const TV *__restrict__ u,
                                                       GmresDev *__restrict__ gd, TV *__restrict__ vj,
                                                       const TV *__restrict__ fac, TV *__restrict__ out,
@@ -614,6 +683,8 @@ __global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(4))) k_
   __shared__ TV shn[BS / 64];
   __shared__ int stop_s;
   const int b = blockIdx.x, t = threadIdx.x;
+  SweepRegs<TV> sr;
+  if (EARLY) bj_sweeps_load<TV, BS>(L, fac, b, t, sr);
   TV sc;
   if (NORM) {
     // workgroup 0 of this same launch may set the stop flag: read it once
@@ -646,9 +717,13 @@ __global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(4))) k_
   if (t == 0) x[BS] = (TV)0;
   // cr is uniform; rv: the block sums of V_j, for the coarse terms of the multi-dot
   if (cr.rcs) restrict_block2<TV, BS>(x, rr, vv, rv, b, t);
-  bj_sweeps<TV, BS>(L, fac, x, b, t);
+  if (!EARLY) bj_sweeps_load<TV, BS>(L, fac, b, t, sr);
+  CoarseRegs<BS> cg;
+  if (EARLY && cr.rcs) coarse_load<BS>(cr, b, t, cg);
+  bj_sweeps_run<TV, BS>(sr, x, t);
   if (row >= 0) out[row] = x[t];
-  if (cr.rcs) coarse_scatter<TV, BS>(cr, x, rr, b, t);
+  if (!EARLY && cr.rcs) coarse_load<BS>(cr, b, t, cg);
+  if (cr.rcs) coarse_scatter<TV, BS>(cr, cg, x, rr, b, t);
 }
 
 // A restart's preconditioned residual out = M_BJ^-1 (b - J y) in one pass:
@@ -677,7 +752,11 @@ __global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(4))) k_
   if (cr.rcs) restrict_block<TV, BS>(x, rr, t);  // cr is uniform
   bj_sweeps<TV, BS>(L, fac, x, b, t);
   if (row >= 0) out[row] = x[t];
-  if (cr.rcs) coarse_scatter<TV, BS>(cr, x, rr, b, t);
+  if (cr.rcs) {
+    CoarseRegs<BS> cg;
+    coarse_load<BS>(cr, b, t, cg);
+    coarse_scatter<TV, BS>(cr, cg, x, rr, b, t);
+  }
 }
 
 // ---------------------------------------------------------------- BLAS-1 with deterministic reductions

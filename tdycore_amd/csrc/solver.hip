@@ -886,14 +886,17 @@ static void spmv_apply(tdyhip_ctx *ctx, const KBufs<TV> &k, const TV *u, TV *vj,
   GmresDev *gd = k.gd;
   const TV *Jk = k.Jk, *fac = k.fac;
   const CoarseRestrict cr = k.cr;
+  const bool early = (int64_t)ws.bj.nblocks * (ws.bj.bs / 64) <= kEarlyWaves;
+#define TDY_SPMV2(BS, TI, EC, NRM)                                                                                  \
+  do {                                                                                                             \
+    if (early) KT(ctx, st, "k_bj_spmv_apply", by, k_bj_spmv_apply<TV, BS, TI, NRM, true><<<nb, BS, 0, st>>>(ws.bj, ws.NB, W, EC, Jk, u, gd, vj, fac, out, stp, cr, nv, rv)); \
+    else KT(ctx, st, "k_bj_spmv_apply", by, k_bj_spmv_apply<TV, BS, TI, NRM, false><<<nb, BS, 0, st>>>(ws.bj, ws.NB, W, EC, Jk, u, gd, vj, fac, out, stp, cr, nv, rv)); \
+  } while (0)
 #define TDY_SPMV(TI, EC, NRM)                                                                                      \
   do {                                                                                                             \
-    if (ws.bj.bs == 64)                                                                                            \
-      KT(ctx, st, "k_bj_spmv_apply", by, k_bj_spmv_apply<TV, 64, TI, NRM><<<nb, 64, 0, st>>>(ws.bj, ws.NB, W, EC, Jk, u, gd, vj, fac, out, stp, cr, nv, rv)); \
-    else if (ws.bj.bs == 256)                                                                                      \
-      KT(ctx, st, "k_bj_spmv_apply", by, k_bj_spmv_apply<TV, 256, TI, NRM><<<nb, 256, 0, st>>>(ws.bj, ws.NB, W, EC, Jk, u, gd, vj, fac, out, stp, cr, nv, rv)); \
-    else                                                                                                           \
-      KT(ctx, st, "k_bj_spmv_apply", by, k_bj_spmv_apply<TV, 512, TI, NRM><<<nb, 512, 0, st>>>(ws.bj, ws.NB, W, EC, Jk, u, gd, vj, fac, out, stp, cr, nv, rv)); \
+    if (ws.bj.bs == 64) TDY_SPMV2(64, TI, EC, NRM);                                                                \
+    else if (ws.bj.bs == 256) TDY_SPMV2(256, TI, EC, NRM);                                                         \
+    else TDY_SPMV2(512, TI, EC, NRM);                                                                              \
   } while (0)
   if (ws.d_ecol16) {
     if (na) TDY_SPMV(int16_t, ws.d_ecol16, true);
@@ -903,6 +906,7 @@ static void spmv_apply(tdyhip_ctx *ctx, const KBufs<TV> &k, const TV *u, TV *vj,
     else TDY_SPMV(int32_t, ws.d_ecol, false);
   }
 #undef TDY_SPMV
+#undef TDY_SPMV2
   // the coarse solve runs in the multi-dot launch that follows (its first
   // workgroups), and the update kernel adds the prolongation
 }
