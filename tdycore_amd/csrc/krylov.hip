@@ -22,8 +22,16 @@ constexpr int kBlkMax = 512;  // max rows per block
 constexpr int kW = 27;        // max in-block entries per row (hexahedral vertex adjacency)
 constexpr int kLU = 13;       // max strictly lower (upper) entries per row
 // Factored block layout per row (slot-major, stride BS): slots 0..12 L
-// multipliers, 13..25 U entries, 26 the inverse diagonal; padded L/U slots hold
-// 0 and point at the zero entry x[BS] of the apply kernel's LDS vector.
+// multipliers (the nearest column first), 13..25 U entries (the nearest column
+// first), 26 the inverse diagonal; padded L/U slots hold 0 and point at the zero
+// entry x[BS] of the apply kernel's LDS vector.
+//
+// Chains: runs of consecutive rows (at most kChainMax, within 16 lanes) whose
+// only coupling inside the run is to the row before, as the lines of a brick.
+// The triangular sweeps solve a chain at once, so their levels are those of
+// the chains (14 for an 8x8x4 brick, against 34 of its rows).
+constexpr int kChainMax = 8;
+constexpr uint16_t kChainLink = 0x8000;  // row t couples to row t-1 (forward) or t+1 (backward) of its chain
 
 // Per-block arrays are strided by the block width BS (64, 256 or 512).
 struct BJLayout {
@@ -35,9 +43,11 @@ struct BJLayout {
   uint16_t *d_lcol = nullptr;  // nblocks*kW*bs local column (0xffff pad)
   uint8_t *d_diag = nullptr;   // nblocks*bs slot of the diagonal
   uint8_t *d_nslot = nullptr;  // nblocks*bs number of slots
-  uint16_t *d_levL = nullptr;  // nblocks*bs
-  uint16_t *d_levU = nullptr;  // nblocks*bs
-  int32_t *d_nlev = nullptr;   // nblocks*2 (L, U level counts)
+  uint16_t *d_levL = nullptr;  // nblocks*bs: level of each row in the factorization
+  int32_t *d_nlev = nullptr;   // nblocks: their count
+  uint16_t *d_swL = nullptr;   // nblocks*bs: level of each row's chain in the forward sweep, | kChainLink
+  uint16_t *d_swU = nullptr;   // nblocks*bs: the same for the backward sweep
+  int32_t *d_nsw = nullptr;    // nblocks*2 (forward, backward level counts)
   int32_t *d_nlu = nullptr;    // nblocks: L/U slots in use (the factor writes and the sweeps read only
                                // these); nullptr when every block uses all kLU
   int32_t *d_bw = nullptr;     // nblocks: ELL slots in use (the block's longest row; the SpMV reads only
@@ -137,7 +147,7 @@ k_bj_factor(BJLayout L, const double *__restrict__ J,
   }
   const int t = tid / TPR, sub = tid % TPR;  // row of the block, lane within the row
   const int lev = L.d_levL[base + t];
-  const int nlev = L.d_nlev[2 * pb];
+  const int nlev = L.d_nlev[pb];
   const int nsl = L.d_nslot[base + t];
   const int di0 = L.d_diag[base + t];
   // The update lists of lower slots p+1 .. p+AHEAD (count and this lane's
@@ -237,7 +247,7 @@ k_bj_factor(BJLayout L, const double *__restrict__ J,
   const int di = dg[t];
   const int nlu = L.d_nlu ? L.d_nlu[pb] : kLU;
   for (int p = sub; p < nlu; p += TPR) {
-    fac[sbase + (int64_t)p * BS + t] = (p < di) ? a[p][t] : (TV)0;
+    fac[sbase + (int64_t)p * BS + t] = (p < di) ? a[di - 1 - p][t] : (TV)0;
     const int q = di + 1 + p;
     fac[sbase + (int64_t)(kLU + p) * BS + t] = (q < nsl) ? a[q][t] : (TV)0;
   }
@@ -444,16 +454,43 @@ __device__ inline void restrict_block2(const TV *x, double &rr, TV v, double *rv
 // must call this; x[t] holds the right-hand side on entry and the solution on
 // return.
 //
+// A chain's rows are one level: each forms its right-hand side less the other
+// chains' products, and the recurrence along the chain, s_t += a_t s_(t-1), is
+// three register-shift steps with the products of consecutive a_t (a_t = 0 at
+// a chain's first row), formed once beside the loads.
+//
 // Between two barriers of a level stand LDS reads, the row's products and one
 // LDS write: on grids too small to hide it, that chain is the kernel's time,
 // so the products go into four sums (levels of thirteen dependent
-// multiply-adds took 68 steps a brick: 1M cells 106.7 -> 101.4 us).
+// multiply-adds: 1M cells 106.7 -> 101.4 us; by chains of rows instead of rows
+// 101.4 -> 89.4, FP32 at 442,368 rows 31.6 -> 22.9, 46k rows 19.0 -> 15.5).
 template <class TV>
 struct SweepRegs {  // a thread's row: factor entries and their local columns
   TV vl[kLU], vu[kLU], dinv;
+  TV al[3], au[3];  // products of 1, 2, 4 consecutive chain couplings
   uint16_t cl[kLU], cu[kLU];
   int levL, levU, nL, nU;
 };
+// v of the lane N before (row_shr) or after (row_shl) within 16 lanes, else 0
+template <int CTRL>
+__device__ inline float lane_shift(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true));
+}
+template <int CTRL>
+__device__ inline double lane_shift(double v) {
+  const uint64_t u = __double_as_longlong(v);
+  const uint32_t lo = __builtin_amdgcn_update_dpp(0, (int)u, CTRL, 0xf, 0xf, true);
+  const uint32_t hi = __builtin_amdgcn_update_dpp(0, (int)(u >> 32), CTRL, 0xf, 0xf, true);
+  return __longlong_as_double((long long)((uint64_t)hi << 32 | lo));
+}
+constexpr int kShr = 0x110, kShl = 0x100;  // + lanes
+template <int DIR, class TV>
+__device__ inline TV chain_solve(TV s, const TV (&a)[3]) {
+  s += a[0] * lane_shift<DIR + 1>(s);
+  s += a[1] * lane_shift<DIR + 2>(s);
+  s += a[2] * lane_shift<DIR + 4>(s);
+  return s;
+}
 template <class TV, int BS>
 __device__ inline void bj_sweeps_load(const BJLayout &L, const TV *__restrict__ fac, int b, int t, SweepRegs<TV> &r) {
   const int pb = L.d_pat ? L.d_pat[b] : b;  // index tables of the block's pattern
@@ -470,10 +507,23 @@ __device__ inline void bj_sweeps_load(const BJLayout &L, const TV *__restrict__ 
     r.cu[p] = in ? L.d_cU[cbase + (int64_t)p * BS + t] : (uint16_t)BS;
   }
   r.dinv = fac[sbase + (int64_t)(2 * kLU) * BS + t];
-  r.levL = L.d_levL[base + t];
-  r.levU = L.d_levU[base + t];
-  r.nL = L.d_nlev[2 * pb];
-  r.nU = L.d_nlev[2 * pb + 1];
+  const int wl = L.d_swL[base + t], wu = L.d_swU[base + t];
+  r.nL = L.d_nsw[2 * pb];
+  r.nU = L.d_nsw[2 * pb + 1];
+  r.levL = wl & ~kChainLink;
+  r.levU = wu & ~kChainLink;
+  // the chain's couplings leave the products: slot 0 is the nearest column
+  const bool ll = wl & kChainLink, lu = wu & kChainLink;
+  r.al[0] = ll ? -r.vl[0] : (TV)0;
+  r.au[0] = lu ? -r.vu[0] * r.dinv : (TV)0;
+  r.vl[0] = ll ? (TV)0 : r.vl[0];
+  r.vu[0] = lu ? (TV)0 : r.vu[0];
+  r.cl[0] = ll ? (uint16_t)BS : r.cl[0];
+  r.cu[0] = lu ? (uint16_t)BS : r.cu[0];
+  r.al[1] = r.al[0] * lane_shift<kShr + 1>(r.al[0]);
+  r.al[2] = r.al[1] * lane_shift<kShr + 2>(r.al[1]);
+  r.au[1] = r.au[0] * lane_shift<kShl + 1>(r.au[0]);
+  r.au[2] = r.au[1] * lane_shift<kShl + 2>(r.au[1]);
 }
 // x - sum v[p] x[c[p]], the products in four sums
 template <class TV>
@@ -491,11 +541,11 @@ __device__ inline void bj_sweeps_run(const SweepRegs<TV> &r, TV *x, int t) {
   __syncthreads();
   // forward: branch-free inner loop, all LDS reads of a level in flight together
   for (int l = 0; l < r.nL; l++) {
-    if (r.levL == l) x[t] = sweep_row(x, x[t], r.vl, r.cl);
+    if (r.levL == l) x[t] = chain_solve<kShr>(sweep_row(x, x[t], r.vl, r.cl), r.al);
     __syncthreads();
   }
   for (int l = 0; l < r.nU; l++) {
-    if (r.levU == l) x[t] = sweep_row(x, x[t], r.vu, r.cu) * r.dinv;
+    if (r.levU == l) x[t] = chain_solve<kShl>(sweep_row(x, x[t], r.vu, r.cu) * r.dinv, r.au);
     __syncthreads();
   }
 }

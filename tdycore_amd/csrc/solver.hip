@@ -20,10 +20,10 @@ struct HostBJ {
   int nblocks = 0, bs = 0;
   std::vector<int32_t> row, jpos;
   std::vector<uint8_t> diag, nslot;
-  std::vector<uint16_t> lcol, levL, levU, cL, cU;
+  std::vector<uint16_t> lcol, levL, swL, swU, cL, cU;
   std::vector<uint32_t> pair;
   std::vector<uint8_t> npair;
-  std::vector<int32_t> nlev;
+  std::vector<int32_t> nlev, nsw;
   std::vector<int32_t> nlu;   // nblocks: most strictly lower (or upper) in-block entries of a row
   std::vector<int32_t> perm;  // nc: block-layout position of each cell
   std::vector<int32_t> bw;    // nblocks: longest row of each block (ELL slots in use)
@@ -103,18 +103,20 @@ static std::string build_bj(const std::vector<int32_t> &jrp, const std::vector<i
   out.diag.assign((size_t)nb * S, 0);
   out.nslot.assign((size_t)nb * S, 0);
   out.levL.assign((size_t)nb * S, 0);
-  out.levU.assign((size_t)nb * S, 0);
+  out.swL.assign((size_t)nb * S, 0);
+  out.swU.assign((size_t)nb * S, 0);
   out.cL.assign((size_t)nb * kLU * S, (uint16_t)S);
   out.cU.assign((size_t)nb * kLU * S, (uint16_t)S);
   out.npair.assign((size_t)nb * kLU * S, 0);
   out.pair.assign((size_t)nb * kPair * S, 0);
-  out.nlev.assign((size_t)nb * 2, 0);
+  out.nlev.assign((size_t)nb, 0);
+  out.nsw.assign((size_t)nb * 2, 0);
   out.nlu.assign((size_t)nb, 0);
   for (int b = 0; b < nb; b++) {
     const auto &mem = members[b];
     const int m = (int)mem.size();
     for (int i = 0; i < m; i++) local[mem[i]] = i;
-    int maxL = 0, maxU = 0;
+    int maxL = 0;
     for (int i = 0; i < m; i++) {
       const int r = mem[i];
       out.row[(size_t)b * S + i] = r;
@@ -132,7 +134,8 @@ static std::string build_bj(const std::vector<int32_t> &jrp, const std::vector<i
       }
       out.nslot[(size_t)b * S + i] = (uint8_t)ns;
     }
-    // levels: L forward, U backward
+    std::vector<int> chain(m, 0);
+    // factorization levels of the rows
     for (int i = 0; i < m; i++) {
       int lv = 0;
       const int di = out.diag[(size_t)b * S + i];
@@ -143,18 +146,51 @@ static std::string build_bj(const std::vector<int32_t> &jrp, const std::vector<i
       out.levL[(size_t)b * S + i] = (uint16_t)lv;
       maxL = std::max(maxL, lv + 1);
     }
-    for (int i = m - 1; i >= 0; i--) {
-      int lv = 0;
-      const int di = out.diag[(size_t)b * S + i], ns = out.nslot[(size_t)b * S + i];
-      for (int p = di + 1; p < ns; p++) {
-        const int k = out.lcol[(size_t)b * kW * S + (size_t)p * S + i];
-        lv = std::max(lv, (int)out.levU[(size_t)b * S + k] + 1);
-      }
-      out.levU[(size_t)b * S + i] = (uint16_t)lv;
-      maxU = std::max(maxU, lv + 1);
+    out.nlev[b] = maxL;
+    // chains (see kChainMax): a row joins the run before it when its only lower
+    // entry inside the run is the row before (the pattern is symmetric, so a
+    // row's only upper entry inside is then the row after)
+    for (int i = 0; i < m; i++) {
+      const int di = out.diag[(size_t)b * S + i];
+      const int prev = di > 0 ? out.lcol[(size_t)b * kW * S + (size_t)(di - 1) * S + i] : -1;
+      const int prev2 = di > 1 ? out.lcol[(size_t)b * kW * S + (size_t)(di - 2) * S + i] : -1;
+      const int start = i > 0 ? chain[i - 1] : 0;
+      // (row i - 1 then has row i as its first upper entry)
+      const bool join = i > 0 && i % 16 != 0 && prev == i - 1 && prev2 < start && i - start < kChainMax;
+      chain[i] = join ? start : i;
     }
-    out.nlev[2 * b] = maxL;
-    out.nlev[2 * b + 1] = maxU;
+    // sweep levels of the chains: forward over the runs, backward from the last
+    int fwd = 0, bwd = 0;
+    for (int i = 0; i < m;) {
+      int e = i, lv = 0;
+      while (e < m && chain[e] == i) {
+        const int di = out.diag[(size_t)b * S + e];
+        for (int p = 0; p < di; p++) {
+          const int k = out.lcol[(size_t)b * kW * S + (size_t)p * S + e];
+          if (k < i) lv = std::max(lv, (out.swL[(size_t)b * S + k] & ~kChainLink) + 1);
+        }
+        e++;
+      }
+      for (int r = i; r < e; r++) out.swL[(size_t)b * S + r] = (uint16_t)(lv | (r > i ? kChainLink : 0));
+      fwd = std::max(fwd, lv + 1);
+      i = e;
+    }
+    for (int e = m; e > 0;) {
+      const int i = chain[e - 1];
+      int lv = 0;
+      for (int r = i; r < e; r++) {
+        const int di = out.diag[(size_t)b * S + r], ns = out.nslot[(size_t)b * S + r];
+        for (int p = di + 1; p < ns; p++) {
+          const int k = out.lcol[(size_t)b * kW * S + (size_t)p * S + r];
+          if (k >= e) lv = std::max(lv, (out.swU[(size_t)b * S + k] & ~kChainLink) + 1);
+        }
+      }
+      for (int r = i; r < e; r++) out.swU[(size_t)b * S + r] = (uint16_t)(lv | (r + 1 < e ? kChainLink : 0));
+      bwd = std::max(bwd, lv + 1);
+      e = i;
+    }
+    out.nsw[2 * b] = fwd;
+    out.nsw[2 * b + 1] = bwd;
     // split L / U column tables (padding -> the zero entry S)
     for (int i = 0; i < m; i++) {
       const int di = out.diag[(size_t)b * S + i], ns = out.nslot[(size_t)b * S + i];
@@ -180,7 +216,7 @@ static std::string build_bj(const std::vector<int32_t> &jrp, const std::vector<i
       }
       for (int p = 0; p < kLU; p++) {
         out.cL[(size_t)b * kLU * S + (size_t)p * S + i] =
-            p < di ? out.lcol[(size_t)b * kW * S + (size_t)p * S + i] : (uint16_t)S;
+            p < di ? out.lcol[(size_t)b * kW * S + (size_t)(di - 1 - p) * S + i] : (uint16_t)S;
         const int q = di + 1 + p;
         out.cU[(size_t)b * kLU * S + (size_t)p * S + i] =
             q < ns ? out.lcol[(size_t)b * kW * S + (size_t)q * S + i] : (uint16_t)S;
@@ -239,8 +275,8 @@ static std::string build_bj(const std::vector<int32_t> &jrp, const std::vector<i
       add(out.jpos, b * sw, sw); add(out.lcol, b * sw, sw);
       add(out.npair, b * lu, lu); add(out.pair, b * pw, pw);
       add(out.diag, (size_t)b * S, S); add(out.nslot, (size_t)b * S, S);
-      add(out.levL, (size_t)b * S, S); add(out.levU, (size_t)b * S, S);
-      add(out.nlev, (size_t)2 * b, 2);
+      add(out.levL, (size_t)b * S, S); add(out.swL, (size_t)b * S, S); add(out.swU, (size_t)b * S, S);
+      add(out.nlev, (size_t)b, 1); add(out.nsw, (size_t)2 * b, 2);
       add(out.nlu, (size_t)b, 1);
       for (int k = 0; k < W; k++) key.append((const char *)(out.ecol16.data() + (size_t)k * NB + (size_t)b * S), (size_t)S * 2);
       auto it = seen.find(key);
@@ -261,7 +297,8 @@ static std::string build_bj(const std::vector<int32_t> &jrp, const std::vector<i
       };
       shrink(out.cL, lu); shrink(out.cU, lu); shrink(out.jpos, sw); shrink(out.lcol, sw);
       shrink(out.npair, lu); shrink(out.pair, pw); shrink(out.diag, S); shrink(out.nslot, S);
-      shrink(out.levL, S); shrink(out.levU, S); shrink(out.nlev, 2); shrink(out.nlu, 1);
+      shrink(out.levL, S); shrink(out.swL, S); shrink(out.swU, S); shrink(out.nlev, 1); shrink(out.nsw, 2);
+      shrink(out.nlu, 1);
       std::vector<int16_t> e16((size_t)npat * W * S);
       for (int q = 0; q < npat; q++)
         for (int k = 0; k < W; k++)
@@ -642,7 +679,8 @@ static int ensure_ws(tdyhip_ctx *ctx, const tdyhip_solver_opts &o) {
   ws.part_version = ctx->pc_part_version;
   if ((rc = up(&ws.bj.d_row, hb.row)) || (rc = up(&ws.bj.d_jpos, hb.jpos)) || (rc = up(&ws.bj.d_lcol, hb.lcol)) ||
       (rc = up(&ws.bj.d_diag, hb.diag)) || (rc = up(&ws.bj.d_nslot, hb.nslot)) || (rc = up(&ws.bj.d_levL, hb.levL)) ||
-      (rc = up(&ws.bj.d_levU, hb.levU)) || (rc = up(&ws.bj.d_nlev, hb.nlev)) || (rc = up(&ws.bj.d_cL, hb.cL)) ||
+      (rc = up(&ws.bj.d_swL, hb.swL)) || (rc = up(&ws.bj.d_swU, hb.swU)) || (rc = up(&ws.bj.d_nlev, hb.nlev)) ||
+      (rc = up(&ws.bj.d_nsw, hb.nsw)) || (rc = up(&ws.bj.d_cL, hb.cL)) ||
       (rc = up(&ws.bj.d_cU, hb.cU)) || (rc = up(&ws.bj.d_npair, hb.npair)) || (rc = up(&ws.bj.d_pair, hb.pair)))
     return rc;
   for (double **p : {&ws.F, &ws.Y, &ws.W, &ws.G, &ws.JY, &ws.Udot, &ws.Uprev_ts, &ws.Usave})
