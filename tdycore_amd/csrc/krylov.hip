@@ -40,11 +40,8 @@ struct BJLayout {
   int32_t *d_row = nullptr;    // nblocks*bs global row (-1 pad)
   int32_t *d_jpos = nullptr;   // nblocks*kW*bs position in the ELL Jacobian less the block's first entry (-1 pad)
   int ell_w = 0;               // ELL width W: block b's entries start at b*W*bs
-  uint16_t *d_lcol = nullptr;  // nblocks*kW*bs local column (0xffff pad)
   uint8_t *d_diag = nullptr;   // nblocks*bs slot of the diagonal
   uint8_t *d_nslot = nullptr;  // nblocks*bs number of slots
-  uint16_t *d_levL = nullptr;  // nblocks*bs: level of each row in the factorization
-  int32_t *d_nlev = nullptr;   // nblocks: their count
   uint16_t *d_swL = nullptr;   // nblocks*bs: level of each row's chain in the forward sweep, | kChainLink
   uint16_t *d_swU = nullptr;   // nblocks*bs: the same for the backward sweep
   int32_t *d_nsw = nullptr;    // nblocks*2 (forward, backward level counts)
@@ -54,11 +51,15 @@ struct BJLayout {
                                // these); nullptr when every block reads all W
   uint16_t *d_cL = nullptr;    // nblocks*kLU*bs local column of L slot (bs = zero entry)
   uint16_t *d_cU = nullptr;    // nblocks*kLU*bs local column of U slot
-  // ILU(0) update lists: for row i and lower slot p (row k), pairs (d, s) with
-  // a_i[d] -= l_ik * a_k[s]; npair[p] pairs per p, each packed d | s << 8 in
-  // 16 bits, pairs q and q+1 of slot p sharing the 32-bit word p*kPairW + q/2.
-  uint8_t *d_npair = nullptr;  // nblocks*kLU*bs
-  uint32_t *d_pair = nullptr;  // nblocks*kPair*bs (kPair = kLU*kPairW words per row)
+  // Factorization: rows by level (lrow, levels starting at lptr[0..nlev]) and,
+  // per row, 16 bytes for each of 32 lanes, lane d standing for slot d: bytes
+  // 0..12 the slot of row k_p (k_p the column of lower slot p) that holds slot
+  // d's column (kNoSlot: none, or d <= p), then slot d's column (16 bits) and the row's
+  // diagonal slot.
+  uint16_t *d_lrow = nullptr;  // nblocks*bs
+  uint16_t *d_lptr = nullptr;  // nblocks*(bs+1)
+  int32_t *d_nlev = nullptr;   // nblocks: levels
+  uint4 *d_ftab = nullptr;     // nblocks*bs*kFacLanes
   // Shared index patterns: every index table above except d_row (and the
   // solver's int16 column offsets) holds one entry per pattern, block b using
   // pattern d_pat[b]; nullptr: every block has its own.
@@ -66,8 +67,8 @@ struct BJLayout {
   int npat = 0;
 };
 
-constexpr int kPairW = (kLU + 1) / 2;  // 32-bit words per lower slot (two 16-bit pairs each)
-constexpr int kPair = kLU * kPairW;    // pair words per row
+constexpr int kFacLanes = 32;   // lanes per row of the factorization
+constexpr uint8_t kNoSlot = kW; // a row's slot past its entries: holds 0 in the factorization's LDS
 
 // ---------------------------------------------------------------- device-resident GMRES cycle
 // State shared by the kernels of one restart cycle; `done` makes every later
@@ -88,170 +89,131 @@ struct GmresDev {
 };
 
 // ---------------------------------------------------------------- ILU(0) factor
-// TPR lanes (adjacent, so in one wavefront) share a row: each computes the
-// row's multiplier for lower slot p and applies its share of the slot's
-// update pairs (the targets of one slot are distinct), which shortens the
-// sequential elimination chain of each level about TPR times.  Lanes of one
-// wavefront issue their LDS operations in program order, so the writes of
-// slot p are seen by the reads of slot p+1 without a barrier.
+// IKJ elimination level by level, half a wavefront per row, lane d holding the
+// row's slot d in a register.  The rows k_p a row eliminates with are finished,
+// so everything read of them (their entry in slot d's column, one LDS read per
+// lower slot, and the reciprocal pivot of the lane's own column) is in flight
+// before the first multiplier; what remains per lower slot is a product, a
+// broadcast through scalar registers and a multiply-add.  The next level's table
+// entries are fetched a level ahead.
+//
+// Bound by that chain: 34 levels of an 8x8x4 brick.  (Values updated in LDS by
+// lists of pairs, four lanes per row, waited for about eight LDS round trips
+// and a division per lower slot: 8x8x4 bricks, 1M cells 1825 -> 472 us, FP32 at
+// 442,368 cells 657 -> 150, 63k 214 -> 74; 4x4x4 bricks, 4k cells 91 -> 31.)
+constexpr int kFacPitch = kW + 2;  // a row's LDS pitch: its slots, the zero kNoSlot points at, odd
 template <int BS>
 struct FactorLanes {
-  static constexpr int TPR = BS <= 256 ? 4 : 2;  // lanes per row (workgroup <= 1024 threads)
-  static constexpr int NT = BS * TPR;
-  static constexpr int WPL = (kPairW + TPR - 1) / TPR;  // pair words per lane
-  static constexpr int AHEAD = 2;                        // lower slots whose update lists are in flight
-  // waves per SIMD the registers are budgeted for (at most 64 VGPRs at 8):
-  // two 16-wave workgroups per CU, as many as the LDS holds at BS <= 256
-  static constexpr int WAVES = BS <= 256 ? 8 : 4;
+  static constexpr int NT = BS == 64 ? 256 : 512;
+  static constexpr int ROWS = NT / kFacLanes;  // rows at once
 };
 
+template <class TV>
+__device__ inline TV lane_bcast(TV v, int lane);  // lane uniform
+template <>
+__device__ inline float lane_bcast<float>(float v, int lane) {
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
+}
+template <>
+__device__ inline double lane_bcast<double>(double v, int lane) {
+  const uint64_t u = __double_as_longlong(v);
+  const uint32_t lo = __builtin_amdgcn_readlane((int)u, lane), hi = __builtin_amdgcn_readlane((int)(u >> 32), lane);
+  return __longlong_as_double((long long)((uint64_t)hi << 32 | lo));
+}
+
 template <class TV, int BS>
-__global__ void __launch_bounds__(FactorLanes<BS>::NT) __attribute__((amdgpu_waves_per_eu(FactorLanes<BS>::WAVES)))
-k_bj_factor(BJLayout L, const double *__restrict__ J,
-                                                                   TV *__restrict__ fac, int *__restrict__ status) {
-  constexpr int TPR = FactorLanes<BS>::TPR, NT = FactorLanes<BS>::NT, WPL = FactorLanes<BS>::WPL;
-  __shared__ TV a[kW][BS];
-  __shared__ uint16_t lc[kW][BS];
-  __shared__ uint8_t dg[BS];
-  __shared__ uint8_t ns[BS];
+__global__ void __launch_bounds__(FactorLanes<BS>::NT)
+k_bj_factor(BJLayout L, const double *__restrict__ J, TV *__restrict__ fac, int *__restrict__ status) {
+  constexpr int NT = FactorLanes<BS>::NT, ROWS = FactorLanes<BS>::ROWS;
+  __shared__ TV a[BS * kFacPitch];
+  __shared__ TV piv[BS];  // reciprocal pivots of the finished rows
+  __shared__ uint16_t lrow[BS], lptr[BS + 1];
   const int b = blockIdx.x, tid = threadIdx.x;
   // index tables of the block's pattern (shared by identical blocks); values per block
   const int pb = L.d_pat ? L.d_pat[b] : b;
   const int64_t base = (int64_t)pb * BS;
   const int64_t ibase = (int64_t)pb * kW * BS;
   const int64_t sbase = (int64_t)b * kW * BS;
+  const int nlev = L.d_nlev[pb];
   {
-    // all of the block's value loads in flight together
-    constexpr int NE = (kW * BS + NT - 1) / NT;
+    // the block's value loads, a batch in flight together
+    constexpr int NB = 14;
     const double *Jb = J + (int64_t)b * L.ell_w * BS;
-    int32_t pos[NE];
-    uint16_t lcv[NE];
+    for (int e0 = tid; e0 < kW * BS; e0 += NB * NT) {
+      int32_t pos[NB];
+      TV v[NB];
 #pragma unroll
-    for (int i = 0; i < NE; i++) {
-      const int e = tid + i * NT;
-      pos[i] = e < kW * BS ? L.d_jpos[ibase + e] : -1;  // relative to the block's first position
-      lcv[i] = e < kW * BS ? L.d_lcol[ibase + e] : (uint16_t)0;
-    }
+      for (int i = 0; i < NB; i++) pos[i] = e0 + i * NT < kW * BS ? L.d_jpos[ibase + e0 + i * NT] : -1;
 #pragma unroll
-    for (int i = 0; i < NE; i++) {
-      const int e = tid + i * NT;
-      if (e < kW * BS) {
-        a[e / BS][e % BS] = (pos[i] >= 0) ? (TV)Jb[pos[i]] : (TV)0;
-        lc[e / BS][e % BS] = lcv[i];
+      for (int i = 0; i < NB; i++) v[i] = pos[i] >= 0 ? (TV)Jb[pos[i]] : (TV)0;  // relative to the block's first position
+#pragma unroll
+      for (int i = 0; i < NB; i++) {
+        const int e = e0 + i * NT;
+        if (e < kW * BS) a[(e % BS) * kFacPitch + e / BS] = v[i];
       }
     }
   }
   for (int r = tid; r < BS; r += NT) {
-    ns[r] = L.d_nslot[base + r];
-    dg[r] = L.d_diag[base + r];
+    a[r * kFacPitch + kNoSlot] = (TV)0;
+    piv[r] = (TV)0;
+    lrow[r] = L.d_lrow[base + r];
   }
-  const int t = tid / TPR, sub = tid % TPR;  // row of the block, lane within the row
-  const int lev = L.d_levL[base + t];
-  const int nlev = L.d_nlev[pb];
-  const int nsl = L.d_nslot[base + t];
-  const int di0 = L.d_diag[base + t];
-  // The update lists of lower slots p+1 .. p+AHEAD (count and this lane's
-  // packed pair words) are in flight while slot p is eliminated, the first
-  // ones fetched before the level loop, so global-memory latency is off the
-  // elimination chain.  The slot loop is unrolled and the loads carry no
-  // condition (the tables hold kLU slots per row; a lane's words past the
-  // row's kPairW re-read the last one and are never used), so each list
-  // lands in registers of its own and the wait before slot p is for slot p's
-  // loads alone.  (A rotating queue in a rolled loop copies registers whose
-  // loads are pending, which waits for every load at every slot.  At 1M
-  // cells the FP32 factor went from 1579 to 1372 us; FP64, 1709 -> 1744 us,
-  // is held by its LDS chain instead.)
-  // A slot's table rows are addressed as a uniform base plus this lane's
-  // 32-bit offset.  The base takes an opaque zero made where it is used, so
-  // the compiler cannot hoist the thirteen slots' addresses out of the level
-  // loop, where they would hold 64-bit addresses in vector registers.
-  const uint32_t *__restrict__ pairs = L.d_pair + (int64_t)pb * kPair * BS;
-  const uint8_t *__restrict__ npair = L.d_npair + (int64_t)pb * kLU * BS;
-  uint32_t woff[WPL];
-#pragma unroll
-  for (int i = 0; i < WPL; i++) woff[i] = (uint32_t)(min(sub + TPR * i, kPairW - 1) * BS + t);
-  auto fetch = [&](int p, int &cnt, uint32_t (&w)[WPL]) {
-    int z;
-    asm volatile("s_mov_b32 %0, 0" : "=s"(z));
-    cnt = (npair + (p * BS + z))[(uint32_t)t];
-    const uint32_t *__restrict__ pp = pairs + (p * kPairW * BS + z);
-#pragma unroll
-    for (int i = 0; i < WPL; i++) w[i] = pp[woff[i]];
-  };
-  constexpr int kAhead = FactorLanes<BS>::AHEAD;
-  int nq[kLU];
-  uint32_t qw[kLU][WPL];
-#pragma unroll
-  for (int d = 0; d < kAhead; d++) fetch(d, nq[d], qw[d]);
+  for (int r = tid; r <= nlev; r += NT) lptr[r] = L.d_lptr[(int64_t)pb * (BS + 1) + r];
   __syncthreads();
+  const int d = tid % kFacLanes, hw = tid / kFacLanes;
+  const bool hi = (tid & 32) != 0;
+  const uint4 *tab = L.d_ftab + (int64_t)pb * BS * kFacLanes + d;
+  auto fetch = [&](int j, int end) {  // the table entry of the level's row j (a row past the end re-reads row 0's)
+    return tab[(int64_t)(j < end ? lrow[j] : 0) * kFacLanes];
+  };
+  uint4 nt = fetch(lptr[0] + hw, lptr[1]);
   for (int l = 0; l < nlev; l++) {
-    if (lev == l && nsl > 0) {
-      // A slot's LDS reads go out as one batch: its own value, the pivot of
-      // row k (finished at an earlier level), the pair sources in row k and
-      // the pair targets in row t (distinct slots above p, so no read of the
-      // batch waits for a write of the same slot), and the next slot's
-      // column; the next column's diagonal slot is read behind the writes.
-      // (the first lists pass through an empty asm here, so nothing derived
-      // from them is hoisted out of the level loop into spilled registers)
+    const int j0 = lptr[l], j1 = lptr[l + 1], j2 = l + 1 < nlev ? lptr[l + 2] : j1;
+    for (int jb = j0; jb < j1; jb += ROWS) {  // uniform over the workgroup
+      const int j = jb + hw;
+      const bool live = j < j1;
+      const uint4 tb = nt;
+      nt = jb + ROWS < j1 ? fetch(jb + ROWS + hw, j1) : fetch(j1 + hw, j2);
+      const int r = live ? lrow[j] : 0;
+      const int c = (tb.w >> 8) & 0xffff, di = live ? (int)(tb.w >> 24) : 0;
+      TV v = d < kW ? a[r * kFacPitch + d] : (TV)0;
+      const TV ip = d < di ? piv[c] : (TV)0;
+      const int pmax = max(__builtin_amdgcn_readlane(di, 0), __builtin_amdgcn_readlane(di, 32));
+      const uint32_t tw[4] = {tb.x, tb.y, tb.z, tb.w};
+      TV src[kLU];
 #pragma unroll
-      for (int d = 0; d < kAhead; d++) {
-        asm volatile("" : "+v"(nq[d]));
+      for (int p = 0; p < kLU; p++)
+        if (p < pmax) {
+          const int k0 = __builtin_amdgcn_readlane(c, p), k1 = __builtin_amdgcn_readlane(c, 32 + p);
+          src[p] = a[(hi ? k1 : k0) * kFacPitch + ((tw[p / 4] >> (8 * (p % 4))) & 0xff)];
+        }
 #pragma unroll
-        for (int i = 0; i < WPL; i++) asm volatile("" : "+v"(qw[d][i]));
-      }
-      int k = di0 > 0 ? lc[0][t] : t;
-      int dk = dg[k];
-#pragma unroll
-      for (int p = 0; p < kLU; p++) {  // lower entries, increasing column
-        if (p + kAhead < kLU) fetch(p + kAhead, nq[p + kAhead], qw[p + kAhead]);
-        if (p < di0) {
-          const int ncur = nq[p];
-          const uint32_t *cur = qw[p];
-          TV src[2 * WPL], tgt[2 * WPL];
-#pragma unroll
-          for (int i = 0; i < WPL; i++) {
-#pragma unroll
-            for (int h = 0; h < 2; h++) {
-              const int q = 2 * (sub + TPR * i) + h;  // pair index of this lane's half-word
-              const uint32_t w = (q < ncur) ? (h ? (cur[i] >> 16) : (cur[i] & 0xffffu)) : 0u;  // unused pairs read slot 0
-              src[2 * i + h] = a[w >> 8][k];
-              tgt[2 * i + h] = a[w & 0xff][t];
-            }
-          }
-          const TV pv = a[dk][k];
-          const TV ap = a[p][t];
-          const int kn = (p + 1 < di0) ? lc[p + 1][t] : k;
-          const TV lik = ap / pv;
-          __builtin_amdgcn_wave_barrier();  // every lane has read a[p][t] before it is overwritten
-          if (sub == 0) a[p][t] = lik;
-#pragma unroll
-          for (int i = 0; i < WPL; i++) {
-#pragma unroll
-            for (int h = 0; h < 2; h++) {
-              const int q = 2 * (sub + TPR * i) + h;
-              const uint32_t w = h ? (cur[i] >> 16) : (cur[i] & 0xffffu);
-              if (q < ncur) a[w & 0xff][t] = tgt[2 * i + h] - lik * src[2 * i + h];
-            }
-          }
-          const int dkn = dg[kn];
-          __builtin_amdgcn_wave_barrier();
-          k = kn;
-          dk = dkn;
+      for (int p = 0; p < kLU; p++)
+        if (p < pmax) {
+          const TV m = v * ip;
+          const TV m0 = lane_bcast(m, p), m1 = lane_bcast(m, 32 + p);
+          v -= (hi ? m1 : m0) * src[p];
+        }
+      if (live && d < kW) {
+        a[r * kFacPitch + d] = d < di ? v * ip : v;
+        if (d == di) {
+          piv[r] = (TV)1 / v;
+          if (v == (TV)0) atomicOr(status, 1);
         }
       }
-      if (sub == 0 && a[dg[t]][t] == (TV)0) atomicOr(status, 1);
     }
     __syncthreads();
   }
-  // split layout: L multipliers, U entries, inverse diagonal
-  const int di = dg[t];
+  // split layout: L multipliers and U entries by distance from the diagonal, reciprocal pivot
   const int nlu = L.d_nlu ? L.d_nlu[pb] : kLU;
-  for (int p = sub; p < nlu; p += TPR) {
-    fac[sbase + (int64_t)p * BS + t] = (p < di) ? a[di - 1 - p][t] : (TV)0;
+  for (int e = tid; e < nlu * BS; e += NT) {
+    const int p = e / BS, t = e % BS;
+    const int di = L.d_diag[base + t], ns = L.d_nslot[base + t];
+    fac[sbase + (int64_t)p * BS + t] = (p < di) ? a[t * kFacPitch + di - 1 - p] : (TV)0;
     const int q = di + 1 + p;
-    fac[sbase + (int64_t)(kLU + p) * BS + t] = (q < nsl) ? a[q][t] : (TV)0;
+    fac[sbase + (int64_t)(kLU + p) * BS + t] = (q < ns) ? a[t * kFacPitch + q] : (TV)0;
   }
-  if (sub == 0) fac[sbase + (int64_t)(2 * kLU) * BS + t] = nsl > 0 ? (TV)1 / a[di][t] : (TV)0;
+  for (int t = tid; t < BS; t += NT) fac[sbase + (int64_t)(2 * kLU) * BS + t] = piv[t];
 }
 
 // This thread's share of p[0..n) in a workgroup of NT threads: the sum of

@@ -20,17 +20,16 @@ struct HostBJ {
   int nblocks = 0, bs = 0;
   std::vector<int32_t> row, jpos;
   std::vector<uint8_t> diag, nslot;
-  std::vector<uint16_t> lcol, levL, swL, swU, cL, cU;
-  std::vector<uint32_t> pair;
-  std::vector<uint8_t> npair;
+  std::vector<uint16_t> lcol, lrow, lptr, swL, swU, cL, cU;
+  std::vector<uint4> ftab;
   std::vector<int32_t> nlev, nsw;
   std::vector<int32_t> nlu;   // nblocks: most strictly lower (or upper) in-block entries of a row
   std::vector<int32_t> perm;  // nc: block-layout position of each cell
   std::vector<int32_t> bw;    // nblocks: longest row of each block (ELL slots in use)
   std::vector<int32_t> ecol;  // W*nblocks*bs: global column of slot k at block position p (k*NB + p)
   std::vector<int16_t> ecol16;  // the same as offsets from the row, when every offset fits in int16
-  // Deduplicated index patterns (int16 offsets only): blocks whose L/U local
-  // columns and column offsets are identical share one copy.  When set, cL/cU
+  // Deduplicated index patterns (int16 offsets only): blocks whose local columns
+  // and column offsets are identical share one copy.  When set, the index tables
   // hold npat patterns and ecol16 is pattern-major: slot k of thread t of
   // pattern q at (q*W + k)*bs + t.
   std::vector<int32_t> pat;     // nblocks: pattern of each block (empty: one copy per block)
@@ -102,21 +101,10 @@ static std::string build_bj(const std::vector<int32_t> &jrp, const std::vector<i
   out.lcol.assign((size_t)nb * kW * S, 0xffff);
   out.diag.assign((size_t)nb * S, 0);
   out.nslot.assign((size_t)nb * S, 0);
-  out.levL.assign((size_t)nb * S, 0);
-  out.swL.assign((size_t)nb * S, 0);
-  out.swU.assign((size_t)nb * S, 0);
-  out.cL.assign((size_t)nb * kLU * S, (uint16_t)S);
-  out.cU.assign((size_t)nb * kLU * S, (uint16_t)S);
-  out.npair.assign((size_t)nb * kLU * S, 0);
-  out.pair.assign((size_t)nb * kPair * S, 0);
-  out.nlev.assign((size_t)nb, 0);
-  out.nsw.assign((size_t)nb * 2, 0);
-  out.nlu.assign((size_t)nb, 0);
   for (int b = 0; b < nb; b++) {
     const auto &mem = members[b];
     const int m = (int)mem.size();
     for (int i = 0; i < m; i++) local[mem[i]] = i;
-    int maxL = 0;
     for (int i = 0; i < m; i++) {
       const int r = mem[i];
       out.row[(size_t)b * S + i] = r;
@@ -134,19 +122,146 @@ static std::string build_bj(const std::vector<int32_t> &jrp, const std::vector<i
       }
       out.nslot[(size_t)b * S + i] = (uint8_t)ns;
     }
-    std::vector<int> chain(m, 0);
-    // factorization levels of the rows
-    for (int i = 0; i < m; i++) {
-      int lv = 0;
-      const int di = out.diag[(size_t)b * S + i];
-      for (int p = 0; p < di; p++) {
-        const int k = out.lcol[(size_t)b * kW * S + (size_t)p * S + i];
-        lv = std::max(lv, (int)out.levL[(size_t)b * S + k] + 1);
-      }
-      out.levL[(size_t)b * S + i] = (uint16_t)lv;
-      maxL = std::max(maxL, lv + 1);
+    for (int i = 0; i < m; i++) local[mem[i]] = -1;
+  }
+  // block-ordered ELL columns (padding slots point at the row itself with a 0 value)
+  out.perm.assign(nc, -1);
+  out.ecol.assign((size_t)W * NB, 0);
+  for (int64_t p = 0; p < NB; p++) {
+    const int r = out.row[p];
+    if (r < 0) continue;
+    out.perm[r] = (int32_t)p;
+    const int len = jrp[r + 1] - jrp[r];
+    for (int k = 0; k < W; k++) out.ecol[(size_t)k * NB + p] = k < len ? jcols[jrp[r] + k] : r;
+  }
+  for (int c = 0; c < nc; c++)
+    if (out.perm[c] < 0) return "cell missing from the block-Jacobi partition";
+  out.bw.assign(out.nblocks, 0);
+  for (int64_t p = 0; p < NB; p++) {
+    const int r = out.row[p];
+    if (r >= 0) out.bw[p / S] = std::max(out.bw[p / S], jrp[r + 1] - jrp[r]);
+  }
+  bool fits = true;
+  for (int64_t p = 0; p < NB && fits; p++) {
+    const int r = out.row[p];
+    for (int k = 0; k < W && fits; k++) {
+      const int64_t off = r < 0 ? 0 : (int64_t)out.ecol[(size_t)k * NB + p] - r;
+      fits = off >= INT16_MIN && off <= INT16_MAX;
     }
-    out.nlev[b] = maxL;
+  }
+  if (fits) {
+    out.ecol16.resize(out.ecol.size());
+    for (int64_t p = 0; p < NB; p++) {
+      const int r = out.row[p];
+      for (int k = 0; k < W; k++)
+        out.ecol16[(size_t)k * NB + p] = r < 0 ? 0 : (int16_t)(out.ecol[(size_t)k * NB + p] - r);
+    }
+    out.ecol.clear();
+    // Blocks of a structured mesh repeat a few index patterns (an interior
+    // brick's in-block columns and column offsets are those of every other
+    // interior brick): keep one copy per pattern when that at least halves
+    // them, so the matvec streams values, not indices.
+    const size_t sw = (size_t)kW * S;
+    std::unordered_map<std::string, int> seen;
+    std::vector<int> rep;
+    std::vector<int32_t> pat(nb);
+    std::string key;
+    auto add = [&](const auto &v, size_t off, size_t n) {
+      key.append((const char *)(v.data() + off), n * sizeof(v[0]));
+    };
+    for (int b = 0; b < nb; b++) {
+      key.clear();
+      add(out.jpos, b * sw, sw); add(out.lcol, b * sw, sw);
+      add(out.diag, (size_t)b * S, S); add(out.nslot, (size_t)b * S, S);
+      for (int k = 0; k < W; k++) key.append((const char *)(out.ecol16.data() + (size_t)k * NB + (size_t)b * S), (size_t)S * 2);
+      auto it = seen.find(key);
+      if (it == seen.end()) {
+        it = seen.emplace(key, (int)rep.size()).first;
+        rep.push_back(b);
+      }
+      pat[b] = it->second;
+    }
+    const int npat = (int)rep.size();
+    if (2 * npat <= nb) {
+      // keep the representative block of every pattern, in pattern order
+      auto shrink = [&](auto &v, size_t per) {
+        std::remove_reference_t<decltype(v)> w(npat * per);
+        for (int q = 0; q < npat; q++)
+          std::copy(v.begin() + (size_t)rep[q] * per, v.begin() + (size_t)(rep[q] + 1) * per, w.begin() + (size_t)q * per);
+        v.swap(w);
+      };
+      shrink(out.jpos, sw); shrink(out.lcol, sw); shrink(out.diag, S); shrink(out.nslot, S);
+      std::vector<int16_t> e16((size_t)npat * W * S);
+      for (int q = 0; q < npat; q++)
+        for (int k = 0; k < W; k++)
+          std::copy(out.ecol16.begin() + (size_t)k * NB + (size_t)rep[q] * S,
+                    out.ecol16.begin() + (size_t)k * NB + (size_t)(rep[q] + 1) * S, e16.begin() + ((size_t)q * W + k) * S);
+      out.ecol16.swap(e16);
+      out.pat.swap(pat);
+      out.npat = npat;
+    }
+  }
+  // What follows from the local columns, per pattern (per block where none are
+  // shared): factorization levels and lane tables, chains and sweep levels, the
+  // split L / U columns.
+  const int nt = out.npat ? out.npat : nb;
+  out.lrow.assign((size_t)nt * S, 0);
+  out.lptr.assign((size_t)nt * (S + 1), 0);
+  out.nlev.assign((size_t)nt, 0);
+  out.ftab.assign((size_t)nt * S * kFacLanes, uint4{0, 0, 0, 0});
+  out.swL.assign((size_t)nt * S, 0);
+  out.swU.assign((size_t)nt * S, 0);
+  out.nsw.assign((size_t)nt * 2, 0);
+  out.nlu.assign((size_t)nt, 0);
+  out.cL.assign((size_t)nt * kLU * S, (uint16_t)S);
+  out.cU.assign((size_t)nt * kLU * S, (uint16_t)S);
+  std::vector<int> chain(S), lev(S);
+  for (int b = 0; b < nt; b++) {
+    int m = 0;  // rows of the block
+    while (m < S && out.nslot[(size_t)b * S + m] > 0) m++;
+    const uint16_t *lc = &out.lcol[(size_t)b * kW * S];  // slot s of row i at s*S + i
+    const uint8_t *dg = &out.diag[(size_t)b * S], *nsl = &out.nslot[(size_t)b * S];
+    for (int i = 0; i < m; i++) {
+      if (dg[i] > kLU || nsl[i] - dg[i] - 1 > kLU) return "more than 13 lower or upper in-block entries in a row";
+      out.nlu[b] = std::max(out.nlu[b], std::max((int)dg[i], nsl[i] - dg[i] - 1));
+    }
+    // factorization levels, rows by level
+    int nlev = 0;
+    for (int i = 0; i < m; i++) {
+      lev[i] = 0;
+      for (int p = 0; p < dg[i]; p++) lev[i] = std::max(lev[i], lev[lc[(size_t)p * S + i]] + 1);
+      nlev = std::max(nlev, lev[i] + 1);
+    }
+    out.nlev[b] = nlev;
+    uint16_t *lp = &out.lptr[(size_t)b * (S + 1)];
+    for (int i = 0; i < m; i++) lp[lev[i] + 1]++;
+    for (int l = 0; l < nlev; l++) lp[l + 1] += lp[l];
+    {
+      std::vector<int> at(lp, lp + nlev);
+      for (int i = 0; i < m; i++) out.lrow[(size_t)b * S + at[lev[i]]++] = (uint16_t)i;
+    }
+    // lane tables: the slots of row k_p that hold this row's columns
+    for (int i = 0; i < m; i++) {
+      uint4 *row = &out.ftab[((size_t)b * S + i) * kFacLanes];
+      uint8_t idx[kFacLanes][16];
+      std::memset(idx, kNoSlot, sizeof(idx));
+      for (int p = 0; p < dg[i]; p++) {
+        const int k = lc[(size_t)p * S + i];
+        int d = p + 1;
+        for (int q = dg[k] + 1; q < nsl[k]; q++) {
+          const int cq = lc[(size_t)q * S + k];
+          while (d < nsl[i] && lc[(size_t)d * S + i] < cq) d++;
+          if (d < nsl[i] && lc[(size_t)d * S + i] == cq) idx[d][p] = (uint8_t)q;
+        }
+      }
+      for (int d = 0; d < kFacLanes; d++) {
+        const uint16_t c = d < nsl[i] ? lc[(size_t)d * S + i] : 0;
+        idx[d][13] = (uint8_t)(c & 0xff);
+        idx[d][14] = (uint8_t)(c >> 8);
+        idx[d][15] = dg[i];
+        std::memcpy(&row[d], idx[d], 16);
+      }
+    }
     // chains (see kChainMax): a row joins the run before it when its only lower
     // entry inside the run is the row before (the pattern is symmetric, so a
     // row's only upper entry inside is then the row after)
@@ -191,123 +306,13 @@ static std::string build_bj(const std::vector<int32_t> &jrp, const std::vector<i
     }
     out.nsw[2 * b] = fwd;
     out.nsw[2 * b + 1] = bwd;
-    // split L / U column tables (padding -> the zero entry S)
-    for (int i = 0; i < m; i++) {
-      const int di = out.diag[(size_t)b * S + i], ns = out.nslot[(size_t)b * S + i];
-      if (di > kLU || ns - di - 1 > kLU) return "more than 13 lower or upper in-block entries in a row";
-      out.nlu[b] = std::max(out.nlu[b], std::max(di, ns - di - 1));
-      // ILU(0) update pairs: row i slot d -= l_ik * row k slot s, for the entries of row k
-      // after its diagonal whose column is in row i's pattern
-      for (int p = 0; p < di; p++) {
-        const int k = out.lcol[(size_t)b * kW * S + (size_t)p * S + i];
-        const int dk = out.diag[(size_t)b * S + k], nk = out.nslot[(size_t)b * S + k];
-        int np = 0, pi = p + 1;
-        for (int q = dk + 1; q < nk; q++) {
-          const int cq = out.lcol[(size_t)b * kW * S + (size_t)q * S + k];
-          while (pi < ns && out.lcol[(size_t)b * kW * S + (size_t)pi * S + i] < cq) pi++;
-          if (pi < ns && out.lcol[(size_t)b * kW * S + (size_t)pi * S + i] == cq) {
-            if (np >= kLU) return "too many ILU(0) update pairs in a row";
-            out.pair[(size_t)b * kPair * S + (size_t)(p * kPairW + np / 2) * S + i] |=
-                (uint32_t)(pi | (q << 8)) << (16 * (np & 1));
-            np++;
-          }
-        }
-        out.npair[(size_t)b * kLU * S + (size_t)p * S + i] = (uint8_t)np;
-      }
+    // split L / U column tables, nearest column first (padding -> the zero entry S)
+    for (int i = 0; i < m; i++)
       for (int p = 0; p < kLU; p++) {
-        out.cL[(size_t)b * kLU * S + (size_t)p * S + i] =
-            p < di ? out.lcol[(size_t)b * kW * S + (size_t)(di - 1 - p) * S + i] : (uint16_t)S;
-        const int q = di + 1 + p;
-        out.cU[(size_t)b * kLU * S + (size_t)p * S + i] =
-            q < ns ? out.lcol[(size_t)b * kW * S + (size_t)q * S + i] : (uint16_t)S;
+        if (p < dg[i]) out.cL[((size_t)b * kLU + p) * S + i] = lc[(size_t)(dg[i] - 1 - p) * S + i];
+        const int q = dg[i] + 1 + p;
+        if (q < nsl[i]) out.cU[((size_t)b * kLU + p) * S + i] = lc[(size_t)q * S + i];
       }
-    }
-    for (int i = 0; i < m; i++) local[mem[i]] = -1;
-  }
-  // block-ordered ELL columns (padding slots point at the row itself with a 0 value)
-  out.perm.assign(nc, -1);
-  out.ecol.assign((size_t)W * NB, 0);
-  for (int64_t p = 0; p < NB; p++) {
-    const int r = out.row[p];
-    if (r < 0) continue;
-    out.perm[r] = (int32_t)p;
-    const int len = jrp[r + 1] - jrp[r];
-    for (int k = 0; k < W; k++) out.ecol[(size_t)k * NB + p] = k < len ? jcols[jrp[r] + k] : r;
-  }
-  for (int c = 0; c < nc; c++)
-    if (out.perm[c] < 0) return "cell missing from the block-Jacobi partition";
-  out.bw.assign(out.nblocks, 0);
-  for (int64_t p = 0; p < NB; p++) {
-    const int r = out.row[p];
-    if (r >= 0) out.bw[p / S] = std::max(out.bw[p / S], jrp[r + 1] - jrp[r]);
-  }
-  bool fits = true;
-  for (int64_t p = 0; p < NB && fits; p++) {
-    const int r = out.row[p];
-    for (int k = 0; k < W && fits; k++) {
-      const int64_t off = r < 0 ? 0 : (int64_t)out.ecol[(size_t)k * NB + p] - r;
-      fits = off >= INT16_MIN && off <= INT16_MAX;
-    }
-  }
-  if (fits) {
-    out.ecol16.resize(out.ecol.size());
-    for (int64_t p = 0; p < NB; p++) {
-      const int r = out.row[p];
-      for (int k = 0; k < W; k++)
-        out.ecol16[(size_t)k * NB + p] = r < 0 ? 0 : (int16_t)(out.ecol[(size_t)k * NB + p] - r);
-    }
-    out.ecol.clear();
-    // Blocks of a structured mesh repeat a few index patterns (an interior
-    // brick's in-block columns and column offsets are those of every other
-    // interior brick): keep one copy per pattern when that at least halves
-    // them, so the matvec streams values, not indices.
-    const size_t lu = (size_t)kLU * S, sw = (size_t)kW * S, pw = (size_t)kPair * S;
-    std::unordered_map<std::string, int> seen;
-    std::vector<int> rep;
-    std::vector<int32_t> pat(nb);
-    std::string key;
-    auto add = [&](const auto &v, size_t off, size_t n) {
-      key.append((const char *)(v.data() + off), n * sizeof(v[0]));
-    };
-    for (int b = 0; b < nb; b++) {
-      key.clear();
-      add(out.cL, b * lu, lu); add(out.cU, b * lu, lu);
-      add(out.jpos, b * sw, sw); add(out.lcol, b * sw, sw);
-      add(out.npair, b * lu, lu); add(out.pair, b * pw, pw);
-      add(out.diag, (size_t)b * S, S); add(out.nslot, (size_t)b * S, S);
-      add(out.levL, (size_t)b * S, S); add(out.swL, (size_t)b * S, S); add(out.swU, (size_t)b * S, S);
-      add(out.nlev, (size_t)b, 1); add(out.nsw, (size_t)2 * b, 2);
-      add(out.nlu, (size_t)b, 1);
-      for (int k = 0; k < W; k++) key.append((const char *)(out.ecol16.data() + (size_t)k * NB + (size_t)b * S), (size_t)S * 2);
-      auto it = seen.find(key);
-      if (it == seen.end()) {
-        it = seen.emplace(key, (int)rep.size()).first;
-        rep.push_back(b);
-      }
-      pat[b] = it->second;
-    }
-    const int npat = (int)rep.size();
-    if (2 * npat <= nb) {
-      // keep the representative block of every pattern, in pattern order
-      auto shrink = [&](auto &v, size_t per) {
-        std::remove_reference_t<decltype(v)> w(npat * per);
-        for (int q = 0; q < npat; q++)
-          std::copy(v.begin() + (size_t)rep[q] * per, v.begin() + (size_t)(rep[q] + 1) * per, w.begin() + (size_t)q * per);
-        v.swap(w);
-      };
-      shrink(out.cL, lu); shrink(out.cU, lu); shrink(out.jpos, sw); shrink(out.lcol, sw);
-      shrink(out.npair, lu); shrink(out.pair, pw); shrink(out.diag, S); shrink(out.nslot, S);
-      shrink(out.levL, S); shrink(out.swL, S); shrink(out.swU, S); shrink(out.nlev, 1); shrink(out.nsw, 2);
-      shrink(out.nlu, 1);
-      std::vector<int16_t> e16((size_t)npat * W * S);
-      for (int q = 0; q < npat; q++)
-        for (int k = 0; k < W; k++)
-          std::copy(out.ecol16.begin() + (size_t)k * NB + (size_t)rep[q] * S,
-                    out.ecol16.begin() + (size_t)k * NB + (size_t)(rep[q] + 1) * S, e16.begin() + ((size_t)q * W + k) * S);
-      out.ecol16.swap(e16);
-      out.pat.swap(pat);
-      out.npat = npat;
-    }
   }
   return std::string();
 }
@@ -677,11 +682,12 @@ static int ensure_ws(tdyhip_ctx *ctx, const tdyhip_solver_opts &o) {
     return rc;
   }
   ws.part_version = ctx->pc_part_version;
-  if ((rc = up(&ws.bj.d_row, hb.row)) || (rc = up(&ws.bj.d_jpos, hb.jpos)) || (rc = up(&ws.bj.d_lcol, hb.lcol)) ||
-      (rc = up(&ws.bj.d_diag, hb.diag)) || (rc = up(&ws.bj.d_nslot, hb.nslot)) || (rc = up(&ws.bj.d_levL, hb.levL)) ||
+  if ((rc = up(&ws.bj.d_row, hb.row)) || (rc = up(&ws.bj.d_jpos, hb.jpos)) || (rc = up(&ws.bj.d_lrow, hb.lrow)) ||
+      (rc = up(&ws.bj.d_lptr, hb.lptr)) || (rc = up(&ws.bj.d_ftab, hb.ftab)) ||
+      (rc = up(&ws.bj.d_diag, hb.diag)) || (rc = up(&ws.bj.d_nslot, hb.nslot)) ||
       (rc = up(&ws.bj.d_swL, hb.swL)) || (rc = up(&ws.bj.d_swU, hb.swU)) || (rc = up(&ws.bj.d_nlev, hb.nlev)) ||
       (rc = up(&ws.bj.d_nsw, hb.nsw)) || (rc = up(&ws.bj.d_cL, hb.cL)) ||
-      (rc = up(&ws.bj.d_cU, hb.cU)) || (rc = up(&ws.bj.d_npair, hb.npair)) || (rc = up(&ws.bj.d_pair, hb.pair)))
+      (rc = up(&ws.bj.d_cU, hb.cU)))
     return rc;
   for (double **p : {&ws.F, &ws.Y, &ws.W, &ws.G, &ws.JY, &ws.Udot, &ws.Uprev_ts, &ws.Usave})
     if ((rc = ws_alloc(ws, p, n))) return rc;
@@ -805,7 +811,7 @@ static double bytes_apply(const SolverWS &ws, size_t tv) {
 static double bytes_factor(const SolverWS &ws, size_t tv) {
   const double rows = (double)ws.bj.nblocks * ws.bj.bs;
   const double idx_rows = ws.bj.npat ? (double)ws.bj.npat * ws.bj.bs : rows;
-  return rows * (kW * 8 + (2 * kLU + 1) * tv) + idx_rows * (kW * (4 + 2) + kLU + kPair * 4 + 1 + 1 + 2);
+  return rows * (kW * 8 + (2 * kLU + 1) * tv) + idx_rows * (kW * 4 + kFacLanes * 16 + 1 + 1 + 4);
 }
 
 // ---------------------------------------------------------------- GMRES in launch pieces

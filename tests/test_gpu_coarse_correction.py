@@ -41,7 +41,7 @@ def _ilu0(A, part):
     return out
 
 
-def _iterations(A, F, part, rtol=1e-5, restart=30):
+def _iterations(A, F, part, rtol=1e-5, restart=30, coarse=True):
     import scipy.sparse as sp
     n, nb = A.shape[0], int(part.max()) + 1
     fac = _ilu0(A, part)
@@ -52,6 +52,8 @@ def _iterations(A, F, part, rtol=1e-5, restart=30):
         w = np.empty(n)
         for rows, L, U in fac:
             w[rows] = U @ (L @ r[rows])
+        if not coarse:
+            return w
         return w + R.T @ (A1 @ (R @ (r - A @ w)))
 
     x, its, tol = np.zeros(n), 0, None
@@ -123,3 +125,41 @@ def test_iterations_match_an_exact_coarse_solve(n, brick, block, fp32):
         assert abs(got - want) <= (2 if fp32 else 1)
     else:
         assert want - 2 <= got <= 1.25 * want + 2
+
+
+@pytest.mark.parametrize("n,brick", [
+    ((1, 9, 9), (1, 8, 8)),      # no row couples to the one before it alone
+    ((2, 9, 8), (2, 8, 8)),
+    ((3, 7, 9), (3, 7, 9)),
+    ((7, 10, 5), (7, 5, 5)),
+    ((16, 9, 6), (8, 8, 4)),     # chains of 8
+    ((9, 7, 6), (9, 7, 4)),      # lines of 9: a chain of 8 and one row
+    ((17, 5, 5), (17, 5, 3)),    # and cut again every 16 lanes
+    ((40, 4, 3), (40, 3, 2)),
+])
+@pytest.mark.parametrize("fp32", [0, 1])
+def test_one_level_iterations_match_plain_sweeps(n, brick, fp32):
+    """The triangular sweeps solve runs of rows at once: with blocks whose
+    lines have any length, GMRES with block ILU(0) alone takes the iterations
+    of plain forward and backward substitution."""
+    import torch
+    from pyoracle import Oracle
+    from tdycore_amd.mpfao import MPFAO
+    print(f"[case] one-level sweeps {n} brick={brick} fp32={fp32}", flush=True)
+    P = workloads.layered_box_problem(*n)
+    args = (P["mesh"], P["face_bc"], P["K"], P["porosity"], P["Sr"])
+    o = Oracle(*args, **P["kw"])
+    o.set_dtime(DAY)
+    o.snes_presolve(P["U0"])
+    F = o.snes_function(P["U0"])
+    A = o.jac_to_csr(o.snes_jacobian(P["U0"])).tocsr()
+    g = MPFAO(*args, **P["kw"])
+    part = mg.brick_partition(P["mesh"], *brick)
+    g.set_pc_partition(part)
+    U = torch.tensor(P["U0"], device="cuda", dtype=torch.float64)
+    g.SetDtime(DAY)
+    g.SNESPreSolve(U)
+    st = g.newton_snes(U, g.solver_options(snes_max_it=1, pc_block=256, krylov_fp32=fp32))
+    g.close()
+    want = _iterations(A, F, np.unique(part, return_inverse=True)[1].ravel(), coarse=False)
+    assert abs(st["linear_its"] - want) <= (2 if fp32 else 1)
