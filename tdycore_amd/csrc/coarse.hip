@@ -7,7 +7,7 @@
 // Galerkin operator A1 = P^T A P; the coarse solve Z ~ A1^-1 acts on what the
 // sweeps leave of r (the residual after block Jacobi, formed by the sweep
 // kernels themselves: CoarseRestrict in krylov.hip).  The blocks are
-// aggregated into at most kNG groups of at most kGMax; P2 is constant on a
+// aggregated into at most kNG (small meshes kNG / 2) groups of at most kGMax; P2 is constant on a
 // group's blocks, A2 = P2^T A1 P2 is inverted exactly as a dense matrix, and
 //
 //   Z r = P2 y + S (r - A1 P2 y),   y = A2^-1 P2^T r,
@@ -18,7 +18,7 @@
 // matrix alone is formed once per Newton step, per group: G1 (the own rows of
 // the overlapped inverse) and M = (P2 - G1 A1 P2) A2^-1, so an application is
 // z = [G1 M] [r of the overlap; P2^T r], one small dense product per group.
-// With a block per group (up to kNG blocks) the level-2 solve is A1^-1 itself
+// With a block per group (up to kNG / 2 blocks) the level-2 solve is A1^-1 itself
 // and G1 is left out.
 //
 // Against the additive form BJ^-1 r + P (G1 + P2 A2^-1 P2^T) P^T r without
