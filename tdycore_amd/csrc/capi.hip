@@ -612,6 +612,11 @@ static int setup_general(tdyhip_ctx *ctx, const tdyhip_mesh *m, const tdyhip_mat
     std::vector<GenGroup> gr;
     GenGroup cur{};
     int32_t od = 0;
+    size_t nrows = 0;
+    for (int v = 0; v < nv; v++) nrows += g->vdesc[(size_t)v * 8 + 7];
+    br.reserve(nrows);
+    bd.reserve(nrows);
+    gr.reserve(nrows / (kGrpRows / 4) + 1);
     for (int v = 0; v < nv; v++) {
       const int32_t *d = g->vdesc.data() + (size_t)v * 8;
       const int ncell = d[0], nface = d[1], ndir = d[3], of = d[5], nrow = d[7], nB = ncell + ndir;
