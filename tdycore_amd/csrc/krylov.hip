@@ -892,20 +892,49 @@ __device__ inline void load_pairs(const TV *__restrict__ V, int64_t ldv, int64_t
     if (j < cnt) f(j, q[j].x, q[j].y);
 }
 
+// The rows r and r + 1 of vectors V_j0 .. V_j0+cnt-1 (cnt <= NS, the same for
+// the whole workgroup): `load` issues every load before the first one is
+// waited for, which a loop over vectors of runtime count, or one whose loads
+// sit behind per-lane bounds checks, does not.  Rows past the end read the last
+// rows instead; the caller drops what becomes of them.
+template <class TV, int NS>
+struct VecRows {
+  using P = typename Pair2<TV>::T;
+  P q[NS];
+  __device__ inline void load(const TV *__restrict__ V, int64_t ldv, int64_t n, int64_t r, int j0, int cnt) {
+    const TV *p = V + (int64_t)j0 * ldv;
+    if (((ldv | n) & 1) == 0) {  // pairs aligned: one access each
+      p += min(r, n - 2);
+#pragma unroll
+      for (int j = 0; j < NS; j++)
+        if (j < cnt) q[j] = *reinterpret_cast<const P *>(p + (int64_t)j * ldv);
+    } else {
+      const int64_t ra = min(r, n - 1), rb = min(r + 1, n - 1);
+#pragma unroll
+      for (int j = 0; j < NS; j++)
+        if (j < cnt) {
+          q[j].x = p[(int64_t)j * ldv + ra];
+          q[j].y = p[(int64_t)j * ldv + rb];
+        }
+    }
+  }
+};
+
 // partial[j*nchunk + chunk] = <w, V_j> over the chunk, j = 0..nv-1.  Each
 // thread holds two adjacent rows and accumulates up to NS dots in registers;
 // one reduce-scatter per wavefront and one barrier per group of NS vectors
-// finish the chunk.  With pro.z1 set, w first receives the coarse
-// prolongation (written back).
+// finish the chunk.
+//
+// BATCH (FP64 on small grids, kBatchGrid): the NS vectors' loads in flight
+// together, in registers that cost a large grid its occupancy.
 //
 // COARSE: the launch's first cd.parts workgroups run the coarse solve; its
 // registers would set the occupancy of the row chunks at NS <= 16 (74), so
-// the budget is held to 7 waves per SIMD there.
-template <class TV, int NS, bool COARSE>
-__global__ void __launch_bounds__(kRedBlock) __attribute__((amdgpu_waves_per_eu(COARSE && NS <= 16 ? 7 : 1))) k_mdot(int64_t n, int nv, const TV *__restrict__ V, int64_t ldv,
-                                                    TV *__restrict__ w, TV *__restrict__ partial, int nchunk,
-                                                    Prolong pro, const int *__restrict__ stop = nullptr,
-                                                    CoarseDot cd = CoarseDot{}) {
+// the budget is held to 7 waves per SIMD there, except on small grids.
+template <class TV, int NS, bool COARSE, bool BATCH>
+__global__ void __launch_bounds__(kRedBlock) __attribute__((amdgpu_waves_per_eu(COARSE && NS <= 16 && !BATCH ? 7 : 1))) k_mdot(int64_t n, int nv, const TV *__restrict__ V, int64_t ldv,
+                                                    const TV *__restrict__ w, TV *__restrict__ partial, int nchunk,
+                                                    const int *__restrict__ stop, CoarseDot cd) {
   static_assert(Red<TV>::E == 2, "two rows per thread");
   __shared__ TV red[kRedBlock / 64][NS];
   if (stop && *stop) return;
@@ -919,21 +948,27 @@ __global__ void __launch_bounds__(kRedBlock) __attribute__((amdgpu_waves_per_eu(
   const int64_t r0 = (int64_t)chunk * Red<TV>::chunk + 2 * t;
   const bool vec = (ldv & 1) == 0;
   TV w0, w1;
-  load2(w, r0, n, true, w0, w1);
-  if (pro.z1) {
-    if (r0 < n) { w0 += (TV)pro.z1[pro.pos[r0] >> pro.bs_log2]; w[r0] = w0; }
-    if (r0 + 1 < n) { w1 += (TV)pro.z1[pro.pos[r0 + 1] >> pro.bs_log2]; w[r0 + 1] = w1; }
-  }
+  load2(w, r0, n, true, w0, w1);  // 0 past the end
   // FP32: every chunk but a ragged last one issues its NS loads together
-  // (8-byte accesses: 22.4 -> 19.4 us at 1M rows).  FP64 keeps one load at
-  // a time, which measured faster there (30.8 against 32.7 us): its 16-byte
-  // loads already keep enough bytes in flight at the higher occupancy.
+  // (8-byte accesses: 22.4 -> 19.4 us at 1M rows).  A large FP64 grid keeps one
+  // load at a time, which measured faster there (30.8 against 32.7 us): its
+  // 16-byte loads already keep enough bytes in flight at the higher occupancy.
   const bool full = sizeof(TV) == 4 && vec && (int64_t)(chunk + 1) * Red<TV>::chunk <= n;
   for (int j0 = 0; j0 < nv; j0 += NS) {
     TV acc[32];
 #pragma unroll
     for (int j = 0; j < 32; j++) acc[j] = 0;
-    if (full) {
+    if (BATCH) {
+      const int cnt = min(NS, nv - j0);
+      VecRows<TV, NS> v;
+      v.load(V, ldv, n, r0, j0, cnt);
+#pragma unroll
+      for (int j = 0; j < NS; j++)
+        if (j < cnt) {
+          acc[j] += w0 * v.q[j].x;
+          acc[j] += w1 * v.q[j].y;
+        }
+    } else if (full) {
       load_pairs<TV, NS>(V, ldv, r0, j0, min(NS, nv - j0), [&](int j, TV v0, TV v1) {
         acc[j] += w0 * v0;
         acc[j] += w1 * v1;
@@ -979,7 +1014,8 @@ __global__ void k_reduce_partials(int nv, int nchunk, const TV *__restrict__ par
 // adjacent rows per thread, as k_mdot).  DOTS: h itself is still the
 // multi-dot's npart partials per vector; every workgroup sums them, eight
 // lanes a vector in a fixed order, and workgroup 0 stores them for the
-// Arnoldi update, so no launch of its own stands between the two kernels.
+// Arnoldi update, so no launch of its own stands between the two kernels;
+// the vectors' rows are on their way while it does.
 constexpr int kMaxpyVecs = 200;  // basis vectors at most (the restart length)
 template <class TV, bool DOTS>
 __global__ void __launch_bounds__(kRedBlock) k_maxpy_norm(int64_t n, int nv, const TV *__restrict__ V, int64_t ldv,
@@ -992,10 +1028,12 @@ __global__ void __launch_bounds__(kRedBlock) k_maxpy_norm(int64_t n, int nv, con
   __shared__ double hs[DOTS ? kMaxpyVecs : 1];
   if (stop && *stop) return;
   const int64_t r0 = (int64_t)blockIdx.x * Red<TV>::chunk + 2 * threadIdx.x;
-  const bool vec = (ldv & 1) == 0;
   TV x0, x1;
   load2(w, r0, n, true, x0, x1);
-  if (pro.z1) {  // the coarse prolongation, when the multi-dot left it out
+  constexpr int NB = 32;
+  VecRows<TV, DOTS ? NB : 1> q;
+  if (DOTS) q.load(V, ldv, n, r0, 0, min(NB, nv));
+  if (pro.z1) {  // the coarse prolongation
     if (r0 < n) x0 += (TV)pro.z1[pro.pos[r0] >> pro.bs_log2];
     if (r0 + 1 < n) x1 += (TV)pro.z1[pro.pos[r0 + 1] >> pro.bs_log2];
   }
@@ -1005,11 +1043,11 @@ __global__ void __launch_bounds__(kRedBlock) k_maxpy_norm(int64_t n, int nv, con
       const TV *p = dots + (int64_t)v * npart;
       TV s = 0;
       for (int c = l; c < npart; c += 64) {
-        TV q[8];
+        TV d[8];
 #pragma unroll
-        for (int u = 0; u < 8; u++) q[u] = c + 8 * u < npart ? p[c + 8 * u] : (TV)0;
+        for (int u = 0; u < 8; u++) d[u] = c + 8 * u < npart ? p[c + 8 * u] : (TV)0;
 #pragma unroll
-        for (int u = 0; u < 8; u++) s += q[u];
+        for (int u = 0; u < 8; u++) s += d[u];
       }
       s += __shfl_xor(s, 1, 64);
       s += __shfl_xor(s, 2, 64);
@@ -1021,12 +1059,27 @@ __global__ void __launch_bounds__(kRedBlock) k_maxpy_norm(int64_t n, int nv, con
     }
     __syncthreads();
   }
-  for (int j = 0; j < nv; j++) {
-    TV v0, v1;
-    load2(V + (int64_t)j * ldv, r0, n, vec, v0, v1);
-    const TV hj = (TV)(DOTS ? hs[j] : h[j]);
-    x0 -= hj * v0;
-    x1 -= hj * v1;
+  if constexpr (DOTS) {
+    for (int j0 = 0; j0 < nv; j0 += NB) {
+      const int cnt = min(NB, nv - j0);
+      if (j0 > 0) q.load(V, ldv, n, r0, j0, cnt);
+#pragma unroll
+      for (int j = 0; j < NB; j++)
+        if (j < cnt) {
+          const TV hj = (TV)hs[j0 + j];
+          x0 -= hj * q.q[j].x;
+          x1 -= hj * q.q[j].y;
+        }
+    }
+  } else {
+    const bool vec = (ldv & 1) == 0;
+    for (int j = 0; j < nv; j++) {
+      TV v0, v1;
+      load2(V + (int64_t)j * ldv, r0, n, vec, v0, v1);
+      const TV hj = (TV)h[j];
+      x0 -= hj * v0;
+      x1 -= hj * v1;
+    }
   }
   TV s = 0;
   if (r0 + 1 < n) {

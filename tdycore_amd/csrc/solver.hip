@@ -1049,6 +1049,14 @@ constexpr int kFuseNormChunks = 512;
 // 100k prisms 29.3 -> 27.5; at 246 partials (63k cells) the two are even.
 constexpr int kFuseDots = 256;
 
+// Up to this many workgroups (one per CU) the FP64 multi-dot has all its loads
+// in flight together, as the update kernel has up to kFuseDots; beyond, the
+// registers cost as much as they gain (131k to 250k cells with the coarse
+// correction within 1%).  With both, a step of 46k cells, one level 15.30 ->
+// 14.70 ms, 110k 18.46 -> 17.60, 20k 8.57 -> 8.36, 63k with the correction 4.96 ->
+// 4.93, 100k prisms 28.91 -> 28.60.
+constexpr int kBatchGrid = 256;
+
 template <class TV>
 static void gmres_cycle(tdyhip_ctx *ctx, const tdyhip_solver_opts &o, const double *bvec, double *yvec,
                         hipStream_t st) {
@@ -1090,17 +1098,26 @@ static void gmres_cycle(tdyhip_ctx *ctx, const tdyhip_solver_opts &o, const doub
     // h = V^T o, o -= V h, ||o||^2, Givens update of column j.  (A single
     // kernel per reduction with a last-block hand-off is much slower here:
     // the device-scope fences it needs write back the per-XCD L2s.)
-    const Prolong none;
     const double bmd = (double)(j + 2) * N * sizeof(TV);
     // FP32: two passes of 16 beyond 16 vectors (67 VGPRs against 83 for one of 32)
-#define TDY_MDOT(NS)                                                                                                 \
+#define TDY_MDOT(NS, BATCH)                                                                                          \
   do {                                                                                                             \
-    if (cd.parts) KT(ctx, st, "k_mdot", bmd, k_mdot<TV, NS, true><<<gmd, kRedBlock, 0, st>>>(N, j + 1, k.V, N, ov, k.part, pst, none, stop, cd)); \
-    else KT(ctx, st, "k_mdot", bmd, k_mdot<TV, NS, false><<<gmd, kRedBlock, 0, st>>>(N, j + 1, k.V, N, ov, k.part, pst, none, stop, cd)); \
+    if (cd.parts) KT(ctx, st, "k_mdot", bmd, k_mdot<TV, NS, true, BATCH><<<gmd, kRedBlock, 0, st>>>(N, j + 1, k.V, N, ov, k.part, pst, stop, cd)); \
+    else KT(ctx, st, "k_mdot", bmd, k_mdot<TV, NS, false, BATCH><<<gmd, kRedBlock, 0, st>>>(N, j + 1, k.V, N, ov, k.part, pst, stop, cd)); \
   } while (0)
-    if (j < 8) TDY_MDOT(8);
-    else if (j < 16 || sizeof(TV) == 4) TDY_MDOT(16);
-    else TDY_MDOT(32);
+#define TDY_MDOT_NS(BATCH)                                \
+  do {                                                    \
+    if (j < 8) TDY_MDOT(8, BATCH);                        \
+    else if (j < 16 || sizeof(TV) == 4) TDY_MDOT(16, BATCH); \
+    else TDY_MDOT(32, BATCH);                             \
+  } while (0)
+    bool batch = false;
+    if constexpr (sizeof(TV) == 8) {
+      batch = pst <= kBatchGrid;
+      if (batch) TDY_MDOT_NS(true);
+    }
+    if (!batch) TDY_MDOT_NS(false);
+#undef TDY_MDOT_NS
 #undef TDY_MDOT
     const double bmx = (double)(j + 3) * N * sizeof(TV) + (pro.z1 ? (double)N * 4 : 0.0);
     if (pst <= kFuseDots) {

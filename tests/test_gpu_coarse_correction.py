@@ -165,3 +165,37 @@ def test_one_level_iterations_match_plain_sweeps(n, brick, fp32):
     g.close()
     want = _iterations(A, F, np.unique(part, return_inverse=True)[1].ravel(), coarse=False)
     assert abs(st["linear_its"] - want) <= (2 if fp32 else 1)
+
+
+@pytest.mark.parametrize("n", [
+    (33, 25, 9),    # an odd number of rows: no aligned pairs, a last chunk of 257
+    (33, 24, 8),    # even, a last chunk of 192
+    (16, 16, 8),    # whole chunks
+    (3, 3, 3),
+])
+@pytest.mark.parametrize("restart", [32, 40])
+def test_small_grid_iterations_match_plain_gmres(n, restart):
+    """On small grids the multi-dot and the update read up to 32 basis vectors
+    at once: odd, ragged and whole row chunks, and cycles longer than that."""
+    import torch
+    from pyoracle import Oracle
+    from tdycore_amd.mpfao import MPFAO
+    print(f"[case] small grid {n} restart={restart}", flush=True)
+    P = workloads.layered_box_problem(*n)
+    args = (P["mesh"], P["face_bc"], P["K"], P["porosity"], P["Sr"])
+    o = Oracle(*args, **P["kw"])
+    o.set_dtime(DAY)
+    o.snes_presolve(P["U0"])
+    F = o.snes_function(P["U0"])
+    A = o.jac_to_csr(o.snes_jacobian(P["U0"])).tocsr()
+    g = MPFAO(*args, **P["kw"])
+    part = mg.brick_partition(P["mesh"], 8, 8, 4)
+    g.set_pc_partition(part)
+    U = torch.tensor(P["U0"], device="cuda", dtype=torch.float64)
+    g.SetDtime(DAY)
+    g.SNESPreSolve(U)
+    st = g.newton_snes(U, g.solver_options(snes_max_it=1, pc_block=256, ksp_restart=restart, ksp_rtol=1e-8))
+    g.close()
+    want = _iterations(A, F, np.unique(part, return_inverse=True)[1].ravel(), rtol=1e-8, restart=restart, coarse=False)
+    print(f"  {st['linear_its']} iterations, plain {want}", flush=True)
+    assert abs(st["linear_its"] - want) <= 1  # rounding at the stop test
