@@ -100,7 +100,7 @@ struct GmresDev {
 // Bound by that chain: 34 levels of an 8x8x4 brick.  (Values updated in LDS by
 // lists of pairs, four lanes per row, waited for about eight LDS round trips
 // and a division per lower slot: 8x8x4 bricks, 1M cells 1825 -> 472 us, FP32 at
-// 442,368 cells 657 -> 150, 63k 214 -> 74; 4x4x4 bricks, 4k cells 91 -> 31.)
+// 442,368 cells 657 -> 150, 63k 215 -> 74; 4x4x4 bricks, 4k cells 85 -> 31.)
 constexpr int kFacPitch = kW + 2;  // a row's LDS pitch: its slots, the zero kNoSlot points at, odd
 template <int BS>
 struct FactorLanes {
@@ -425,7 +425,9 @@ __device__ inline void restrict_block2(const TV *x, double &rr, TV v, double *rv
 // LDS write: on grids too small to hide it, that chain is the kernel's time,
 // so the products go into four sums (levels of thirteen dependent
 // multiply-adds: 1M cells 106.7 -> 101.4 us; by chains of rows instead of rows
-// 101.4 -> 89.4, FP32 at 442,368 rows 31.6 -> 22.9, 46k rows 19.0 -> 15.5).
+// 101.4 -> 89.4, FP32 at 442,368 rows 31.6 -> 22.9, 46k rows 19.0 -> 15.5; means
+// over a solve's launches, those that return at once past its end among them.
+// The launches that work take 110 us at 1M rows, 4.5 TB/s).
 template <class TV>
 struct SweepRegs {  // a thread's row: factor entries and their local columns
   TV vl[kLU], vu[kLU], dinv;

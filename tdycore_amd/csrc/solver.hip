@@ -1013,7 +1013,7 @@ static void gmres_prep(tdyhip_ctx *ctx, const tdyhip_solver_opts &o, const doubl
     const hipStream_t cs = side ? ws.side : st;
     if (C.ng <= 64) KT(ctx, cs, "k_coarse_invert", (double)C.ng * C.ng * 16, k_coarse_invert<64><<<1, TiledGJ<64>::NT, 0, cs>>>(C));
     else KT(ctx, cs, "k_coarse_invert", (double)C.ng * C.ng * 16, k_coarse_invert<kNG><<<1, TiledGJ<kNG>::NT, 0, cs>>>(C));
-const double bfold = (double)C.ng * C.ng * C.gsz * 8;
+    const double bfold = (double)C.ng * C.ng * C.gsz * 8;
     if (C.gsz <= 4) KT(ctx, cs, "k_coarse_fold", bfold, k_coarse_fold<2, 32><<<C.ng, kFoldThreads, 0, cs>>>(C));
     else if (C.gsz <= 16) KT(ctx, cs, "k_coarse_fold", bfold, k_coarse_fold<8, 32><<<C.ng, kFoldThreads, 0, cs>>>(C));
     else KT(ctx, cs, "k_coarse_fold", bfold, k_coarse_fold<32, 16><<<C.ng, kFoldThreads, 0, cs>>>(C));
