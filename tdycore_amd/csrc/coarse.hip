@@ -7,8 +7,9 @@
 // Galerkin operator A1 = P^T A P; the coarse solve Z ~ A1^-1 acts on what the
 // sweeps leave of r (the residual after block Jacobi, formed by the sweep
 // kernels themselves: CoarseRestrict in krylov.hip).  The blocks are
-// aggregated into at most kNG (small meshes kNG / 2) groups of at most kGMax; P2 is constant on a
-// group's blocks, A2 = P2^T A1 P2 is inverted exactly as a dense matrix, and
+// aggregated into at most kNG (small meshes kNG / 2) groups of at most kGMax;
+// P2 is constant on a group's blocks, A2 = P2^T A1 P2 is inverted exactly as a
+// dense matrix, and
 //
 //   Z r = P2 y + S (r - A1 P2 y),   y = A2^-1 P2^T r,
 //

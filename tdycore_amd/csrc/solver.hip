@@ -1046,7 +1046,7 @@ constexpr int kFuseNormChunks = 512;
 // With up to this many partials per dot, the update kernel sums them itself
 // (every workgroup, up to restart x 256 values from L2), which takes less than
 // the launch it saves: 4k cells 4.05 -> 3.34 ms a step, 46k one-level 20.7 -> 20.1,
-// 100k prisms 29.3 -> 27.5; at 246 partials (63k cells) the two are even.
+// 100k prisms 29.3 -> 27.5; at 246 partials the two are even.
 constexpr int kFuseDots = 256;
 
 // Up to this many workgroups (one per CU) the FP64 multi-dot has all its loads
