@@ -141,11 +141,10 @@ static void iter_solve(BatchMember *m) {
   tdyhip_ctx *ctx = m->ctx;
   SolverWS &ws = *ctx->ws;
   hipStream_t st = ctx->stream;
-  tdyhip_solver_opts ok = m->o;
-  if (ok.krylov_fp32) ok.ksp_max_it = std::min(m->o.ksp_max_it, kFp32MaxIt);
+  const tdyhip_solver_opts &o = m->o;
   int its = 0;
-  const int rc = ok.krylov_fp32 ? gmres<float>(ctx, ok, ws.F, ws.Y, &its, st, true)
-                                : gmres<double>(ctx, ok, ws.F, ws.Y, &its, st, true);
+  const int rc = o.krylov_fp32 ? gmres<float>(ctx, o, ws.F, ws.Y, &its, st, true, kFp32MaxIt)
+                               : gmres<double>(ctx, o, ws.F, ws.Y, &its, st, true);
   if (rc && rc != TDYHIP_ERR_SINGULAR && rc != TDYHIP_ERR_NOCONV) { m->rc = rc; m->err = thread_error(); return; }
   newton_tail_pre(ctx, m->U, st);
   if (hipGetLastError() != hipSuccess) { m->rc = TDYHIP_ERR_HIP; m->err = "Newton tail launch failed"; }
@@ -246,7 +245,7 @@ static int begin_attempt(BatchMember *m) {
   }
   SCHK(hipMemcpyAsync(ws.Usave, m->U, sizeof(double) * ctx->nc, hipMemcpyDeviceToDevice, st));
   if ((rc = tdyhip_snes_presolve(ctx, m->U, st))) return rc;
-  k_set_dyn<<<1, 1, 0, st>>>(ws.dyn, ctx->dtime, 0.0);
+  set_dyn(ctx, 0.0, m->o, st);
   SCHK(hipGetLastError());
   return 0;
 }

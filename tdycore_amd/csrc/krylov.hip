@@ -1125,28 +1125,30 @@ __global__ void k_convert(int64_t n, const TA *__restrict__ a, TB *__restrict__ 
   if (i < n) b[i] = (TB)a[i];
 }
 
-__global__ void k_gmres_init(GmresDev *gd, int *status, int maxit) {
+// dyn: the solver's device-resident parameters (SolverWS::dyn); cap: iterations
+// this attempt gets at most.
+__global__ void k_gmres_init(GmresDev *gd, int *status, const double *__restrict__ dyn, int cap) {
   gd->its = 0;
   gd->done = 0;
   gd->converged = 0;
   gd->finished = 0;
   gd->diverged = 0;
   gd->jcur = 0;
-  gd->maxit = maxit;
+  gd->maxit = min((int)dyn[4], cap);
   *status = 0;
 }
 
 // Start of a cycle: beta = sqrt(h[0]) from a norm reduction; sets tol on the first cycle.
 // After the solve has finished, a later cycle is empty: no columns, stop flag set.
-__global__ void k_cycle_start(GmresDev *gd, const double *__restrict__ h, double *__restrict__ g, int m, double rtol,
-                              double atol, int first) {
+__global__ void k_cycle_start(GmresDev *gd, const double *__restrict__ h, double *__restrict__ g, int m,
+                              const double *__restrict__ dyn, int first) {
   if (!first && gd->finished) {
     gd->jcur = 0;
     gd->done = 1;
     return;
   }
   const double beta = sqrt(h[0]);
-  if (first) gd->tol = fmax(rtol * beta, atol);
+  if (first) gd->tol = fmax(dyn[2] * beta, dyn[3]);
   for (int i = 0; i <= m; i++) g[i] = 0.0;
   g[0] = beta;
   gd->resid = beta;

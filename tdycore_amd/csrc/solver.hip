@@ -570,13 +570,17 @@ struct SolverWS {
   struct NewtonGraph {
     const double *X;
     int type, fp32, cycles;
+    const double *src;  // the residual's source term, or nullptr
     hipGraphExec_t exec;
   };
   std::vector<NewtonGraph> newton_graphs;
   int cycles_hint = 1;            // restart cycles the last Newton iteration's solve needed
   struct NewtonDev *nd = nullptr; // the Newton iteration's outcome on the device
   double *nh = nullptr;           // 4 norms / dots of the Newton tail
-  double *dyn = nullptr;          // dtime, shift (1 / dt of the TS form) read by the solver's launches
+  // what may change between solves, read by the solver's launches (a captured
+  // graph follows them): dtime, shift (1 / dt of the TS form), ksp_rtol,
+  // ksp_atol, ksp_max_it
+  double *dyn = nullptr;
 };
 
 constexpr int kMaxGraphCycles = 8;    // restart cycles inside one Newton-iteration graph
@@ -714,7 +718,7 @@ static int ensure_ws(tdyhip_ctx *ctx, const tdyhip_solver_opts &o) {
   if ((rc = ws_alloc(ws, &ws.status, 1))) return rc;
   if ((rc = ws_alloc(ws, (char **)&ws.nd, 256))) return rc;  // a NewtonDev (defined with the solver below)
   if ((rc = ws_alloc(ws, &ws.nh, 4))) return rc;
-  if ((rc = ws_alloc(ws, &ws.dyn, 2))) return rc;
+  if ((rc = ws_alloc(ws, &ws.dyn, 5))) return rc;
   ws.coarse_req = o.pc_coarse ? 1 : 0;
   if (o.pc_coarse) {
     HostCoarse hc;
@@ -973,14 +977,14 @@ static void norm2_to_h0(tdyhip_ctx *ctx, const TV *v, const int *stp, hipStream_
 
 template <class TV>
 static void gmres_prep(tdyhip_ctx *ctx, const tdyhip_solver_opts &o, const double *bvec, double *yvec,
-                       hipStream_t st) {
+                       hipStream_t st, int cap = INT32_MAX) {
   SolverWS &ws = *ctx->ws;
   const KBufs<TV> k = kbufs<TV>(ctx, o.ksp_restart);
   const unsigned g256 = (unsigned)((k.N + 255) / 256);
   if (!std::is_same<TV, double>::value)
     KT(ctx, st, "k_convert_J", (double)ws.nnz * (8 + sizeof(TV)),
        k_convert<double, TV><<<(unsigned)((ws.nnz + 255) / 256), 256, 0, st>>>(ws.nnz, ws.J, k.Jk));
-  k_gmres_init<<<1, 1, 0, st>>>(k.gd, ws.status, o.ksp_max_it);
+  k_gmres_init<<<1, 1, 0, st>>>(k.gd, ws.status, ws.dyn, cap);
   // coarse correction: column sums and Galerkin rows, the groups' overlapped
   // inverses, the level-2 inverse and its product with them for this
   // Jacobian.  The column sums and group inverses run first (the factor's
@@ -1034,7 +1038,7 @@ static void gmres_prep(tdyhip_ctx *ctx, const tdyhip_solver_opts &o, const doubl
   }
   pc_apply<TV>(ctx, k, k.b, k.w, nullptr, st);  // r0 = M^-1 b  (y0 = 0)
   norm2_to_h0<TV>(ctx, k.w, nullptr, st);
-  k_cycle_start<<<1, 1, 0, st>>>(k.gd, ws.h, k.dg, k.m, o.ksp_rtol, o.ksp_atol, 1);
+  k_cycle_start<<<1, 1, 0, st>>>(k.gd, ws.h, k.dg, k.m, ws.dyn, 1);
 }
 
 // On meshes of up to this many reduction chunks, step j > 0 finishes column
@@ -1142,7 +1146,7 @@ static void gmres_cycle(tdyhip_ctx *ctx, const tdyhip_solver_opts &o, const doub
   resid_pc_apply<TV>(ctx, k, bvec, yvec, k.w, fin, st);
   norm2_to_h0<TV>(ctx, k.w, fin, st);
   ctx->kt.tag = -1;
-  k_cycle_start<<<1, 1, 0, st>>>(gd, ws.h, k.dg, m, o.ksp_rtol, o.ksp_atol, 0);
+  k_cycle_start<<<1, 1, 0, st>>>(gd, ws.h, k.dg, m, ws.dyn, 0);
 }
 
 // The one-cycle graph of precision TV (captured on first use, replayed by
@@ -1166,9 +1170,9 @@ static hipGraphExec_t cycle_graph(tdyhip_ctx *ctx, const tdyhip_solver_opts &o, 
 // each, until the solve has finished.
 template <class TV>
 static int gmres(tdyhip_ctx *ctx, const tdyhip_solver_opts &o, const double *bvec, double *yvec, int *its_out,
-                 hipStream_t st, bool allow_graph) {
+                 hipStream_t st, bool allow_graph, int cap = INT32_MAX) {
   SolverWS &ws = *ctx->ws;
-  gmres_prep<TV>(ctx, o, bvec, yvec, st);
+  gmres_prep<TV>(ctx, o, bvec, yvec, st, cap);
   SCHK(hipGetLastError());
   const bool graph = allow_graph && o.hip_graphs && !ctx->kt.on && bvec == ws.F && yvec == ws.Y;
   hipGraphExec_t cyc = graph ? cycle_graph<TV>(ctx, o, st) : nullptr;
@@ -1333,9 +1337,16 @@ __global__ void k_nt_final(NewtonDev *nd, const double *__restrict__ h, const Gm
 
 __global__ void k_nt_set_fnorm(NewtonDev *nd, const double *__restrict__ h) { nd->fnorm = sqrt(h[0]); }
 __global__ void k_set_scalar(double *p, double v) { *p = v; }
-__global__ void k_set_dyn(double *dyn, double d0, double d1) {
-  dyn[0] = d0;
-  dyn[1] = d1;
+// The solver's device-resident parameters (SolverWS::dyn) for the solve that follows.
+__global__ void k_set_dyn(double *dyn, double dtime, double shift, double rtol, double atol, double max_it) {
+  dyn[0] = dtime;
+  dyn[1] = shift;
+  dyn[2] = rtol;
+  dyn[3] = atol;
+  dyn[4] = max_it;
+}
+static void set_dyn(tdyhip_ctx *ctx, double shift, const tdyhip_solver_opts &o, hipStream_t st) {
+  k_set_dyn<<<1, 1, 0, st>>>(ctx->ws->dyn, ctx->dtime, shift, o.ksp_rtol, o.ksp_atol, o.ksp_max_it);
 }
 
 // nh[slot] = <x, y> (skipped with the stop flag)
@@ -1386,32 +1397,42 @@ static int newton_tail(tdyhip_ctx *ctx, const Form &fm, double *X, hipStream_t s
   return hipGetLastError() == hipSuccess ? 0 : TDYHIP_ERR_HIP;
 }
 
+// FP32 Krylov: the FP32 attempt gets at most kFp32MaxIt iterations; if it
+// does not converge (or its ILU(0) meets a zero pivot), the same Newton
+// correction is solved again in FP64 from scratch.
+constexpr int kFp32MaxIt = 1000;
+
 // The whole Newton iteration as one launch sequence: Jacobian, preparation,
 // `cycles` restart cycles (those past the end of the solve return at once)
 // and the tail.
-static int newton_iter_launch(tdyhip_ctx *ctx, const Form &fm, double *X, const tdyhip_solver_opts &ok, int fp32,
+static int newton_iter_launch(tdyhip_ctx *ctx, const Form &fm, double *X, const tdyhip_solver_opts &o, int fp32,
                               int cycles, hipStream_t st) {
   SolverWS &ws = *ctx->ws;
   int rc = eval_J(ctx, fm, X, ws.J, st);
   if (rc) return rc;
   if (fp32) {
-    gmres_prep<float>(ctx, ok, ws.F, ws.Y, st);
-    for (int c = 0; c < cycles; c++) gmres_cycle<float>(ctx, ok, ws.F, ws.Y, st);
+    gmres_prep<float>(ctx, o, ws.F, ws.Y, st, kFp32MaxIt);
+    for (int c = 0; c < cycles; c++) gmres_cycle<float>(ctx, o, ws.F, ws.Y, st);
   } else {
-    gmres_prep<double>(ctx, ok, ws.F, ws.Y, st);
-    for (int c = 0; c < cycles; c++) gmres_cycle<double>(ctx, ok, ws.F, ws.Y, st);
+    gmres_prep<double>(ctx, o, ws.F, ws.Y, st);
+    for (int c = 0; c < cycles; c++) gmres_cycle<double>(ctx, o, ws.F, ws.Y, st);
   }
   return newton_tail(ctx, fm, X, st);
 }
 
-// Captured graphs keyed by the iterate's pointer, the form, the Krylov
-// precision and the cycle count (cycles = 0: the tail alone).
-static hipGraphExec_t newton_graph(tdyhip_ctx *ctx, const Form &fm, double *X, const tdyhip_solver_opts &ok,
+// Captured graphs keyed by what their launches hold as arguments and a later
+// solve may change: the iterate's pointer, the form, the Krylov precision, the
+// cycle count (cycles = 0: the tail alone) and the source term.  The time step
+// and the Krylov tolerances are read from ws.dyn; a new restart length, block
+// size, partition or coarse setting makes a new workspace.
+static hipGraphExec_t newton_graph(tdyhip_ctx *ctx, const Form &fm, double *X, const tdyhip_solver_opts &o,
                                    int fp32, int cycles, bool tail_only, hipStream_t st) {
   SolverWS &ws = *ctx->ws;
   const int key_c = tail_only ? 0 : cycles;
+  const double *src = ctx->has_source ? ctx->d_source : nullptr;
   for (auto &e : ws.newton_graphs)
-    if (e.X == X && e.type == fm.type && e.fp32 == fp32 && e.cycles == key_c) return e.exec;
+    if (e.X == X && e.type == fm.type && e.fp32 == fp32 && e.cycles == key_c && e.src == src)
+      return e.exec;
   if (ws.newton_graphs.size() >= kMaxNewtonGraphs) {
     (void)hipStreamSynchronize(st);  // the oldest graph may still be in flight
     (void)hipGraphExecDestroy(ws.newton_graphs.front().exec);
@@ -1419,7 +1440,7 @@ static hipGraphExec_t newton_graph(tdyhip_ctx *ctx, const Form &fm, double *X, c
   }
   hipGraph_t gr = nullptr;
   if (hipStreamBeginCapture(st, hipStreamCaptureModeRelaxed) != hipSuccess) return nullptr;
-  const int rc = tail_only ? newton_tail(ctx, fm, X, st) : newton_iter_launch(ctx, fm, X, ok, fp32, cycles, st);
+  const int rc = tail_only ? newton_tail(ctx, fm, X, st) : newton_iter_launch(ctx, fm, X, o, fp32, cycles, st);
   const hipError_t ec = hipStreamEndCapture(st, &gr);
   if (rc || ec != hipSuccess) {
     if (gr) (void)hipGraphDestroy(gr);
@@ -1428,7 +1449,7 @@ static hipGraphExec_t newton_graph(tdyhip_ctx *ctx, const Form &fm, double *X, c
   hipGraphExec_t ex = nullptr;
   if (hipGraphInstantiate(&ex, gr, nullptr, nullptr, 0) != hipSuccess) ex = nullptr;
   (void)hipGraphDestroy(gr);
-  if (ex) ws.newton_graphs.push_back({X, fm.type, fp32, key_c, ex});
+  if (ex) ws.newton_graphs.push_back({X, fm.type, fp32, key_c, src, ex});
   return ex;
 }
 
@@ -1438,11 +1459,6 @@ static int read_newton(tdyhip_ctx *ctx, NewtonDev &h, hipStream_t st) {
   return 0;
 }
 
-// FP32 Krylov: the FP32 attempt gets at most kFp32MaxIt iterations; if it
-// does not converge (or its ILU(0) meets a zero pivot), the same Newton
-// correction is solved again in FP64 from scratch.
-constexpr int kFp32MaxIt = 1000;
-
 // One Newton iteration up to and including the full step's test: on return h
 // holds the linear solve's outcome, the step length and, when the solve
 // converged, the residual norm at the full step and whether it was taken.
@@ -1450,8 +1466,6 @@ static int newton_iteration(tdyhip_ctx *ctx, const Form &fm, double *X, const td
                             tdyhip_solver_stats &stats, hipStream_t st, NewtonDev &h) {
   SolverWS &ws = *ctx->ws;
   const int fp32 = o.krylov_fp32 ? 1 : 0;
-  tdyhip_solver_opts ok = o;
-  if (fp32) ok.ksp_max_it = std::min(o.ksp_max_it, kFp32MaxIt);
   // (a context on an evaluation fuser has its evaluations launched by the
   // fuser's thread, outside any graph of its own)
   const bool graphs = o.hip_graphs && !ctx->kt.on && !ctx->fuser;
@@ -1461,12 +1475,12 @@ static int newton_iteration(tdyhip_ctx *ctx, const Form &fm, double *X, const td
     // tail in one replay; a solve that needs more cycles continues one cycle
     // graph at a time, then replays the tail alone.
     const int C = std::max(1, std::min(ws.cycles_hint, kMaxGraphCycles));
-    hipGraphExec_t ex = newton_graph(ctx, fm, X, ok, fp32, C, false, st);
+    hipGraphExec_t ex = newton_graph(ctx, fm, X, o, fp32, C, false, st);
     if (!ex) { set_error("Newton iteration graph capture failed"); return TDYHIP_ERR_HIP; }
     SCHK(hipGraphLaunch(ex, st));
     if ((rc = read_newton(ctx, h, st))) return rc;
     if (!h.finished && !h.pc_status) {
-      hipGraphExec_t cyc = fp32 ? cycle_graph<float>(ctx, ok, st) : cycle_graph<double>(ctx, ok, st);
+      hipGraphExec_t cyc = fp32 ? cycle_graph<float>(ctx, o, st) : cycle_graph<double>(ctx, o, st);
       if (!cyc) { set_error("GMRES cycle graph capture failed"); return TDYHIP_ERR_HIP; }
       GmresDev hg;
       do {
@@ -1475,7 +1489,7 @@ static int newton_iteration(tdyhip_ctx *ctx, const Form &fm, double *X, const td
         SCHK(hipMemcpyAsync(&hg, ws.gdev, sizeof(GmresDev), hipMemcpyDeviceToHost, st));
         SCHK(hipStreamSynchronize(st));
       } while (!hg.finished);
-      hipGraphExec_t tail = newton_graph(ctx, fm, X, ok, fp32, 0, true, st);
+      hipGraphExec_t tail = newton_graph(ctx, fm, X, o, fp32, 0, true, st);
       if (!tail) { set_error("Newton tail graph capture failed"); return TDYHIP_ERR_HIP; }
       SCHK(hipGraphLaunch(tail, st));
       if ((rc = read_newton(ctx, h, st))) return rc;
@@ -1483,7 +1497,8 @@ static int newton_iteration(tdyhip_ctx *ctx, const Form &fm, double *X, const td
   } else {
     if ((rc = eval_J(ctx, fm, X, ws.J, st))) return rc;
     int its = 0;
-    rc = fp32 ? gmres<float>(ctx, ok, ws.F, ws.Y, &its, st, false) : gmres<double>(ctx, ok, ws.F, ws.Y, &its, st, false);
+    rc = fp32 ? gmres<float>(ctx, o, ws.F, ws.Y, &its, st, false, kFp32MaxIt)
+              : gmres<double>(ctx, o, ws.F, ws.Y, &its, st, false);
     if (rc && rc != TDYHIP_ERR_SINGULAR && rc != TDYHIP_ERR_NOCONV) return rc;
     if ((rc = newton_tail(ctx, fm, X, st)) || (rc = read_newton(ctx, h, st))) return rc;
   }
@@ -1522,7 +1537,7 @@ static int newton(tdyhip_ctx *ctx, const Form &fm, double *X, const tdyhip_solve
   const unsigned g = nblk(n, 256);
   const double minlambda = 1e-12, divtol = 1e4;
   int rc;
-  k_set_dyn<<<1, 1, 0, st>>>(ws.dyn, ctx->dtime, fm.type == 0 ? 1.0 / fm.dt : 0.0);
+  set_dyn(ctx, fm.type == 0 ? 1.0 / fm.dt : 0.0, o, st);
   if ((rc = eval_F(ctx, fm, X, ws.F, st))) return rc;
   dot_to(ctx, ws.F, ws.F, 0, nullptr, st);
   k_nt_set_fnorm<<<1, 1, 0, st>>>(ws.nd, ws.nh);
