@@ -112,7 +112,8 @@ def load():
         "tdyhip_batch_size": [P, P], "tdyhip_batch_round": [P, C.c_int32, P, P, P, P],
         "tdyhip_fuser_create": [P], "tdyhip_fuser_destroy": [P], "tdyhip_set_fuser": [P, P],
         "tdyhip_fuser_stats": [P, P], "tdyhip_fuser_set_window": [P, C.c_int32],
-        # test hook (exported, not declared in the header)
+        # test hooks (exported, not declared in the header)
+        "tdyhip_test_coarse_layout": [P, P, C.c_int32, C.c_int32, P, P, P, P, P],
         "tdyhip_test_dense_inverse": [P, C.c_int32, C.c_int32, P],
     }
     for name, args in sig.items():

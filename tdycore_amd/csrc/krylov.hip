@@ -262,6 +262,10 @@ __device__ inline TV block_sum_n(TV v, TV *sh) {
 // teams of 8 lanes (kCoarsePad).
 constexpr int kCQ = 32;  // neighbour blocks of a block (itself included)
 constexpr uint16_t kCoarsePad = 0xffff;
+// Teams a block's lists may hold: rows of 27 entries in 27 lists, each list's
+// last team short.  (Rows of up to 32 entries, scattered over a block's 32
+// neighbours, could need more: the set-up counts them, build_coarse.)
+constexpr int coarse_teams(int bs) { return bs * 27 / 8 + kCQ; }
 struct CoarseRestrict {
   const double *cown = nullptr;    // nblocks*bs: the own block's column sums
   const int32_t *eptr = nullptr;   // nblocks+1: first list entry of each block (multiples of 8)
@@ -282,8 +286,7 @@ struct CoarseRestrict {
 // barrier inside.
 template <int BS, class F>
 __device__ inline double coarse_block_sums(int ne, int i0, int i1, bool ownq, int t, double own, F &&value) {
-  constexpr int kTeams = BS * 27 / 8 + kCQ;  // every row in 27 lists, each list's last team short
-  __shared__ double tm[kTeams];
+  __shared__ double tm[coarse_teams(BS)];
   __shared__ double ow[BS / 64];
   for (int off = 32; off > 0; off >>= 1) own += __shfl_down(own, off, 64);
   if ((t & 63) == 0) ow[t >> 6] = own;

@@ -336,6 +336,7 @@ struct HostCoarse {
 static std::string build_coarse(const HostBJ &hb, const std::vector<int32_t> &jrp, const std::vector<int32_t> &jcols,
                                 int nc, int W, HostCoarse &out) {
   const int S = hb.bs, nb = hb.nblocks;
+  if (W > 32) return "a row has more than 32 entries";
   const int64_t NB = (int64_t)nb * S;
   std::vector<int32_t> blk(nc);
   for (int c = 0; c < nc; c++) blk[c] = hb.perm[c] / S;
@@ -388,6 +389,7 @@ static std::string build_coarse(const HostBJ &hb, const std::vector<int32_t> &jr
       team += (cnt[q] + 7) / 8;
     }
     out.tq[(size_t)b * (kCQ + 1) + kCQ] = (uint16_t)team;
+    if (team > coarse_teams(S)) return "a block's rows reach too many neighbour blocks";
     out.cent.resize(e0 + (size_t)8 * team, kCoarsePad);
     for (int i = 0; i < S; i++)
       for (uint32_t w = rowmask[i]; w; w &= w - 1) {
@@ -722,8 +724,7 @@ static int ensure_ws(tdyhip_ctx *ctx, const tdyhip_solver_opts &o) {
   ws.coarse_req = o.pc_coarse ? 1 : 0;
   if (o.pc_coarse) {
     HostCoarse hc;
-    // (the Galerkin row kernel handles up to 32 slots per row)
-    if (ctx->jell_w <= 32 && build_coarse(hb, ctx->h_jrp, ctx->h_jcols, ctx->nc, ctx->jell_w, hc).empty()) {
+    if (build_coarse(hb, ctx->h_jrp, ctx->h_jcols, ctx->nc, ctx->jell_w, hc).empty()) {
       CoarseLayout &C = ws.cl;
       CoarseRestrict &R = C.R;
       C.nb = hc.nb; C.ng = hc.ng; C.gsz = hc.gsz; C.nov = hc.nov;
@@ -1766,6 +1767,36 @@ int tdyhip_run_tdyti(tdyhip_ctx *ctx, double *U, double dt_init, double growth, 
     if (dt > dt_max) dt = dt_max;
   }
   SCHK(hipStreamSynchronize(ctx->stream));
+  return 0;
+}
+
+// Test hook, not part of the interface in include/tdyhip.h, host only: the
+// blocks of a row pattern (part: block of each row, or NULL for the breadth-first
+// default) and the structure the coarse correction builds on them.  sizes: blocks,
+// groups, blocks of a group and of a group with overlap (at most), LDS
+// teams of a block (at most).  blk[nc]: block of each row; grp[nc]: group of each
+// block; gov[nc*128]: blocks of each group, then its overlap (-1 pad, as many
+// per group as sizes[3]; only with groups of several blocks).  TDYHIP_ERR_ARG
+// where the correction would not be used.
+int tdyhip_test_coarse_layout(const int32_t *jrp, const int32_t *jcols, int32_t nc, int32_t pc_block,
+                              const int32_t *part, int32_t *sizes, int32_t *blk, int32_t *grp, int32_t *gov) {
+  using namespace tdyhip;
+  if (!jrp || !jcols || nc < 1 || !sizes || !blk || !grp || !gov) { set_error("bad argument"); return TDYHIP_ERR_ARG; }
+  const std::vector<int32_t> rp(jrp, jrp + nc + 1), cols(jcols, jcols + jrp[nc]);
+  std::vector<int32_t> pv;
+  if (part) pv.assign(part, part + nc);
+  int W = 0;
+  for (int c = 0; c < nc; c++) W = std::max(W, rp[c + 1] - rp[c]);
+  HostBJ hb;
+  HostCoarse hc;
+  std::string msg = build_bj(rp, cols, nc, W, pc_block, pv, hb);
+  if (msg.empty()) msg = build_coarse(hb, rp, cols, nc, W, hc);
+  if (!msg.empty()) { set_error(msg); return TDYHIP_ERR_ARG; }
+  sizes[0] = hc.nb; sizes[1] = hc.ng; sizes[2] = hc.gsz; sizes[3] = hc.nov; sizes[4] = 0;
+  for (int b = 0; b < hc.nb; b++) sizes[4] = std::max(sizes[4], (int)hc.tq[(size_t)b * (kCQ + 1) + kCQ]);
+  for (int c = 0; c < nc; c++) blk[c] = hb.perm[c] / hb.bs;
+  std::copy(hc.grp.begin(), hc.grp.end(), grp);
+  std::copy(hc.gov.begin(), hc.gov.end(), gov);
   return 0;
 }
 
