@@ -472,6 +472,7 @@ __global__ void __launch_bounds__(kGenJBlock) k_gather_general_J(GenGatherArgs a
   if (c >= a.nc) return;  // uniform over the cell's lanes (the wavefront's other cells are independent)
   const int r0 = a.jrp[c], len = a.jrp[c + 1] - r0;
   for (int k = l; k < len; k += kGenJLanes) acc[g][k] = 0.0;
+  wave_lds_fence();
   // rows l and l + 16: T at T[to ..], the columns' slots, the signed factor,
   // and the sums of the sides' terms (this cell's, the other cell's)
   int to[2], ns[2];  // ns: columns | side << 8
@@ -539,7 +540,7 @@ __global__ void __launch_bounds__(kGenJBlock) k_gather_general_J(GenGatherArgs a
                                      : a.dM[c] * a.vol[c] * (1.0 / dtime);
     atomicAdd(&acc[g][a.jdiag[c]], self + dvc);
   }
-  __builtin_amdgcn_wave_barrier();
+  wave_lds_fence();
   int64_t st = 1;
   double *row = a.J + r0;
   if (a.perm) {
@@ -759,20 +760,25 @@ __device__ inline void cell_jac_block(const RowArgs &ra, const GatherArgs &a, co
       if (((code >> (18 + m)) & 1 ? dn[m] : up[m]) >= 0) atomicAdd(&sd[(code >> (21 + 3 * m)) & 7][t], other[m]);
     sw[t] = w;
   }
-  // A cell's eight lanes share a wavefront, whose LDS operations run in
-  // program order: no barrier from here on.
-  __builtin_amdgcn_wave_barrier();
+  // a cell's eight lanes share a wavefront: no barrier from here on
+  wave_lds_fence();
   if (c < 0) return;
   // corner by corner, lane k adds column k's sum into its slot: a region's
   // cells are distinct, so a corner's 8 slots are (apart from kJacSlots,
   // which is never read), and every slot is summed in corner order
   const int base8 = t - corner;
+  unsigned sl[8];
+  double v[8];
 #pragma unroll
   for (int j = 0; j < 8; j++) {
     const unsigned b = (unsigned)(sw[base8 + j] >> (8 * corner)) & 0xffu;
-    const unsigned sl = b == 0xffu ? kJacSlots : b;
-    acc[sl][cl] += sd[corner][base8 + j];
-    __builtin_amdgcn_wave_barrier();
+    sl[j] = b == 0xffu ? kJacSlots : b;
+    v[j] = sd[corner][base8 + j];
+  }
+#pragma unroll
+  for (int j = 0; j < 8; j++) {
+    acc[sl[j]][cl] += v[j];
+    wave_lds_fence();
   }
   if (corner == 0) acc[dslot][cl] += dv;
   if (WITH_R) {
@@ -789,7 +795,7 @@ __device__ inline void cell_jac_block(const RowArgs &ra, const GatherArgs &a, co
     for (int lf = 0; lf < 6; lf++) s += __shfl(fs, (base8 & 63) + lf, 64);
     if (corner == 0) a.R[c] = cell_residual(a, c, s);
   }
-  __builtin_amdgcn_wave_barrier();
+  wave_lds_fence();
   int64_t base = c, stride = 1;
   jac_row_addr(a, c, base, stride);
   const int len = a.jrp ? a.jrp[c + 1] - a.jrp[c] : a.ell_w;

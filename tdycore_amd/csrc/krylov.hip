@@ -366,7 +366,7 @@ __device__ inline void coarse_scatter(const CoarseRestrict &R, const CoarseRegs<
     if (c.dst >= 0) R.rcs[c.dst] = v;
     qv[t] = v;
     qg[t] = (uint8_t)c.grp;
-    __builtin_amdgcn_wave_barrier();  // one wavefront: its LDS operations run in program order
+    wave_lds_fence();  // one wavefront
     if (c.dst2 >= 0) {
       double g = 0.0;
 #pragma unroll

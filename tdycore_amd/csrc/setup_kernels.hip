@@ -243,10 +243,7 @@ __global__ void __launch_bounds__(kTeam * kTeamsPerBlock)
       }
     }
   }
-  // the team lives in one wavefront: a wavefront-scope fence orders the LDS
-  // writes above before the reads below
-  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-  __builtin_amdgcn_wave_barrier();
+  wave_lds_fence();  // the team lives in one wavefront
   // flux rows of internal and Dirichlet faces: T = C_up X - F_up (+ C_up,dir)
   if (has_face && role != 1) {
     const int64_t r = d->row[lane];

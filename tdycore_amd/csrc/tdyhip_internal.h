@@ -65,6 +65,15 @@ __host__ __device__ inline int64_t trans_index(int64_t nrows, int k, int64_t r) 
   return ((k >> 1) * nrows + r) * 2 + (k & 1);
 }
 
+// Hands LDS values from lane to lane of one wavefront: what lanes wrote before
+// it is seen by reads after it.  The hardware runs a wavefront's LDS operations
+// in program order, so no instruction is emitted; the fence keeps the compiler
+// to that order (the barrier alone is no memory fence to it).
+__device__ inline void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
 // Builds the host topology; returns an error message or empty string.  A mesh
 // that only exceeds the hexahedral kernels' fixed limits (over_limit) is
 // valid: it takes the general path.
