@@ -371,13 +371,14 @@ __global__ void __launch_bounds__(TiledGJ<N>::NT) k_coarse_groups(CoarseLayout C
 // M = H A2^-1 of group g (one workgroup of 256 threads per group, groups of
 // at most 2*RB blocks; H in M on entry): each thread a column and half of the
 // rows, A2^-1 read by rows, H through LDS K groups at a time.  Small in LDS
-// so that it fits beside the factor's workgroups.
+// so that it fits beside the factor's workgroups.  (It does not look at the
+// status: the factor beside it may set it while a workgroup's threads read, and
+// they would part at the barriers.  After a singular block M is not used.)
 constexpr int kFoldThreads = 2 * kNG;
 template <int RB, int K>
 __global__ void __launch_bounds__(kFoldThreads) k_coarse_fold(CoarseLayout C) {
   __shared__ double hs[K][2 * RB];
   const int g = blockIdx.x, t = threadIdx.x, G = C.gsz, ng = C.ng;
-  if (*C.status) return;  // a singular coarse block: nothing of M is used
   const int col = t % kNG, r0 = (t / kNG) * RB;
   double *M = C.M + (int64_t)g * ng * G;
   double s[RB];
