@@ -111,8 +111,9 @@ def footprint_bytes(nc, nf, nv, nbnd, rows, krylov_fp32=True, restart=30):
     ctx = 425 * nc + 609 * nf + 32 * nv + 36 * nbnd
     setup_tmp = 768 * nc + 64 * nf + 264 * nv
     # Newton vectors, block-ordered Jacobian and its columns, Krylov basis,
-    # block-Jacobi tables and factor (rows = the block layout's row count)
-    ws = 64 * nc + 4 * nc + rows * 27 * (8 + 4) + (restart + 5) * nc * tv + rows * (548 + 27 * tv)
+    # block-Jacobi tables (of every block: none shared) and factor (rows = the
+    # block layout's row count)
+    ws = 64 * nc + 4 * nc + rows * 27 * (8 + 4) + (restart + 5) * nc * tv + rows * (686 + 27 * tv)
     ws += rows * 27 * 4  # FP32 copy of the Jacobian (kept in both precisions)
     # coarse correction: slot maps, column sums and their lists per row; lists,
     # basis sums and inverses per block (a server's blocks hold 256 rows); tables
