@@ -721,7 +721,6 @@ static int ensure_ws(tdyhip_ctx *ctx, const tdyhip_solver_opts &o) {
   if ((rc = ws_alloc(ws, (char **)&ws.nd, 256))) return rc;  // a NewtonDev (defined with the solver below)
   if ((rc = ws_alloc(ws, &ws.nh, 4))) return rc;
   if ((rc = ws_alloc(ws, &ws.dyn, 5))) return rc;
-  ws.coarse_req = o.pc_coarse ? 1 : 0;
   if (o.pc_coarse) {
     HostCoarse hc;
     if (build_coarse(hb, ctx->h_jrp, ctx->h_jcols, ctx->nc, ctx->jell_w, hc).empty()) {
@@ -768,6 +767,7 @@ static int ensure_ws(tdyhip_ctx *ctx, const tdyhip_solver_opts &o) {
       ws.coarse = true;
     }
   }
+  ws.coarse_req = o.pc_coarse ? 1 : 0;  // last: after a failure above the next solve starts over
   return 0;
 }
 
