@@ -94,30 +94,37 @@ class Request:
     dt: float = 3600.0
 
 
+def block_width(brick):
+    """Rows of the layout a brick takes."""
+    bs = brick[0] * brick[1] * brick[2]
+    return 64 if bs <= 64 else 256 if bs <= 256 else 512
+
+
 def block_rows(nx, ny, nz, brick):
     """Rows of the block-Jacobi layout: one 64-, 256- or 512-wide slab per brick."""
     bx, by, bz = brick
-    nb = -(-nx // bx) * -(-ny // by) * -(-nz // bz)
-    bs = bx * by * bz
-    return nb * (64 if bs <= 64 else 256 if bs <= 256 else 512)
+    return -(-nx // bx) * -(-ny // by) * -(-nz // bz) * block_width(brick)
 
 
-def footprint_bytes(nc, nf, nv, nbnd, rows, krylov_fp32=True, restart=30):
+def footprint_bytes(nc, nf, nv, nbnd, rows, krylov_fp32=True, restart=30, width=256):
     """Upper bound of the device bytes a request holds while it solves (the
     library's setup arrays, its setup temporaries and the Newton/Krylov
-    workspace), from the mesh counts.  Hexahedral meshes: at most 27 Jacobian
+    workspace), from the mesh counts, the block layout's rows and the width of
+    its blocks (64, 256 or 512).  Hexahedral meshes: at most 27 Jacobian
     entries per row."""
     tv = 8  # Krylov buffers are sized for FP64 (the fallback of a failed FP32 solve)
-    ctx = 425 * nc + 609 * nf + 32 * nv + 36 * nbnd
+    # connectivity, materials, flow state and T, G and fluxes of 4 rows per face
+    ctx = 305 * nc + 353 * nf + 96 * nv + 52 * nbnd
     setup_tmp = 768 * nc + 64 * nf + 264 * nv
     # Newton vectors, block-ordered Jacobian and its columns, Krylov basis,
-    # block-Jacobi tables (of every block: none shared) and factor (rows = the
-    # block layout's row count)
+    # block-Jacobi tables (of every block: none shared) and factor
     ws = 64 * nc + 4 * nc + rows * 27 * (8 + 4) + (restart + 5) * nc * tv + rows * (686 + 27 * tv)
     ws += rows * 27 * 4  # FP32 copy of the Jacobian (kept in both precisions)
-    # coarse correction: slot maps, column sums and their lists per row; lists,
-    # basis sums and inverses per block (a server's blocks hold 256 rows); tables
-    ws += rows * (27 + 27 + 8 + 24) + -(-rows // 256) * (3600 + 8 * (restart + 1)) + (2 << 20)
+    # coarse correction: slot maps, column sums and their lists per row (small
+    # blocks have more neighbours per row); lists, basis sums and inverses per
+    # block; tables
+    ws += rows * (27 + 27 + 8 + (48 if width == 64 else 24)) + -(-rows // width) * (4100 + 8 * (restart + 1))
+    ws += 2 << 20
     return int(ctx + max(setup_tmp, ws) + (1 << 20))
 
 
@@ -255,7 +262,8 @@ class EnsembleServer:
             P = workloads.ensemble_box_problem(r.nx, r.ny, r.nz, r.seed, r.sigma)
             m = P["mesh"]
             rows = block_rows(r.nx, r.ny, r.nz, self.brick)
-            job.need = footprint_bytes(m.nc, m.nf, m.nv, m.nbnd, rows, self.krylov_fp32)
+            job.need = footprint_bytes(m.nc, m.nf, m.nv, m.nbnd, rows, self.krylov_fp32,
+                                       width=block_width(self.brick))
             if job.need > self.hbm_budget:
                 raise MemoryError(f"request {r.rid} needs {job.need} B, above the HBM budget {self.hbm_budget} B")
             if self._draining:
