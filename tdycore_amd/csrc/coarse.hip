@@ -42,10 +42,8 @@ struct CoarseLayout {
   int nb = 0, ng = 0, gsz = 0;    // blocks, groups, max blocks per group
   int nov = 0;                    // blocks of a group with overlap, at most (0: a block per group)
   int g2max = 0;                  // entries of r2c of a group, at most
-  int32_t *nbr = nullptr;         // nb*kCQ neighbour block ids, ascending (-1 pad)
-  uint8_t *cq = nullptr;          // W*NB, block-contiguous as the ELL: position in nbr[block(p)] of slot k's column block (255 none)
+  uint8_t *cq = nullptr;          // W*NB, block-contiguous as the ELL: place of slot k's column block among the neighbours of p's block (255 none)
   uint8_t *tslot = nullptr;       // W*NB: slot of row i's mirror entry A_ci in the row c of its slot k (255 none)
-  int32_t *grp = nullptr;         // nb: group of each block
   int32_t *gmem = nullptr;        // ng*gsz: blocks of each group (-1 pad)
   int32_t *gov = nullptr;         // ng*nov: blocks of each group, then its overlap (-1 pad)
   uint8_t *gpos = nullptr;        // ng*nov*kCQ: place in gov of each member's neighbour q (255 none)
@@ -185,7 +183,9 @@ __device__ inline double wave_max(double v) {
 // and the loop stays rolled: a small body, as its first pass through the
 // instruction cache costs more than a step.  128 x 128 alone 318 -> 170 us,
 // 64 x 64 164 -> 51 us against 4x4 tiles per thread with the pivot search, both
-// rows and the column published in turn (four barriers a step).
+// rows and the column published in turn (four barriers a step).  (At 128 x 128 a
+// lane's 64 values and the pivot row's 32 take 248 + 32 registers and 140 bytes of
+// scratch.)
 template <int N>
 struct TiledGJ {
   static constexpr int NT = 256, RL = N / 64, CW = N / 4;

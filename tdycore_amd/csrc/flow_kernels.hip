@@ -887,7 +887,7 @@ struct VelArgs {
   double gabs;  // |g|
   const uint8_t *face_flags;
   const int32_t *face_verts, *vcols;                          // hexahedra: rows by vertex columns
-  const double *T;                                            // hexahedra: slot-major over rows
+  const double *T;                                            // hexahedra: pairs of columns over rows (trans_index)
   const int32_t *rtoff, *rinfo, *roc, *rdc, *ccell, *vdcol;   // general meshes: per-row blocks
   const double *Tgen;
   const int32_t *bnd_cell;

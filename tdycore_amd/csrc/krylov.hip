@@ -8,12 +8,13 @@
 //
 // Block-Jacobi ILU(0): cells are partitioned (host) into compact blocks of at
 // most BS cells (BS = 64: one wavefront per block; BS = 256 or 512: one 4- or
-// 8-wave workgroup per block; at 512 the FP64 factor holds 137 KB of LDS).  Inside a block rows keep their global order;
+// 8-wave workgroup per block; at 512 the FP64 factor holds 125 KB of LDS).  Inside a block rows keep their global order;
 // entries coupling different blocks are dropped.  The factorization (IKJ)
 // and the two triangular solves advance level by level (levels of the
 // in-block dependency DAG, computed on the host) with the block's rows in
 // LDS, so no grid-wide synchronisation is ever needed.  The Jacobian is held
-// slot-major (slot s of row i at s*n + i) so every sweep is coalesced.
+// block by block (slot s of row t of block b at (b*W + s)*BS + t) so every sweep
+// is coalesced.
 #include "tdyhip_internal.h"
 
 namespace tdyhip {

@@ -732,10 +732,10 @@ static int ensure_ws(tdyhip_ctx *ctx, const tdyhip_solver_opts &o) {
       int32_t *eptr, *wdst, *w2dst;
       uint16_t *cent, *tq;
       uint8_t *ownq, *gsl;
-      if ((rc = up(&C.nbr, hc.nbr)) || (rc = up(&C.cq, block_contiguous(hc.cq, ctx->jell_w, hb.bs, hb.nblocks))) ||
-          (rc = up(&C.grp, hc.grp)) || (rc = up(&C.gmem, hc.gmem)) || (rc = up(&C.gov, hc.gov)) ||
-          (rc = up(&C.gpos, hc.gpos)) || (rc = up(&C.gent, hc.gent)) || (rc = up(&C.gep, hc.gep)) || (rc = up(&C.g2ptr, hc.g2ptr)) || (rc = up(&eptr, hc.eptr)) ||
-          (rc = up(&cent, hc.cent)) || (rc = up(&tq, hc.tq)) || (rc = up(&ownq, hc.ownq)) || (rc = up(&gsl, hc.gsl)) ||
+      if ((rc = up(&C.cq, block_contiguous(hc.cq, ctx->jell_w, hb.bs, hb.nblocks))) ||
+          (rc = up(&C.gmem, hc.gmem)) || (rc = up(&C.gov, hc.gov)) || (rc = up(&C.gpos, hc.gpos)) ||
+          (rc = up(&C.gent, hc.gent)) || (rc = up(&C.gep, hc.gep)) || (rc = up(&C.g2ptr, hc.g2ptr)) ||
+          (rc = up(&eptr, hc.eptr)) || (rc = up(&cent, hc.cent)) || (rc = up(&tq, hc.tq)) || (rc = up(&ownq, hc.ownq)) || (rc = up(&gsl, hc.gsl)) ||
           (rc = up(&wdst, hc.wdst)) || (rc = up(&w2dst, hc.w2dst)))
         return rc;
       if ((rc = ws_alloc(ws, &C.tslot, nel)) || (rc = ws_alloc(ws, &C.cown, (size_t)ws.NB)) ||
@@ -1801,10 +1801,10 @@ int tdyhip_test_coarse_layout(const int32_t *jrp, const int32_t *jcols, int32_t 
 }
 
 // Test hook, not part of the interface in include/tdyhip.h: Ainv = A^-1 for
-// one dense n x n row-major matrix by the coarse correction's register-tiled
-// Gauss-Jordan at width 64 (the group inverses, n <= 64) or 128 (the level-2
-// inverse, n <= 128), on the current device.  A zero pivot returns
-// TDYHIP_ERR_SINGULAR.
+// one dense n x n row-major matrix by the coarse correction's register
+// Gauss-Jordan at width 64 (n <= 64) or 128 (n <= 128), on the current device:
+// the group inverses take the width their overlap needs, the level-2 inverse the
+// width of the groups.  A zero pivot returns TDYHIP_ERR_SINGULAR.
 int tdyhip_test_dense_inverse(const double *A, int32_t n, int32_t width, double *Ainv) {
   using namespace tdyhip;
   if (!A || !Ainv || (width != kGMax && width != kNG) || n < 1 || n > width) { set_error("bad argument"); return TDYHIP_ERR_ARG; }
