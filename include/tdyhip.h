@@ -167,8 +167,9 @@ typedef struct {
                                              blocks and at most 128 group values solved exactly);
                                              not in the reference, whose PETSc
                                              default is one-level block Jacobi.  Used only when the
-                                             mesh fits its limits (<= 32 neighbour blocks per block,
-                                             <= 8192 blocks).  Default 0. */
+                                             mesh fits its limits (<= 32 entries per row and
+                                             neighbour blocks per block, <= 8192 blocks, a block's
+                                             rows in <= 27 neighbours each on average).  Default 0. */
 } tdyhip_solver_opts;
 
 typedef struct {
